@@ -95,38 +95,6 @@ __device__ inline void half_cell_frac(float4 x, const DevParams* __restrict__ dp
 // the scaled coordinates (a few ulp of at most 2048 half-cells, < 1e-3).
 constexpr float kReach2 = 1.0201f;
 
-// Visits the particle ranges of the half-cells around hc that a sphere of
-// radius h about the particle can reach: a (dy, dz) row is skipped when its
-// nearest face is out of reach, and its x-range keeps the neighbours on
-// either side only when they are in reach. Within a row the half-cells
-// 2k, 2k+1 share a cell and are Morton-adjacent; each maximal such piece
-// of the x-range is one run (at most two per row).
-template <typename R>
-__device__ inline void for_each_run(const uint32_t hc[3], const float fr[3], uint32_t base,
-                                    const uint32_t* __restrict__ ht, uint32_t Fc, uint32_t n,
-                                    R&& run) {
-  const float lo_x = fr[0] * fr[0], hi_x = (1.f - fr[0]) * (1.f - fr[0]);
-  for (int dz = -1; dz <= 1; ++dz) {
-    const float az = dz < 0 ? fr[2] : (dz > 0 ? 1.f - fr[2] : 0.f);
-    for (int dy = -1; dy <= 1; ++dy) {
-      const float ay = dy < 0 ? fr[1] : (dy > 0 ? 1.f - fr[1] : 0.f);
-      const float ryz = az * az + ay * ay;
-      if (ryz >= kReach2) continue;
-      const uint32_t y = hc[1] + (uint32_t)dy, z = hc[2] + (uint32_t)dz;
-      const uint32_t xa = lo_x + ryz < kReach2 ? hc[0] - 1u : hc[0];
-      const uint32_t xb = hi_x + ryz < kReach2 ? hc[0] + 1u : hc[0];
-      uint32_t x = xa;
-      for (int piece = 0; piece < 2 && x <= xb; ++piece) {
-        const uint32_t xe = (x | 1u) < xb ? (x | 1u) : xb;
-        uint32_t s, e;
-        half_range(base + half_key(x, y, z), xe - x + 1u, ht, Fc, n, s, e);
-        run(s, e);
-        x = xe + 1u;
-      }
-    }
-  }
-}
-
 // Two- and four-lane unsigned vectors, held in aligned register pairs and
 // quads; the neighbour list's rows are addressed as global memory.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -200,37 +168,14 @@ struct DensityWalk {
   }
 };
 
-// The walk over the sorted positions in HBM: the reach-pruned half-cell runs
-// of for_each_run, candidates loaded four at a time so that their latencies
-// overlap (pos is padded by 4 entries past the particles, so a group needs no
-// clamp).
-__device__ inline void density_walk_global(DensityWalk& w, uint32_t i, float4 xi,
-                                           const uint32_t hc[3], const float fr[3],
-                                           const DevParams* __restrict__ dp, uint32_t F,
-                                           const float4* __restrict__ pos,
-                                           const uint32_t* __restrict__ table, float h2,
-                                           uint32_t n) {
-  for_each_run(hc, fr, dp->key_base, table, F, n, [&](uint32_t s, uint32_t e) {
-    for (uint32_t j0 = s; j0 < e; j0 += 4) {
-      const float4* pj = pos + j0;
-      float4 c[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) c[u] = pj[u];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t j = j0 + u;
-        w.visit(j < e, dist2(xi, c[u]), h2, (u32x2){j, j}, i);
-      }
-    }
-  });
-}
-
-// The same walk over a cell's halo staged in LDS: the 4x4x4 half-cells
+// One lane's walk over its cell's halo staged in LDS: the 4x4x4 half-cells
 // around the particle's cell (side 2h), half-cell q = x + 4y + 16z at
 // cand[off[q], off[q + 1]) in sorted order, each entry (x, y, z, sorted
 // index). The particle sits at local coordinates 1 + (hc & 1), so each row
-// (dy, dz) of its 3x3x3 block is one contiguous range. Visiting order, and
-// so every sum and list, is that of density_walk_global.
+// (dy, dz) of its 3x3x3 block is one contiguous range. A row is skipped when
+// its nearest face is out of reach, and its x-range keeps the half-cells on
+// either side only when they are in reach. Candidates are visited in z, y, x
+// order, four loaded at a time.
 __device__ inline void density_walk_halo(DensityWalk& w, uint32_t i, float4 xi,
                                          const uint32_t hc[3], const float fr[3],
                                          const float4* cand, const uint32_t* off, float h2) {
@@ -265,6 +210,212 @@ __device__ inline void density_walk_halo(DensityWalk& w, uint32_t i, float4 xi,
   }
 }
 
+// Density and pressure of particle i from its kernel sum (sph.cl:36-39), and
+// what the later stages read: its neighbour count, its force inputs
+// fab[2i] = (x, p / rho^2), fab[2i + 1] = (v, m / rho) and, with `nu`, the
+// learned surrogate's node inputs.
+__device__ inline void density_store(const DevParams* __restrict__ dp, uint32_t i, float4 xi,
+                                     float sum, uint32_t count, const float4* __restrict__ vel,
+                                     float* __restrict__ rho, float* __restrict__ prs,
+                                     float4* __restrict__ fab, uint32_t* __restrict__ nbr_count,
+                                     float2* __restrict__ nu) {
+  nbr_count[i] = count;
+  // density = sum m * poly6 * (h^2 - r^2)^3 ; Tait pressure
+  float m = dp->p.particle_mass;
+  float d = m * (dp->t.poly_6 * sum);
+  float q = d / dp->p.fluid_density;
+  float q2 = q * q, q4 = q2 * q2;
+  float p = dp->p.K * (q4 * q2 * q - 1.f);
+  rho[i] = d;
+  prs[i] = p;
+  float4 vi = vel[i];
+  fab[2u * i] = make_float4(xi.x, xi.y, xi.z, p / (d * d));
+  fab[2u * i + 1u] = make_float4(vi.x, vi.y, vi.z, m / d);
+  if (nu) nu[i] = node_in(d, p, dp->p.fluid_density, dp->p.K);
+}
+
+// Orders a wave's own LDS accesses (its lanes exchange data, no other wave
+// is involved).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// LDS of one particle in a walk by L lanes.
+constexpr uint32_t kRuns = 18;  // runs of a particle's half-cells: 9 rows of at most two
+template <int L>
+struct LaneWalk {
+  static constexpr uint32_t kHits = L == 16 ? 64u : 32u;
+  float t[kHits];                // neighbours not yet summed: h^2 - r^2
+  uint32_t j[kHits];             // and their sorted indices
+  uint32_t run_end[kRuns + 1];   // the runs laid end to end
+  uint32_t run_shift[kRuns + 1]; // sorted index less laid-out index
+};
+
+// Density sum and neighbour list of one particle i by L consecutive lanes,
+// straight from the sorted positions: its runs of half-cells are looked up by
+// the lanes in parallel and laid end to end, and each round takes the next L
+// candidates, four rounds' loads in flight. A ballot ranks the neighbours
+// found in a round, so that they land in the particle's LDS list in visiting
+// order; the sum then runs over that list: the additions, in their order, of
+// DensityWalk over the same candidates. Every lane of the wave calls it
+// (`live` false: nothing is written) and gets its particle's sum and count.
+template <int L>
+__device__ inline void density_walk_lanes(LaneWalk<L>& w, bool live, uint32_t i, float4 xi,
+                                          const DevParams* __restrict__ dp, uint32_t F,
+                                          const float4* __restrict__ pos,
+                                          const uint32_t* __restrict__ table,
+                                          uint4* __restrict__ nbr, uint32_t n, float& sum,
+                                          uint32_t& count) {
+  constexpr uint32_t kHits = LaneWalk<L>::kHits;
+  const uint32_t sub = threadIdx.x % L, lane = threadIdx.x & 63u, first = lane - sub;
+  const float h = dp->p.h, h2 = h * h;
+  uint32_t hc[3];
+  float fr[3];
+  half_cell_frac(xi, dp, hc, fr);
+  // run r: row r / 2 (dy fastest); along x the half-cells 2k and 2k + 1 share
+  // a cell and are Morton-adjacent, so the reach's x-range is cut after the
+  // first odd coordinate (r even: up to there, r odd: the rest)
+  uint32_t laid = 0;
+  const float lo_x = fr[0] * fr[0], hi_x = (1.f - fr[0]) * (1.f - fr[0]);
+#pragma unroll
+  for (uint32_t r0 = 0; r0 < kRuns; r0 += L) {
+    const uint32_t r = r0 + sub, row = r >> 1;
+    const int dy = (int)(row % 3u) - 1, dz = (int)(row / 3u) - 1;
+    const float az = dz < 0 ? fr[2] : (dz > 0 ? 1.f - fr[2] : 0.f);
+    const float ay = dy < 0 ? fr[1] : (dy > 0 ? 1.f - fr[1] : 0.f);
+    const float ryz = az * az + ay * ay;
+    uint32_t s = 0, e = 0;
+    if (r < kRuns && live && ryz < kReach2) {
+      const uint32_t xa = lo_x + ryz < kReach2 ? hc[0] - 1u : hc[0];
+      const uint32_t xb = hi_x + ryz < kReach2 ? hc[0] + 1u : hc[0];
+      const uint32_t mid = (xa | 1u) < xb ? (xa | 1u) : xb;
+      const uint32_t x0 = (r & 1u) ? mid + 1u : xa, x1 = (r & 1u) ? xb : mid;
+      if (x0 <= x1)
+        half_range(dp->key_base + half_key(x0, hc[1] + (uint32_t)dy, hc[2] + (uint32_t)dz),
+                   x1 - x0 + 1u, table, F, n, s, e);
+    }
+    uint32_t incl = e - s;
+#pragma unroll
+    for (uint32_t o = 1; o < (uint32_t)L; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o, L);
+      if (sub >= o) incl += y;
+    }
+    if (r < kRuns) {
+      w.run_end[r] = laid + incl;
+      w.run_shift[r] = s - (laid + incl - (e - s));
+    }
+    laid += __shfl(incl, L - 1, L);
+  }
+  wave_lds_fence();
+
+  float acc = (h2 * h2) * h2;    // the particle's own term
+  uint32_t total = 0, pend = 0;  // neighbours summed and listed in nbr; waiting in LDS
+  // sums and lists the waiting neighbours: all of them, or whole groups of
+  // four (a group is one entry of nbr); what is left moves to the front
+  auto drain = [&](bool all) {
+    wave_lds_fence();
+    const uint32_t whole = pend & ~3u, take = all ? pend : whole;
+    for (uint32_t k = 0; k < take; k += 4u) {
+      const float4 t4 = *(const float4*)(w.t + k);
+      const float tt[4] = {t4.x, t4.y, t4.z, t4.w};
+#pragma unroll
+      for (uint32_t u = 0; u < 4u; ++u) {
+        const float t = k + u < take ? tt[u] : 0.f;
+        acc = __builtin_fmaf(t, t * t, acc);
+      }
+    }
+    for (uint32_t k = 4u * sub; k < take && total + k < kMaxNeighbours; k += 4u * L) {
+      const uint4 j4 = *(const uint4*)(w.j + k);
+      const uint32_t left = take - k;
+      nbr[(size_t)((total + k) >> 2) * n + i] =
+          make_uint4(j4.x, left > 1u ? j4.y : 0u, left > 2u ? j4.z : 0u, left > 3u ? j4.w : 0u);
+    }
+    total += take;
+    const uint32_t left = pend - take;
+    float mt = 0.f;
+    uint32_t mj = 0;
+    if (sub < left) mt = w.t[whole + sub], mj = w.j[whole + sub];
+    wave_lds_fence();
+    if (sub < left) w.t[sub] = mt, w.j[sub] = mj;
+    pend = left;
+    wave_lds_fence();
+  };
+
+  constexpr uint32_t kAhead = 4;
+  uint32_t r = 0, r_end = w.run_end[0], shift = w.run_shift[0];
+  for (uint32_t a = 0; __any(a < laid); a += kAhead * L) {
+    float4 c[kAhead];
+    uint32_t j[kAhead];
+#pragma unroll
+    for (uint32_t u = 0; u < kAhead; ++u) {
+      const uint32_t k = a + u * L + sub;
+      if (k < laid) {
+        while (k >= r_end) {  // ends: the last run ends at laid
+          ++r;
+          r_end = w.run_end[r];
+          shift = w.run_shift[r];
+        }
+      }
+      j[u] = k < laid ? k + shift : i;  // past the end: the particle itself, no neighbour
+      c[u] = pos[j[u]];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kAhead; ++u) {
+      if (__any(pend + L > kHits)) drain(false);
+      const float d2 = dist2(xi, c[u]);
+      const bool hit = d2 < h2 && j[u] != i;
+      const uint32_t found = (uint32_t)(__ballot(hit) >> first) & ((1u << L) - 1u);
+      if (hit) {
+        const uint32_t at = pend + (uint32_t)__popc(found & ((1u << sub) - 1u));
+        w.t[at] = h2 - d2;
+        w.j[at] = j[u];
+      }
+      pend += (uint32_t)__popc(found);
+    }
+  }
+  drain(true);
+  sum = acc;
+  count = total;
+}
+
+// The density stage by L lanes per particle, for states too small to fill the
+// chip with one particle per lane (rule in launch_density). Bound by the
+// latency of its four dependent loads (position, table, candidates twice) and
+// the ordered sum: 12 us at 4,096 particles, where one lane's walk took 66.
+constexpr int kLanesBlock = 256;
+constexpr uint32_t kLanes16Max = 40960;   // particles up to which 16 lanes take one
+constexpr uint32_t kLanes4Max = 147456;   // and up to which 4 lanes do
+template <int L>
+__global__ __launch_bounds__(kLanesBlock) void k_density_lanes(
+    const float4* __restrict__ pos, const float4* __restrict__ vel,
+    const uint32_t* __restrict__ table, const BlockDesc* __restrict__ blocks,
+    const DevParams* __restrict__ dps, const BatchParams* __restrict__ bp,
+    float* __restrict__ rho, float* __restrict__ prs, float4* __restrict__ fab,
+    uint4* __restrict__ nbr, uint32_t* __restrict__ nbr_count, float2* __restrict__ nu,
+    uint32_t n) {
+  constexpr uint32_t kParts = kLanesBlock / L;  // particles per work-group
+  __shared__ __attribute__((aligned(16))) LaneWalk<L> walks[kParts];
+  // a 64-particle entry of the work list is shared by 64 / kParts work-groups
+  constexpr uint32_t kShare = 64u / kParts;
+  const BlockDesc b = blocks[blockIdx.x / kShare];
+  const DevParams* dp = dps + b.scene;
+  const uint32_t part = threadIdx.x / L;
+  const uint32_t p = b.first + (blockIdx.x % kShare) * kParts + part;
+  const uint32_t se = dp->begin + dp->n;
+  const bool live = p < se;
+  if (!__any(live)) return;
+  const uint32_t i = live ? p : se - 1u;
+  const float4 xi = pos[i];
+  float sum;
+  uint32_t count;
+  density_walk_lanes<L>(walks[part], live, i, xi, dp, usable_key_end(dp, bp), pos, table, nbr, n,
+                        sum, count);
+  if (live && threadIdx.x % L == 0u)
+    density_store(dp, i, xi, sum, count, vel, rho, prs, fab, nbr_count, nu);
+}
+
 // Inverse of spread10: the 10 bits at positions 3k.
 __device__ inline uint32_t compact10(uint32_t v) {
   v &= 0x09249249u;
@@ -292,18 +443,26 @@ struct DensityHalos {
   uint32_t wave_sum[WAVES];
   uint32_t wave_cells[WAVES];
 };
+// Lanes per particle outside the staged halos, and what their walks keep in
+// the candidates' bytes (two 80 KB work-groups per CU leave no others).
+constexpr int kRestLanes = 4;
+template <int WAVES>
+struct DensityRest {
+  LaneWalk<kRestLanes> walk[WAVES * 64 / kRestLanes];
+  uint16_t thread[WAVES * 64];
+};
 
 // Density and pressure (sph.cl:9-40, forces.cl:15-43) of the particles
 // [first, first + 64 WAVES) of one scene, with each particle's neighbour
-// list (self excluded) in visiting order into nbr[q * n + i], its count into
-// nbr_count[i], the force inputs fab[2i] = (x, p / rho^2), fab[2i + 1] =
-// (v, m / rho), and with `nu` the learned surrogate's node inputs. The
-// work-group first stages, for each distinct cell (side 2h) its particles
-// fall in, the cell's 4x4x4 half-cell halo in LDS (coalesced runs
-// of the sorted positions); particles then walk their 3x3x3 half-cells
-// there. Cells beyond the staging capacity, and every particle when the
-// table is unusable, walk the sorted positions in HBM instead, with the same
-// visiting order.
+// list (self excluded) in visiting order into nbr[q * n + i]. The work-group
+// first stages, for each distinct cell (side 2h) its particles fall in, the
+// cell's 4x4x4 half-cell halo in LDS (coalesced runs of the sorted
+// positions); particles then walk their 3x3x3 half-cells there, one to a
+// lane. Those of cells beyond the staging capacity, and every particle when
+// the table is unusable, are then walked from HBM by four lanes each, with
+// the same visiting order: a lane's walk of HBM by itself took 30-50 us, in
+// some work-group of every launch (with four lanes 262,144 particles take 70
+// instead of 80 us, 1,048,576 after 1,000 substeps 211 instead of 223).
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel,
@@ -412,30 +571,46 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
   }
   __syncthreads();
 
-  if (!live) return;
-  const float4 xi = pos[i];
-  uint32_t hc[3];
-  float fr[3];
-  half_cell_frac(xi, dp, hc, fr);
-  DensityWalk w(nbr, i, n, h2);
-  if (ci < staged)
+  if (live && ci < staged) {
+    const float4 xi = pos[i];
+    uint32_t hc[3];
+    float fr[3];
+    half_cell_frac(xi, dp, hc, fr);
+    DensityWalk w(nbr, i, n, h2);
     density_walk_halo(w, i, xi, hc, fr, sh.cand, sh.off + 64u * ci, h2);
-  else
-    density_walk_global(w, i, xi, hc, fr, dp, F, pos, table, h2, n);
-  w.finish();
-  nbr_count[i] = w.cnt;
-  // density = sum m * poly6 * (h^2 - r^2)^3 ; Tait pressure (sph.cl:36-39)
-  float m = dp->p.particle_mass;
-  float d = m * (dp->t.poly_6 * w.acc);
-  float q = d / dp->p.fluid_density;
-  float q2 = q * q, q4 = q2 * q2;
-  float p = dp->p.K * (q4 * q2 * q - 1.f);
-  rho[i] = d;
-  prs[i] = p;
-  float4 vi = vel[i];
-  fab[2u * i] = make_float4(xi.x, xi.y, xi.z, p / (d * d));
-  fab[2u * i + 1u] = make_float4(vi.x, vi.y, vi.z, m / d);
-  if (nu) nu[i] = node_in(d, p, dp->p.fluid_density, dp->p.K);
+    w.finish();
+    density_store(dp, i, xi, w.acc, w.cnt, vel, rho, prs, fab, nbr_count, nu);
+  }
+  if (staged == cells) return;  // uniform: every cell was staged
+  // the rest, in the order of their threads
+  const bool left = live && ci >= staged;
+  const uint64_t lm = __ballot(left);
+  if (lane == 0) sh.wave_sum[wv] = (uint32_t)__popcll(lm);
+  __syncthreads();  // also: the staged walks are done with cand
+  uint32_t at = 0, rest = 0;
+  for (int q = 0; q < WAVES; ++q) {
+    at += (uint32_t)q < wv ? sh.wave_sum[q] : 0u;
+    rest += sh.wave_sum[q];
+  }
+  using Rest = DensityRest<WAVES>;
+  static_assert(sizeof(Rest) <= sizeof(sh.cand), "it fits in the candidates' bytes");
+  Rest& rest_lds = reinterpret_cast<Rest&>(sh.cand);
+  if (left) rest_lds.thread[at + (uint32_t)__popcll(lm & ((1ull << lane) - 1ull))] = (uint16_t)t;
+  __syncthreads();
+  constexpr uint32_t kParts = WAVES * 64 / kRestLanes;
+  LaneWalk<kRestLanes>& walk = rest_lds.walk[t / kRestLanes];
+  for (uint32_t r0 = 0; r0 < rest; r0 += kParts) {
+    const uint32_t r = r0 + t / kRestLanes;
+    const bool on = r < rest;
+    if (!__any(on)) break;
+    const uint32_t ip = b.first + rest_lds.thread[on ? r : 0u];
+    const float4 xi = pos[ip];
+    float sum;
+    uint32_t count;
+    density_walk_lanes<kRestLanes>(walk, on, ip, xi, dp, F, pos, table, nbr, n, sum, count);
+    if (on && t % kRestLanes == 0u)
+      density_store(dp, ip, xi, sum, count, vel, rho, prs, fab, nbr_count, nu);
+  }
 }
 
 // Pair terms of compute_internal_forces_with_grid (forces.cl:60-101) for one
@@ -587,6 +762,22 @@ __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__
 
 void launch_density(clsph_state* s, float2* nu) {
   if (s->n == 0) return;
+  // Lanes per particle. One (k_density) does the least work, but its time is
+  // at least a wave's walk, 30-50 us; below that many particles the chip has
+  // lanes to spare. Stage time on evolved dam breaks, 1 / 4 / 16 lanes:
+  // 16,384 particles 86 / 25 / 15 us, 50,021 49 / 31 / 30, 65,536
+  // 48 / 34 / 36, 131,071 62 / 49 / 58, 180,000 47 / 58 / 77.
+  if (s->n <= kLanes4Max) {
+    // 64-particle entries of the work list, whatever the stage's block size
+    auto lanes = [&](auto kernel, uint32_t share) {
+      hipLaunchKernelGGL(kernel, dim3(s->nblocks[0] * share), dim3(kLanesBlock), 0,
+                         s->ctx->stream, s->pos_s, s->vel_s, s->table, s->blocks[0], s->dps, s->bp,
+                         s->rho_s, s->prs_s, s->fab, s->nbr, s->nbr_count, nu, s->n);
+    };
+    if (s->n <= kLanes16Max) lanes(k_density_lanes<16>, 4);
+    else lanes(k_density_lanes<4>, 1);
+    return;
+  }
   const int bs = s->bs_of(kStageDensity);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(s->nblocks_of(kStageDensity)), dim3(bs), 0, s->ctx->stream,
