@@ -72,7 +72,8 @@ struct clsph_gnn {
 
   // neighbour graph of the current evaluation (dst-major CSR)
   uint32_t n = 0, e = 0;
-  uint32_t* off = nullptr;      // n_cap + 1
+  bool cut = false;             // some particle has more neighbours than kMaxEdges
+  uint32_t* off = nullptr;      // n_cap + 2: the edges before each particle, all, and the cut flag
   uint32_t* src = nullptr;      // e_cap
   uint32_t* dst = nullptr;      // e_cap
   uint32_t* scan_part = nullptr;
@@ -85,7 +86,6 @@ struct clsph_gnn {
   uint16_t* s1[2] = {};
   float* z2[2] = {};
   uint16_t* S[2] = {};          // n x 128: bf16(sum_j s2 / C)
-  float* tmp = nullptr;         // n x 256 float scratch
   uint16_t* u1 = nullptr;       // n x 144
   float* p1 = nullptr;
   uint16_t* y1 = nullptr;
@@ -109,7 +109,6 @@ struct clsph_gnn {
   uint16_t* dpb = nullptr;      // n x 256 bf16 scratch
   float* dS = nullptr;          // n x 128
   uint16_t* dz2 = nullptr;      // e x 128
-  float* ds1 = nullptr;         // e x 128
   uint16_t* dz1 = nullptr;      // e x 128
   float* dPA = nullptr;
   float* dPB = nullptr;

@@ -34,14 +34,12 @@ __device__ inline float dsilu(float x) {
   return s * (1.f + x * (1.f - s));
 }
 
-// The bf16 matrix-core GEMM of the corrective surrogate (nn.hip):
-// C (f32, M x N, ldc) = alpha * op(A) op(B) [+ rowscale[m] * bias[n]], or
-// added to C with `add`.
-inline void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
-                 const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
-                 const float* bias = nullptr, const float* rowscale = nullptr) {
-  nn::gemm_public(s, ta, tb, add, A, lda, B, ldb, C, ldc, M, N, K, alpha, bias, rowscale);
-}
+// the bf16 matrix-core GEMM of the corrective surrogate (nn.hip)
+using nn::colsum;
+using nn::gemm;
+using nn::gemm_dsilu;
+using nn::gemm_silu;
+using nn::gemm_weight_grad;
 
 // ---------------------------------------------------------------------------
 // Exclusive scan of min(count, kMaxEdges) into off[0..n], off[n] = total.
@@ -71,11 +69,16 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_local(const uint32_t* __res
   __shared__ uint32_t lds[4];
   uint32_t base = blockIdx.x * kScanChunk + threadIdx.x * kScanItems;
   uint32_t v[kScanItems], sum = 0;
+  bool cut = false;
   for (int t = 0; t < kScanItems; ++t) {
     uint32_t i = base + t;
     v[t] = i < n ? min(count[i], kMaxEdges) : 0u;
+    cut = cut || (i < n && count[i] > kMaxEdges);
     sum += v[t];
   }
+  // the chunk's second word: a list was cut short at kMaxEdges
+  const int any = __syncthreads_or(cut ? 1 : 0);
+  if (threadIdx.x == 0) part[2 * blockIdx.x + 1] = any ? 1u : 0u;
   uint32_t total;
   uint32_t ex = block_scan_256(sum, lds, total);
   for (int t = 0; t < kScanItems; ++t) {
@@ -83,34 +86,41 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_local(const uint32_t* __res
     if (i < n) off[i] = ex;
     ex += v[t];
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = total;
+  if (threadIdx.x == 0) part[2 * blockIdx.x] = total;
 }
 
-// One work-group scans the chunk totals (any count) in place.
+// One work-group scans the chunk totals (any count) in place; total_out[0] is
+// their sum, total_out[1] whether any chunk's second word is set.
 __global__ __launch_bounds__(kScanBlock) void k_scan_parts(uint32_t* __restrict__ part,
                                                            uint32_t nparts,
                                                            uint32_t* __restrict__ total_out) {
   __shared__ uint32_t lds[4];
   uint32_t carry = 0;
+  int cut = 0;
   for (uint32_t b = 0; b < nparts; b += kScanBlock) {
     uint32_t i = b + threadIdx.x;
-    uint32_t v = i < nparts ? part[i] : 0u;
+    uint32_t v = i < nparts ? part[2 * i] : 0u;
+    cut |= __syncthreads_or(i < nparts && part[2 * i + 1] ? 1 : 0);
     uint32_t total;
     uint32_t ex = block_scan_256(v, lds, total);
-    if (i < nparts) part[i] = carry + ex;
+    if (i < nparts) part[2 * i] = carry + ex;
     carry += total;
   }
-  if (threadIdx.x == 0) *total_out = carry;
+  if (threadIdx.x == 0) {
+    total_out[0] = carry;
+    total_out[1] = cut ? 1u : 0u;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_scan_add(uint32_t* __restrict__ off,
                                                   const uint32_t* __restrict__ part, uint32_t n) {
   uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) off[i] += part[i / kScanChunk];
+  if (i < n) off[i] += part[2 * (i / kScanChunk)];
 }
 
 // ---------------------------------------------------------------------------
-// src / dst of every edge (dst-major, the density kernel's neighbour order).
+// src / dst of every edge (dst-major, the density kernel's neighbour order);
+// blockIdx.y of gridDim.y takes every gridDim.y-th group of four neighbours.
 __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
                                                const uint32_t* __restrict__ count,
                                                const uint32_t* __restrict__ off, uint32_t n,
@@ -120,7 +130,7 @@ __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
   uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   uint32_t deg = min(count[i], kMaxEdges), o = off[i];
-  for (uint32_t q = 0; q < deg; q += 4) {
+  for (uint32_t q = 4 * blockIdx.y; q < deg; q += 4 * gridDim.y) {
     uint4 js = nbr[(size_t)(q >> 2) * n + i];
     uint32_t jj[4] = {js.x, js.y, js.z, js.w};
     for (uint32_t t = 0; t < 4 && q + t < deg; ++t) {
@@ -128,7 +138,7 @@ __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
       dst[o + q + t] = i;
     }
   }
-  degc[i] = (float)deg / kAggC;
+  if (blockIdx.y == 0) degc[i] = (float)deg / kAggC;
 }
 
 // The 16 edge inputs of edge (i <- j) in float32 (12 used, 4 zero).
@@ -596,12 +606,6 @@ __global__ __launch_bounds__(512) void k_node2(const uint16_t* __restrict__ S1,
 
 // ---------------------------------------------------------------------------
 // Elementwise and row kernels (grid-stride loops).
-__global__ void k_silu_bf16(const float* __restrict__ z, uint16_t* __restrict__ s, size_t count) {
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x)
-    s[k] = to_bf16(silu(z[k]));
-}
-
 __global__ void k_cast_2d(const float* __restrict__ x, int ldx, uint16_t* __restrict__ y, int ldy,
                           size_t rows, int cols) {
   size_t count = rows * cols;
@@ -624,42 +628,26 @@ __global__ void k_copy_2d(const float* __restrict__ x, int ldx, float* __restric
   }
 }
 
-// dz = bf16(dy * silu'(p)); dy has row stride ldy, p and dz are dense.
-__global__ void k_dsilu(const float* __restrict__ dy, int ldy, const float* __restrict__ p,
-                        uint16_t* __restrict__ dz, size_t rows, int cols) {
-  size_t count = rows * cols;
+// dz2[e] = bf16(dS[dst[e]] * silu'(z2[e])), 128 features per edge, eight per
+// thread.
+__global__ __launch_bounds__(256) void k_edge_dz(const float* __restrict__ dS,
+                                                 const float* __restrict__ z2,
+                                                 const uint32_t* __restrict__ dst,
+                                                 uint16_t* __restrict__ dz, size_t e) {
+  const size_t count = e * (kWidth / 8);
   for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
        k += (size_t)gridDim.x * blockDim.x) {
-    size_t r = k / cols;
-    int c = (int)(k % cols);
-    dz[k] = to_bf16(dy[r * ldy + c] * dsilu(p[k]));
-  }
-}
-
-// dz2[e] = bf16(dS[dst[e]] * silu'(z2[e])), 128 features per edge.
-__global__ void k_edge_dz(const float* __restrict__ dS, const float* __restrict__ z2,
-                          const uint32_t* __restrict__ dst, uint16_t* __restrict__ dz,
-                          size_t e) {
-  size_t count = e * kWidth;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t ed = k / kWidth;
-    int c = (int)(k % kWidth);
-    dz[k] = to_bf16(dS[(size_t)dst[ed] * kWidth + c] * dsilu(z2[k]));
-  }
-}
-
-// z1[e] += PA[dst[e]] + PB[src[e]] (bf16 node terms of round 2).
-__global__ void k_edge_add(float* __restrict__ z1, const uint16_t* __restrict__ PA,
-                           const uint16_t* __restrict__ PB, const uint32_t* __restrict__ src,
-                           const uint32_t* __restrict__ dst, size_t e) {
-  size_t count = e * kWidth;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t ed = k / kWidth;
-    int c = (int)(k % kWidth);
-    float z = z1[k] + from_bf16(PA[(size_t)dst[ed] * kWidth + c]);
-    z1[k] = z + from_bf16(PB[(size_t)src[ed] * kWidth + c]);
+    const size_t ed = k / (kWidth / 8), c = 8 * (k % (kWidth / 8));
+    const float4* zp = (const float4*)(z2 + ed * kWidth + c);
+    const float4* dp = (const float4*)(dS + (size_t)dst[ed] * kWidth + c);
+    uint32_t w[4];
+    for (int h = 0; h < 2; ++h) {
+      const float4 zz = zp[h], dd = dp[h];
+      w[2 * h] = (uint32_t)to_bf16(dd.x * dsilu(zz.x)) | ((uint32_t)to_bf16(dd.y * dsilu(zz.y)) << 16);
+      w[2 * h + 1] =
+          (uint32_t)to_bf16(dd.z * dsilu(zz.z)) | ((uint32_t)to_bf16(dd.w * dsilu(zz.w)) << 16);
+    }
+    *(u32x4*)(dz + ed * kWidth + c) = u32x4{w[0], w[1], w[2], w[3]};
   }
 }
 
@@ -697,6 +685,54 @@ __global__ __launch_bounds__(256) void k_segsum_rows(const uint16_t* __restrict_
   out[(size_t)i * kWidth + 2 * lane + 1] = a1;
 }
 
+// out[j] = sum over the edges e with src[e] = j of x[e] (bf16 rows, 128 wide),
+// when no neighbour list was cut short: neighbours are then mutual, so those
+// edges are j's own neighbours i, each at the place of j in i's list. One wave
+// per particle; four neighbours' lists, then their rows, in flight. (Adding
+// every row with atomics instead takes 357 us for 557,000 edges, this 53.)
+__global__ __launch_bounds__(256) void k_gather_rows(const uint16_t* __restrict__ x,
+                                                     const uint32_t* __restrict__ off,
+                                                     const uint32_t* __restrict__ src, uint32_t n,
+                                                     float* __restrict__ out) {
+  const uint32_t j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  if (j >= n) return;
+  const uint32_t k0 = off[j], k1 = off[j + 1];
+  float a0 = 0.f, a1 = 0.f;
+  for (uint32_t k = k0; k < k1; k += 4) {
+    uint32_t lo[4], hi[4], v[4][2];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      const bool on = k + u < k1;
+      const uint32_t i = on ? src[k + u] : j;
+      lo[u] = off[i];
+      hi[u] = on ? off[i + 1] : lo[u];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      static_assert(kMaxEdges == 128, "a list is two lanes' worth");
+      v[u][0] = lo[u] + lane < hi[u] ? src[lo[u] + lane] : 0xFFFFFFFFu;
+      v[u][1] = lo[u] + lane + 64u < hi[u] ? src[lo[u] + lane + 64u] : 0xFFFFFFFFu;
+    }
+    uint32_t w[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      const uint64_t b0 = __ballot(v[u][0] == j), b1 = __ballot(v[u][1] == j);
+      w[u] = 0u;
+      if (b0 | b1) {
+        const uint32_t e = lo[u] + (b0 ? (uint32_t)__builtin_ctzll(b0)
+                                       : 64u + (uint32_t)__builtin_ctzll(b1));
+        w[u] = *(const uint32_t*)(x + (size_t)e * kWidth + 2 * lane);
+      }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      a0 += from_bf16((uint16_t)(w[u] & 0xFFFFu));
+      a1 += from_bf16((uint16_t)(w[u] >> 16));
+    }
+  }
+  *(float2*)(out + (size_t)j * kWidth + 2 * lane) = make_float2(a0, a1);
+}
+
 // out[src[e]] += x[e] (atomics; 128 wide).
 __global__ void k_scatter_rows(const uint16_t* __restrict__ x, const uint32_t* __restrict__ src,
                                size_t e, float* __restrict__ out) {
@@ -712,52 +748,24 @@ __global__ void k_scatter_rows(const uint16_t* __restrict__ x, const uint32_t* _
   }
 }
 
-// Column sums (optionally row-weighted) atomically added into out[0..cols).
-// One thread per column over a chunk of 512 rows.
-template <typename T>
-__device__ inline float load_val(const T* p);
-template <>
-__device__ inline float load_val<float>(const float* p) { return *p; }
-template <>
-__device__ inline float load_val<uint16_t>(const uint16_t* p) { return from_bf16(*p); }
-
-template <typename T>
-__global__ void k_colsum(const T* __restrict__ x, int ldx, size_t rows, int cols,
-                         const float* __restrict__ rowscale, float* __restrict__ out) {
-  int c = threadIdx.x;
-  if (c >= cols) return;
-  size_t r0 = (size_t)blockIdx.x * 512, r1 = r0 + 512 < rows ? r0 + 512 : rows;
-  float a = 0.f;
-  for (size_t r = r0; r < r1; ++r) {
-    float v = load_val<T>(x + r * ldx + c);
-    a += rowscale ? v * rowscale[r] : v;
-  }
-  atomicAdd(out + c, a);
+// u1[:, 128:] = bf16([nu, 0...]) (the GEMM of M1 writes the first 128 of 144).
+__global__ __launch_bounds__(256) void k_tail_u1(const float* __restrict__ nu, uint32_t n,
+                                                 uint16_t* __restrict__ u1) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  u32x4* o = (u32x4*)(u1 + (size_t)i * kIn1 + kWidth);
+  o[0] = u32x4{(uint32_t)to_bf16(nu[2 * i]) | ((uint32_t)to_bf16(nu[2 * i + 1]) << 16), 0u, 0u, 0u};
+  o[1] = u32x4{0u, 0u, 0u, 0u};
 }
 
-// u1 = bf16([M1, nu, 0...]) (144 wide).
-__global__ void k_pack_u1(const float* __restrict__ M, const float* __restrict__ nu, uint32_t n,
-                          uint16_t* __restrict__ u1) {
-  size_t count = (size_t)n * kIn1;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t i = k / kIn1;
-    int c = (int)(k % kIn1);
-    float v = c < kWidth ? M[i * kWidth + c] : (c < kWidth + 2 ? nu[2 * i + c - kWidth] : 0.f);
-    u1[k] = to_bf16(v);
-  }
-}
-
-// u2 = [H (bf16), bf16(M2)] (256 wide).
-__global__ void k_pack_u2(const uint16_t* __restrict__ Hb, const float* __restrict__ M2,
-                          uint32_t n, uint16_t* __restrict__ u2) {
-  size_t count = (size_t)n * kIn2;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t i = k / kIn2;
-    int c = (int)(k % kIn2);
-    u2[k] = c < kWidth ? Hb[i * kWidth + c] : to_bf16(M2[i * kWidth + c - kWidth]);
-  }
+// u2[:, :128] = H (the GEMM of M2 writes the second half of 256); eight
+// features per thread.
+__global__ __launch_bounds__(256) void k_head_u2(const uint16_t* __restrict__ Hb, uint32_t n,
+                                                 uint16_t* __restrict__ u2) {
+  const size_t k = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (k >= (size_t)n * (kWidth / 8)) return;
+  const size_t i = k / (kWidth / 8), c = 8 * (k % (kWidth / 8));
+  *(u32x4*)(u2 + i * kIn2 + c) = *(const u32x4*)(Hb + i * kWidth + c);
 }
 
 // Loss = sum over particles and the 3 used outputs of (out - target)^2 / n;
@@ -848,7 +856,7 @@ void launch_edge_inputs(clsph_gnn* m, clsph_state* st) {
   hipStream_t s = st->ctx->stream;
   uint32_t n = m->n, e = m->e;
   const DevParams& d = st->host_dps[0];
-  hipLaunchKernelGGL(k_graph, grid_for(n), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
+  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
                      m->src, m->dst, m->degc);
   uint32_t cnt = e > n ? e : n;
   hipLaunchKernelGGL(k_edge_inputs, grid_for(cnt), dim3(256), 0, s, st->pos_s, st->vel_s,
@@ -860,60 +868,53 @@ static inline const float* P(const clsph_gnn* m, int id) { return m->params + pa
 static inline const uint16_t* W(const clsph_gnn* m, int id) { return m->wb + param_offset(id); }
 static inline float* G(clsph_gnn* m, int id) { return m->grad + param_offset(id); }
 
-// Edge MLP of one round: z1 (already holding e W1 + b1 [+ node terms]) ->
-// s1 -> z2 -> S = bf16(sum silu(z2) / C).
+// bf16(A B [+ rowscale bias]) into out16 (row stride ldo).
+static void gemm_cast(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* out16, int ldo,
+                      int M, const float* bias = nullptr, const float* rowscale = nullptr) {
+  nn::GemmArgs g{};
+  g.A = A, g.lda = kWidth, g.B = B, g.ldb = kWidth, g.out16 = out16, g.ldc = ldo;
+  g.M = M, g.N = kWidth, g.K = kWidth, g.alpha = 1.f, g.bias = bias, g.rowscale = rowscale;
+  gemm(s, false, false, nn::kEpiCast, g);
+}
+
+// Second and third layer of an edge round: s1 -> z2 -> S = bf16(sum silu(z2) / C).
 static void edge_tail(clsph_gnn* m, int r, int w2, int b2, hipStream_t s) {
-  size_t ew = (size_t)m->e * kWidth;
-  hipLaunchKernelGGL(k_silu_bf16, grid_for(ew), dim3(256), 0, s, m->z1[r], m->s1[r], ew);
   gemm(s, false, false, false, m->s1[r], kWidth, W(m, w2), kWidth, m->z2[r], kWidth, (int)m->e,
        kWidth, kWidth, 1.f, P(m, b2));
   hipLaunchKernelGGL(k_segsum_silu, dim3((m->n + 3) / 4), dim3(256), 0, s, m->z2[r], m->off,
                      m->n, 1.f / kAggC, m->S[r]);
 }
 
-// Three-layer SiLU MLP over n rows: input u (bf16, kin wide) ->
-// pre1/act1 -> pre2/act2 -> y (f32, kout wide).
-static void mlp3(clsph_gnn* m, const uint16_t* u, int kin, int w1, float* pre1, uint16_t* act1,
-                 float* pre2, uint16_t* act2, float* y, int kout, hipStream_t s) {
+// First two layers of a three-layer SiLU MLP over n rows: input u (bf16, kin
+// wide) -> pre1/act1 -> pre2/act2.
+static void mlp2(clsph_gnn* m, const uint16_t* u, int kin, int w1, float* pre1, uint16_t* act1,
+                 float* pre2, uint16_t* act2, hipStream_t s) {
   int n = (int)m->n;
-  size_t nw = (size_t)n * kWidth;
-  gemm(s, false, false, false, u, kin, W(m, w1), kWidth, pre1, kWidth, n, kWidth, kin, 1.f,
-       P(m, w1 + 1));
-  hipLaunchKernelGGL(k_silu_bf16, grid_for(nw), dim3(256), 0, s, pre1, act1, nw);
-  gemm(s, false, false, false, act1, kWidth, W(m, w1 + 2), kWidth, pre2, kWidth, n, kWidth,
-       kWidth, 1.f, P(m, w1 + 3));
-  hipLaunchKernelGGL(k_silu_bf16, grid_for(nw), dim3(256), 0, s, pre2, act2, nw);
-  gemm(s, false, false, false, act2, kWidth, W(m, w1 + 4), kout, y, kout, n, kout, kWidth, 1.f,
-       P(m, w1 + 5));
+  gemm_silu(s, u, kin, W(m, w1), kWidth, P(m, w1 + 1), pre1, act1, n, kWidth, kin);
+  gemm_silu(s, act1, kWidth, W(m, w1 + 2), kWidth, P(m, w1 + 3), pre2, act2, n, kWidth, kWidth);
 }
 
 // Node part of round 1: M1 from S[0], node MLP 1 -> H (bf16), and the
 // round-2 node terms PA = bf16(H Wa), PB = bf16(H Wb).
 static void node_round1(clsph_gnn* m, hipStream_t s) {
   int n = (int)m->n;
-  size_t nw = (size_t)n * kWidth;
-  gemm(s, false, false, false, m->S[0], kWidth, W(m, E1_W3), kWidth, m->tmp, kWidth, n, kWidth,
-       kWidth, 1.f, P(m, E1_B3), m->degc);
-  hipLaunchKernelGGL(k_pack_u1, grid_for((size_t)n * kIn1), dim3(256), 0, s, m->tmp, m->nu,
-                     m->n, m->u1);
-  mlp3(m, m->u1, kIn1, N1_W1, m->p1, m->y1, m->p2, m->y2, m->tmp, kWidth, s);
-  hipLaunchKernelGGL(k_cast, grid_for(nw), dim3(256), 0, s, m->tmp, m->Hb, nw);
-  gemm(s, false, false, false, m->Hb, kWidth, W(m, E2_WA), kWidth, m->tmp, kWidth, n, kWidth,
-       kWidth, 1.f);
-  hipLaunchKernelGGL(k_cast, grid_for(nw), dim3(256), 0, s, m->tmp, m->PA, nw);
-  gemm(s, false, false, false, m->Hb, kWidth, W(m, E2_WB), kWidth, m->tmp, kWidth, n, kWidth,
-       kWidth, 1.f);
-  hipLaunchKernelGGL(k_cast, grid_for(nw), dim3(256), 0, s, m->tmp, m->PB, nw);
+  gemm_cast(s, m->S[0], W(m, E1_W3), m->u1, kIn1, n, P(m, E1_B3), m->degc);
+  hipLaunchKernelGGL(k_tail_u1, grid_for(n), dim3(256), 0, s, m->nu, m->n, m->u1);
+  mlp2(m, m->u1, kIn1, N1_W1, m->p1, m->y1, m->p2, m->y2, s);
+  gemm_cast(s, m->y2, W(m, N1_W3), m->Hb, kWidth, n, P(m, N1_B3));
+  gemm_cast(s, m->Hb, W(m, E2_WA), m->PA, kWidth, n);
+  gemm_cast(s, m->Hb, W(m, E2_WB), m->PB, kWidth, n);
 }
 
 // Node part of round 2: M2 from S[1], node MLP 2 -> out, accelerations.
 static void node_round2(clsph_gnn* m, float4* acc, float gx, float gy, float gz, hipStream_t s) {
   int n = (int)m->n;
-  gemm(s, false, false, false, m->S[1], kWidth, W(m, E2_W3), kWidth, m->tmp, kWidth, n, kWidth,
-       kWidth, 1.f, P(m, E2_B3), m->degc);
-  hipLaunchKernelGGL(k_pack_u2, grid_for((size_t)n * kIn2), dim3(256), 0, s, m->Hb, m->tmp,
-                     m->n, m->u2);
-  mlp3(m, m->u2, kIn2, N2_W1, m->q1, m->w1, m->q2, m->w2, m->out, kOut, s);
+  gemm_cast(s, m->S[1], W(m, E2_W3), m->u2 + kWidth, kIn2, n, P(m, E2_B3), m->degc);
+  hipLaunchKernelGGL(k_head_u2, grid_for((size_t)n * (kWidth / 8)), dim3(256), 0, s, m->Hb, m->n,
+                     m->u2);
+  mlp2(m, m->u2, kIn2, N2_W1, m->q1, m->w1, m->q2, m->w2, s);
+  gemm(s, false, false, false, m->w2, kWidth, W(m, N2_W3), kOut, m->out, kOut, n, kOut, kWidth,
+       1.f, P(m, N2_B3));
   if (acc)
     hipLaunchKernelGGL(k_write_acc, grid_for(n), dim3(256), 0, s, m->out, m->n, gx, gy, gz, acc);
 }
@@ -923,16 +924,16 @@ void forward(clsph_gnn* m, const DevParams* dp, float4* acc, float gx, float gy,
   hipStream_t s = m->ctx->stream;
   int e = (int)m->e;
   // round 1 edges
-  gemm(s, false, false, false, m->E1, kFeat, W(m, E1_W1), kWidth, m->z1[0], kWidth, e, kWidth,
-       kFeat, 1.f, P(m, E1_B1));
+  gemm_silu(s, m->E1, kFeat, W(m, E1_W1), kWidth, P(m, E1_B1), m->z1[0], m->s1[0], e, kWidth,
+            kFeat);
   edge_tail(m, 0, E1_W2, E1_B2, s);
   node_round1(m, s);
-  // round 2 edges
-  gemm(s, false, false, false, m->E1, kFeat, W(m, E2_W1), kWidth, m->z1[1], kWidth, e, kWidth,
-       kFeat, 1.f, P(m, E2_B1));
-  size_t ew = (size_t)e * kWidth;
-  hipLaunchKernelGGL(k_edge_add, grid_for(ew), dim3(256), 0, s, m->z1[1], m->PA, m->PB, m->src,
-                     m->dst, (size_t)e);
+  // round 2 edges, with the node terms PA[dst] + PB[src]
+  nn::GemmArgs g{};
+  g.A = m->E1, g.lda = kFeat, g.B = W(m, E2_W1), g.ldb = kWidth, g.C = m->z1[1], g.ldc = kWidth;
+  g.M = e, g.N = kWidth, g.K = kFeat, g.alpha = 1.f, g.bias = P(m, E2_B1);
+  g.out16 = m->s1[1], g.row_add = m->PA, g.row_of = m->dst, g.row_add2 = m->PB, g.row_of2 = m->src;
+  gemm(s, false, false, nn::kEpiEdgeSilu, g);
   edge_tail(m, 1, E2_W2, E2_B2, s);
   node_round2(m, acc, gx, gy, gz, s);
 }
@@ -997,24 +998,13 @@ static void mlp3_back(clsph_gnn* m, int w1, const uint16_t* u, int kin, const fl
   int n = (int)m->n;
   // layer 3
   gemm(s, true, false, true, act2, kWidth, dy_b, kout, G(m, w1 + 4), kout, kWidth, kout, n, 1.f);
-  hipLaunchKernelGGL((k_colsum<float>), dim3((n + 511) / 512), dim3(kout), 0, s, dy, ldy,
-                     (size_t)n, kout, nullptr, G(m, w1 + 5));
-  gemm(s, false, true, false, dy_b, kout, W(m, w1 + 4), kout, m->dY, kWidth, n, kWidth, kout, 1.f);
-  hipLaunchKernelGGL(k_dsilu, grid_for((size_t)n * kWidth), dim3(256), 0, s, m->dY, kWidth, pre2,
-                     m->dpb, (size_t)n, kWidth);
-  // layer 2
-  gemm(s, true, false, true, act1, kWidth, m->dpb, kWidth, G(m, w1 + 2), kWidth, kWidth, kWidth, n,
-       1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), dim3((n + 511) / 512), dim3(kWidth), 0, s, m->dpb,
-                     kWidth, (size_t)n, kWidth, nullptr, G(m, w1 + 3));
-  gemm(s, false, true, false, m->dpb, kWidth, W(m, w1 + 2), kWidth, m->dY, kWidth, n, kWidth,
-       kWidth, 1.f);
-  hipLaunchKernelGGL(k_dsilu, grid_for((size_t)n * kWidth), dim3(256), 0, s, m->dY, kWidth, pre1,
-                     m->dpb, (size_t)n, kWidth);
+  colsum(s, dy, ldy, n, kout, nullptr, G(m, w1 + 5));
+  gemm_dsilu(s, dy_b, kout, W(m, w1 + 4), kout, pre2, m->dpb, n, kWidth, kout);
+  // layer 2; each work-group's rows of dpb are its own input and output
+  gemm_weight_grad(s, act1, kWidth, m->dpb, kWidth, G(m, w1 + 2), G(m, w1 + 3), kWidth, kWidth, n);
+  gemm_dsilu(s, m->dpb, kWidth, W(m, w1 + 2), kWidth, pre1, m->dpb, n, kWidth, kWidth);
   // layer 1
-  gemm(s, true, false, true, u, kin, m->dpb, kWidth, G(m, w1), kWidth, kin, kWidth, n, 1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), dim3((n + 511) / 512), dim3(kWidth), 0, s, m->dpb,
-                     kWidth, (size_t)n, kWidth, nullptr, G(m, w1 + 1));
+  gemm_weight_grad(s, u, kin, m->dpb, kWidth, G(m, w1), G(m, w1 + 1), kin, kWidth, n);
   gemm(s, false, true, false, m->dpb, kWidth, W(m, w1), kWidth, m->dY, kIn2, n, kin_used, kWidth,
        1.f);
 }
@@ -1024,31 +1014,20 @@ static void mlp3_back(clsph_gnn* m, int w1, const uint16_t* u, int kin, const fl
 static void edge_back(clsph_gnn* m, int r, int w1, int w2, int w3, const float* dM, int ldm,
                       hipStream_t s) {
   int n = (int)m->n, e = (int)m->e;
-  size_t ew = (size_t)e * kWidth;
   // bf16(dM) into dpb (n x 128)
   hipLaunchKernelGGL(k_cast_2d, grid_for((size_t)n * kWidth), dim3(256), 0, s, dM, ldm, m->dpb,
                      kWidth, (size_t)n, kWidth);
   gemm(s, true, false, true, m->S[r], kWidth, m->dpb, kWidth, G(m, w3), kWidth, kWidth, kWidth, n,
        1.f);
-  hipLaunchKernelGGL((k_colsum<float>), dim3((n + 511) / 512), dim3(kWidth), 0, s, dM, ldm,
-                     (size_t)n, kWidth, m->degc, G(m, w3 + 1));
+  colsum(s, dM, ldm, n, kWidth, m->degc, G(m, w3 + 1));
   gemm(s, false, true, false, m->dpb, kWidth, W(m, w3), kWidth, m->dS, kWidth, n, kWidth, kWidth,
        1.f / kAggC);
   // edges
-  hipLaunchKernelGGL(k_edge_dz, grid_for(ew), dim3(256), 0, s, m->dS, m->z2[r], m->dst, m->dz2,
-                     (size_t)e);
-  gemm(s, true, false, true, m->s1[r], kWidth, m->dz2, kWidth, G(m, w2), kWidth, kWidth, kWidth, e,
-       1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), dim3((e + 511) / 512), dim3(kWidth), 0, s, m->dz2,
-                     kWidth, (size_t)e, kWidth, nullptr, G(m, w2 + 1));
-  gemm(s, false, true, false, m->dz2, kWidth, W(m, w2), kWidth, m->ds1, kWidth, e, kWidth, kWidth,
-       1.f);
-  hipLaunchKernelGGL(k_dsilu, grid_for(ew), dim3(256), 0, s, m->ds1, kWidth, m->z1[r], m->dz1,
-                     (size_t)e, kWidth);
-  gemm(s, true, false, true, m->E1, kFeat, m->dz1, kWidth, G(m, w1), kWidth, kFeat, kWidth, e,
-       1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), dim3((e + 511) / 512), dim3(kWidth), 0, s, m->dz1,
-                     kWidth, (size_t)e, kWidth, nullptr, G(m, w1 + 1));
+  hipLaunchKernelGGL(k_edge_dz, grid_for((size_t)e * (kWidth / 8)), dim3(256), 0, s, m->dS,
+                     m->z2[r], m->dst, m->dz2, (size_t)e);
+  gemm_weight_grad(s, m->s1[r], kWidth, m->dz2, kWidth, G(m, w2), G(m, w2 + 1), kWidth, kWidth, e);
+  gemm_dsilu(s, m->dz2, kWidth, W(m, w2), kWidth, m->z1[r], m->dz1, e, kWidth, kWidth);
+  gemm_weight_grad(s, m->E1, kFeat, m->dz1, kWidth, G(m, w1), G(m, w1 + 1), kFeat, kWidth, e);
 }
 
 void backward(clsph_gnn* m) {
@@ -1073,9 +1052,14 @@ void backward(clsph_gnn* m) {
   edge_back(m, 1, E2_W1, E2_W2, E2_W3, m->dY + kWidth, kIn2, s);
   hipLaunchKernelGGL(k_segsum_rows, dim3((n + 3) / 4), dim3(256), 0, s, m->dz1, m->off, m->n,
                      m->dPA);
-  fill(m->dPB, nw, 0.f, s);
-  hipLaunchKernelGGL(k_scatter_rows, grid_for((size_t)m->e * (kWidth / 2)), dim3(256), 0, s,
-                     m->dz1, m->src, (size_t)m->e, m->dPB);
+  if (!m->cut) {
+    hipLaunchKernelGGL(k_gather_rows, dim3((m->n + 3) / 4), dim3(256), 0, s, m->dz1, m->off,
+                       m->src, m->n, m->dPB);
+  } else {
+    fill(m->dPB, nw, 0.f, s);
+    hipLaunchKernelGGL(k_scatter_rows, grid_for((size_t)m->e * (kWidth / 2)), dim3(256), 0, s,
+                       m->dz1, m->src, (size_t)m->e, m->dPB);
+  }
   hipLaunchKernelGGL(k_cast, grid_for(nw), dim3(256), 0, s, m->dPA, m->dPA_b, nw);
   hipLaunchKernelGGL(k_cast, grid_for(nw), dim3(256), 0, s, m->dPB, m->dPB_b, nw);
   gemm(s, true, false, true, m->Hb, kWidth, m->dPA_b, kWidth, G(m, E2_WA), kWidth, kWidth, kWidth,

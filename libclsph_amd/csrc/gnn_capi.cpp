@@ -21,11 +21,11 @@ void free_gnn(clsph_gnn* m) {
   dfree(m->off), dfree(m->src), dfree(m->dst), dfree(m->scan_part);
   dfree(m->E1), dfree(m->nu), dfree(m->degc);
   for (int r = 0; r < 2; ++r) dfree(m->z1[r]), dfree(m->s1[r]), dfree(m->z2[r]), dfree(m->S[r]);
-  dfree(m->tmp), dfree(m->u1), dfree(m->p1), dfree(m->y1), dfree(m->p2), dfree(m->y2);
+  dfree(m->u1), dfree(m->p1), dfree(m->y1), dfree(m->p2), dfree(m->y2);
   dfree(m->Hb), dfree(m->PA), dfree(m->PB), dfree(m->u2), dfree(m->q1), dfree(m->w1);
   dfree(m->q2), dfree(m->w2), dfree(m->out);
   dfree(m->target), dfree(m->loss), dfree(m->dout), dfree(m->dY), dfree(m->dpb), dfree(m->dS);
-  dfree(m->dz2), dfree(m->ds1), dfree(m->dz1), dfree(m->dPA), dfree(m->dPB), dfree(m->dH);
+  dfree(m->dz2), dfree(m->dz1), dfree(m->dPA), dfree(m->dPB), dfree(m->dH);
   dfree(m->dPA_b), dfree(m->dPB_b);
 }
 
@@ -42,9 +42,12 @@ int gnn_check_state(clsph_gnn* m, clsph_state* st) {
 // inputs; reads the edge count back (one synchronisation).
 int gnn_build_graph(clsph_gnn* m, clsph_state* st) {
   gnn::launch_graph(m, st);
-  HIPCK(m->ctx, hipMemcpyAsync(&m->e, m->off + st->n, sizeof(uint32_t), hipMemcpyDeviceToHost,
+  uint32_t end[2] = {0, 0};
+  HIPCK(m->ctx, hipMemcpyAsync(end, m->off + st->n, sizeof(end), hipMemcpyDeviceToHost,
                                m->ctx->stream));
   HIPCK(m->ctx, hipStreamSynchronize(m->ctx->stream));
+  m->e = end[0];
+  m->cut = end[1] != 0;
   if (m->e > m->e_cap)
     return fail(m->ctx, CLSPH_ENOMEM,
                 "neighbour graph has " + std::to_string(m->e) +
@@ -78,18 +81,18 @@ int clsph_gnn_create(clsph_ctx* ctx, uint32_t n_cap, uint32_t e_cap, clsph_gnn**
 #define AL(ptr, count) \
   if (rc == CLSPH_OK) rc = dalloc(ctx, &(ptr), (count))
   AL(m->params, P); AL(m->wb, P); AL(m->grad, P); AL(m->adam_m, P); AL(m->adam_v, P);
-  AL(m->off, N + 1); AL(m->src, E); AL(m->dst, E);
-  AL(m->scan_part, N / 1024 + 2);
+  AL(m->off, N + 2); AL(m->src, E); AL(m->dst, E);
+  AL(m->scan_part, 2 * (N / 1024 + 2));
   AL(m->E1, E * gnn::kFeat); AL(m->nu, 2 * N); AL(m->degc, N);
   for (int r = 0; r < 2; ++r) {
     AL(m->z1[r], E * Wd); AL(m->s1[r], E * Wd); AL(m->z2[r], E * Wd); AL(m->S[r], N * Wd);
   }
-  AL(m->tmp, N * gnn::kIn2); AL(m->u1, N * gnn::kIn1); AL(m->p1, N * Wd); AL(m->y1, N * Wd);
+  AL(m->u1, N * gnn::kIn1); AL(m->p1, N * Wd); AL(m->y1, N * Wd);
   AL(m->p2, N * Wd); AL(m->y2, N * Wd); AL(m->Hb, N * Wd); AL(m->PA, N * Wd); AL(m->PB, N * Wd);
   AL(m->u2, N * gnn::kIn2); AL(m->q1, N * Wd); AL(m->w1, N * Wd); AL(m->q2, N * Wd);
   AL(m->w2, N * Wd); AL(m->out, N * gnn::kOut);
   AL(m->target, 3 * N); AL(m->loss, 1); AL(m->dout, N * gnn::kOut); AL(m->dY, N * gnn::kIn2);
-  AL(m->dpb, N * gnn::kIn2); AL(m->dS, N * Wd); AL(m->dz2, E * Wd); AL(m->ds1, E * Wd);
+  AL(m->dpb, N * gnn::kIn2); AL(m->dS, N * Wd); AL(m->dz2, E * Wd);
   AL(m->dz1, E * Wd); AL(m->dPA, N * Wd); AL(m->dPB, N * Wd); AL(m->dH, N * Wd);
   AL(m->dPA_b, N * Wd); AL(m->dPB_b, N * Wd);
 #undef AL

@@ -79,7 +79,7 @@ struct clsph_nn {
   uint16_t* E1 = nullptr;       // e x 32 edge inputs
   float* nu = nullptr;          // n x 2
   float* degc = nullptr;        // deg / C
-  float* z = nullptr;           // e x 32 edge pre-activations
+  uint32_t* mask = nullptr;     // e: one bit per edge feature, z > 0
   uint16_t* S = nullptr;        // n x 32: bf16(sum_j relu(z) / C)
   uint16_t* u = nullptr;        // n x 64 node inputs
   float* p1 = nullptr;          // n x 64
@@ -95,7 +95,6 @@ struct clsph_nn {
   uint16_t* dout_b = nullptr;   // n x 32
   float* dY = nullptr;          // n x 64
   uint16_t* dpb = nullptr;      // n x 64
-  uint16_t* dz = nullptr;       // e x 32
   float* sum = nullptr;         // n x 3 acceleration sums of the mean target
   uint32_t* loc = nullptr;      // n: inverse of a state's ids
   uint32_t* inv = nullptr;      // n: inverse of a sort permutation
@@ -145,10 +144,43 @@ constexpr size_t kScratchBytes = size_t(8) << 20;
 // Device address of that workspace on `device` (which must be current),
 // looked up on the first call for the device.
 hipError_t scratch_address(int device, void** ptr);
-// The bf16 matrix-core GEMM (see nn.hip) for direct use and testing.
-void gemm_public(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
-                 const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
-                 const float* bias, const float* rowscale);
+// The bf16 matrix-core GEMM (nn.hip). What becomes of the product v:
+enum GemmEpilogue {
+  kEpiStore,     // C = v
+  kEpiAdd,       // C += v (atomics), and colsum += the column sums of B
+  kEpiSilu,      // C = v, out16 = bf16(silu(v))
+  kEpiEdgeSilu,  // v += row_add[row_of[m]] + row_add2[row_of2[m]] first, then as kEpiSilu
+  kEpiCast,      // out16 = bf16(v)
+  kEpiDsilu,     // out16 = bf16(v silu'(C)), C an input
+};
+struct GemmArgs {
+  const uint16_t* A;
+  const uint16_t* B;
+  float* C;
+  int M, N, K, lda, ldb, ldc;  // ldc: of C, out16 and the added rows
+  float alpha;
+  const float* bias;
+  const float* rowscale;
+  int k_chunk;
+  float* colsum;
+  uint16_t* out16;
+  const uint16_t* row_add;
+  const uint16_t* row_add2;
+  const uint32_t* row_of;
+  const uint32_t* row_of2;
+};
+void gemm(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g);
+void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
+          const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
+          const float* bias = nullptr, const float* rowscale = nullptr);
+void gemm_weight_grad(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+                      float* W, float* b, int M, int N, int K);
+void gemm_silu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+               const float* bias, float* C, uint16_t* out16, int M, int N, int K);
+void gemm_dsilu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+                const float* pre, uint16_t* out16, int M, int N, int K);
+void colsum(hipStream_t s, const float* x, int ldx, int rows, int cols, const float* rowscale,
+            float* out);
 
 }  // namespace nn
 }  // namespace clsph

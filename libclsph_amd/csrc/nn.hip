@@ -4,6 +4,7 @@
 // backward passes are sequences of these launches on the context stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -34,34 +35,90 @@ __device__ inline float dsilu(float x) {
   return s * (1.f + x * (1.f - s));
 }
 
-// ---------------------------------------------------------------------------
-// GEMM: C (f32, M x N, ldc) = alpha * op(A) op(B) [+ rowscale[m] * bias[n]]
-// (ADD: atomically added to C). op(A) is M x K: A row-major M x K (lda), or
-// with TA stored K x M. op(B) is K x N: B row-major K x N (ldb), or with TB
-// stored N x K. Tiles of 128 x 128, K steps of 32 through LDS, four waves of
-// 2 x 2 32x32x16 bf16 matrix-core blocks. blockIdx.z splits K into chunks of
-// k_chunk (a multiple of 32); with more than one chunk ADD must be set.
-// The contiguous dimension of each operand must be a multiple of 8 and
-// 16-byte aligned (checked by the host wrapper).
-constexpr int kTile = 128;
-constexpr int kStep = 32;
-constexpr int kLds = kStep + 8;  // u16 per LDS row (padding against bank conflicts)
+// Eight floats to bf16 (round to nearest even), as one vector conversion so
+// that each pair becomes one two-operand v_cvt_pk_bf16_f32.
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-struct GemmArgs {
-  const uint16_t* A;
-  const uint16_t* B;
-  float* C;
-  int M, N, K, lda, ldb, ldc;
-  float alpha;
-  const float* bias;
-  const float* rowscale;
-  int k_chunk;
+__device__ __attribute__((always_inline)) inline u32x4 pack8(const float v[8]) {
+  const f32x8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+  return __builtin_bit_cast(u32x4, __builtin_convertvector(x, bf16x8));
+}
+
+// Orders a wave's own LDS accesses (its lanes exchange data, no other wave is
+// involved).
+__device__ __attribute__((always_inline)) inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---------------------------------------------------------------------------
+// GEMM: op(A) op(B) of bf16 operands, accumulated in f32. op(A) is M x K: A
+// row-major M x K (lda), or with TA stored K x M. op(B) is K x N: B row-major
+// K x N (ldb), or with TB stored N x K. Tiles of 128 x 128, K steps of 64
+// through LDS (both operands as rows of K), four waves of 2 x 2 32x32x16 bf16
+// matrix-core blocks. blockIdx.z splits K into chunks of k_chunk (a multiple
+// of the step); with more than one chunk the epilogue adds. What becomes of
+// the product v = alpha op(A) op(B) [+ rowscale[m] * bias[n]] is the epilogue
+// (GemmArgs::epi). The contiguous dimension of each operand must be a
+// multiple of 8 and 16-byte aligned (checked by the host wrapper).
+//
+// The shapes here are long and thin (edges x 128, or a 128 x 128 weight
+// gradient over all edges), so a work-group does few steps and each is bound
+// by the latency of its loads: a step's loads are issued before the previous
+// step's products. An operand whose rows run across K is turned by 4 x 8
+// blocks in registers (16 byte permutes) on its way to LDS.
+constexpr int kTile = 128;
+constexpr int kStep = 64;
+// u16 per LDS row: 144 bytes put 16 rows' 16-byte reads on distinct banks
+constexpr int kLds = kStep + 8;
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// A 128 x 64 tile of an operand in flight: 64 bytes per thread.
+template <bool ACROSS>  // the operand's rows run across K
+struct TileLoad {
+  u32x4 v[4];
+  // row r0 + .. of `rows` (along M or N), K from k0 up to ke
+  __device__ inline void load(const uint16_t* __restrict__ P, int ld, int r0, int rows, int k0,
+                              int ke) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int r = ACROSS ? r0 + (t >> 4) * 8 : r0 + (t >> 3) + 32 * it;
+      const int k = ACROSS ? k0 + (t & 15) * 4 + it : k0 + (t & 7) * 8;
+      v[it] = u32x4{0u, 0u, 0u, 0u};
+      if (r < rows && k < ke)
+        v[it] = *(const u32x4*)(P + (ACROSS ? (size_t)k * ld + r : (size_t)r * ld + k));
+    }
+  }
+  __device__ inline void store(uint16_t* lds) const {
+    const int t = threadIdx.x;
+    if constexpr (!ACROSS) {
+#pragma unroll
+      for (int it = 0; it < 4; ++it)
+        *(u32x4*)(lds + ((t >> 3) + 32 * it) * kLds + (t & 7) * 8) = v[it];
+    } else {
+      uint16_t* at = lds + (t >> 4) * 8 * kLds + (t & 15) * 4;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        // rows 2p and 2p + 1: the low and high halves of dword p of each k
+        const uint2 lo = make_uint2(__builtin_amdgcn_perm(v[1][p], v[0][p], 0x05040100u),
+                                    __builtin_amdgcn_perm(v[3][p], v[2][p], 0x05040100u));
+        const uint2 hi = make_uint2(__builtin_amdgcn_perm(v[1][p], v[0][p], 0x07060302u),
+                                    __builtin_amdgcn_perm(v[3][p], v[2][p], 0x07060302u));
+        *(uint2*)(at + (2 * p) * kLds) = lo;
+        *(uint2*)(at + (2 * p + 1) * kLds) = hi;
+      }
+    }
+  }
 };
 
-template <bool TA, bool TB, bool ADD>
+template <bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[kTile * kLds];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[kTile * kLds];
+  __shared__ __attribute__((aligned(16))) uint16_t tiles[2 * kTile * kLds];
+  uint16_t* As = tiles;
+  uint16_t* Bs = tiles + kTile * kLds;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.x * kTile, n0 = blockIdx.y * kTile;
   const int kb = blockIdx.z * g.k_chunk;
@@ -71,41 +128,22 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j)
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
+  // column sums of B, in the first row of tiles' upper waves
+  const bool sums = EPI == kEpiAdd && g.colsum != nullptr && blockIdx.x == 0 && wm == 0;
+  float csum[2] = {0.f, 0.f};
+  TileLoad<TA> la;
+  TileLoad<!TB> lb;
+  la.load(g.A, g.lda, m0, g.M, kb, ke);
+  lb.load(g.B, g.ldb, n0, g.N, kb, ke);
   for (int k0 = kb; k0 < ke; k0 += kStep) {
-    for (int it = 0; it < 2; ++it) {
-      int idx = tid + 256 * it;
-      if (!TA) {
-        int m = idx >> 2, kq = (idx & 3) * 8;
-        int gm = m0 + m, gk = k0 + kq;
-        u32x4 v = zero;
-        if (gm < g.M && gk < ke) v = *(const u32x4*)(g.A + (size_t)gm * g.lda + gk);
-        *(u32x4*)(As + m * kLds + kq) = v;
-      } else {
-        int k = idx >> 4, mq = (idx & 15) * 8;
-        int gm = m0 + mq, gk = k0 + k;
-        u32x4 v = zero;
-        if (gm < g.M && gk < ke) v = *(const u32x4*)(g.A + (size_t)gk * g.lda + gm);
-        const uint16_t* e = (const uint16_t*)&v;
-        for (int t = 0; t < 8; ++t) As[(mq + t) * kLds + k] = e[t];
-      }
-      if (!TB) {
-        int k = idx >> 4, nq = (idx & 15) * 8;
-        int gn = n0 + nq, gk = k0 + k;
-        u32x4 v = zero;
-        if (gn < g.N && gk < ke) v = *(const u32x4*)(g.B + (size_t)gk * g.ldb + gn);
-        const uint16_t* e = (const uint16_t*)&v;
-        for (int t = 0; t < 8; ++t) Bs[(nq + t) * kLds + k] = e[t];
-      } else {
-        int n = idx >> 2, kq = (idx & 3) * 8;
-        int gn = n0 + n, gk = k0 + kq;
-        u32x4 v = zero;
-        if (gn < g.N && gk < ke) v = *(const u32x4*)(g.B + (size_t)gn * g.ldb + gk);
-        *(u32x4*)(Bs + n * kLds + kq) = v;
-      }
-    }
+    la.store(As);
+    lb.store(Bs);
     __syncthreads();
-    for (int ks = 0; ks < kStep; ks += 16) {
+    if (k0 + kStep < ke) {
+      la.load(g.A, g.lda, m0, g.M, k0 + kStep, ke);
+      lb.load(g.B, g.ldb, n0, g.N, k0 + kStep, ke);
+    }
+    for (int ks = 0; ks < kStep && k0 + ks < ke; ks += 16) {
       const int kk = ks + 8 * (lane >> 5);
       bf16x8 a[2], b[2];
       for (int i = 0; i < 2; ++i)
@@ -117,53 +155,203 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
       for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      if (EPI == kEpiAdd && sums) {
+        const bf16x2 one = {(__bf16)1.f, (__bf16)1.f};
+        for (int j = 0; j < 2; ++j)
+          for (int q = 0; q < 4; ++q)
+            csum[j] = __builtin_amdgcn_fdot2_f32_bf16(
+                (bf16x2){b[j][2 * q], b[j][2 * q + 1]}, one, csum[j], false);
+      }
     }
     __syncthreads();
   }
+  if (EPI == kEpiAdd && sums)
+    for (int j = 0; j < 2; ++j) {
+      const float c = csum[j] + __shfl_xor(csum[j], 32, 64);
+      const int col = n0 + wn + 32 * j + (lane & 31);
+      if (lane < 32 && col < g.N) atomicAdd(g.colsum + col, c);
+    }
   // D layout of the 32x32 block: register r of lane l holds
   // row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
-      for (int r = 0; r < 16; ++r) {
-        int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        int col = n0 + wn + 32 * j + (lane & 31);
-        if (row < g.M && col < g.N) {
-          float v = g.alpha * acc[i][j][r];
-          if (g.bias && blockIdx.z == 0) v += g.bias[col] * (g.rowscale ? g.rowscale[row] : 1.f);
-          float* c = g.C + (size_t)row * g.ldc + col;
-          if (ADD)
-            atomicAdd(c, v);
-          else
-            *c = v;
+  if constexpr (EPI == kEpiAdd || EPI == kEpiStore) {
+    for (int i = 0; i < 2; ++i)
+      for (int j = 0; j < 2; ++j)
+        for (int r = 0; r < 16; ++r) {
+          const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+          const int col = n0 + wn + 32 * j + (lane & 31);
+          if (row < g.M && col < g.N) {
+            float v = g.alpha * acc[i][j][r];
+            if (g.bias && blockIdx.z == 0)
+              v = __builtin_fmaf(g.bias[col], g.rowscale ? g.rowscale[row] : 1.f, v);
+            float* at = g.C + (size_t)row * g.ldc + col;
+            if constexpr (EPI == kEpiAdd) atomicAdd(at, v);
+            else *at = v;
+          }
         }
+  } else {
+    // The wave's 32 x 64 half turned through LDS, so that a lane has eight
+    // consecutive columns and its reads and bf16 stores are 16 bytes (N a
+    // multiple of 8). A 2-byte access per lane and register left these
+    // epilogues waiting on their loads: over 557,000 edges the silu' one took
+    // 196 us and the one with two gathered rows 255, now 78 and 98.
+    constexpr int kPitch = 64 + 4;
+    static_assert(4 * 32 * kPitch * sizeof(float) <= sizeof(tiles), "fits in the tiles' bytes");
+    float* turn = reinterpret_cast<float*>(tiles) + wave * 32 * kPitch;
+    for (int i = 0; i < 2; ++i) {
+      wave_fence();
+      for (int j = 0; j < 2; ++j)
+        for (int r = 0; r < 16; ++r)
+          turn[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kPitch + 32 * j + (lane & 31)] =
+              acc[i][j][r];
+      wave_fence();
+      const int col = n0 + wn + (lane & 7) * 8;
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int lr = 8 * it + (lane >> 3), row = m0 + wm + 32 * i + lr;
+        if (row >= g.M || col >= g.N) continue;
+        const float* tv = turn + lr * kPitch + (lane & 7) * 8;
+        float v[8];
+        if (g.bias) {
+          const float rs = g.rowscale ? g.rowscale[row] : 1.f;
+          for (int q = 0; q < 8; ++q) v[q] = __builtin_fmaf(g.bias[col + q], rs, g.alpha * tv[q]);
+        } else {
+          for (int q = 0; q < 8; ++q) v[q] = g.alpha * tv[q];
+        }
+        const size_t at = (size_t)row * g.ldc + col;
+        if constexpr (EPI == kEpiDsilu) {
+          const float4 x = *(const float4*)(g.C + at), y = *(const float4*)(g.C + at + 4);
+          const float pre[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+          for (int q = 0; q < 8; ++q) v[q] *= dsilu(pre[q]);
+        }
+        if constexpr (EPI == kEpiEdgeSilu) {
+          const u32x4 x = *(const u32x4*)(g.row_add + (size_t)g.row_of[row] * g.ldc + col);
+          const u32x4 y = *(const u32x4*)(g.row_add2 + (size_t)g.row_of2[row] * g.ldc + col);
+          for (int q = 0; q < 8; ++q) {
+            v[q] += from_bf16((uint16_t)(x[q >> 1] >> (16 * (q & 1))));
+            v[q] += from_bf16((uint16_t)(y[q >> 1] >> (16 * (q & 1))));
+          }
+        }
+        if constexpr (EPI == kEpiSilu || EPI == kEpiEdgeSilu) {
+          *(float4*)(g.C + at) = make_float4(v[0], v[1], v[2], v[3]);
+          *(float4*)(g.C + at + 4) = make_float4(v[4], v[5], v[6], v[7]);
+          for (int q = 0; q < 8; ++q) v[q] = silu(v[q]);
+        }
+        *(u32x4*)(g.out16 + at) = pack8(v);
       }
+    }
+  }
 }
 
-// Host wrapper. `add` accumulates atomically; large-K products (K > 4096)
-// are split over the K dimension, which requires `add`.
-void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
-          const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
-          const float* bias = nullptr, const float* rowscale = nullptr) {
-  if (M <= 0 || N <= 0 || K <= 0) return;
-  GemmArgs g{A, B, C, M, N, K, lda, ldb, ldc, alpha, bias, rowscale, 0};
+// Fills the shape's split of K and launches. Adding products are split over K
+// until about two work-groups per compute unit share it, 256 of K each at
+// least: a weight gradient over 16,384 particles runs on 64 work-groups, not
+// on 4 (311 -> 15 us), over 557,000 edges on 512, not on 136 (357 -> 55).
+void gemm(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g) {
+  if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
+  const int mt = (g.M + kTile - 1) / kTile, nt = (g.N + kTile - 1) / kTile;
   int splits = 1;
-  if (add && K > 4096) splits = (K + 4095) / 4096;
-  if (splits > 1024) splits = 1024;
-  int chunk = (K + splits - 1) / splits;
+  if (epi == kEpiAdd) {
+    splits = 512 / (mt * nt);
+    if (splits > g.K / 256) splits = g.K / 256;
+    if (splits < 1) splits = 1;
+  }
+  int chunk = (g.K + splits - 1) / splits;
   chunk = (chunk + kStep - 1) / kStep * kStep;
-  splits = (K + chunk - 1) / chunk;
+  splits = (g.K + chunk - 1) / chunk;
   g.k_chunk = chunk;
-  dim3 grid((M + kTile - 1) / kTile, (N + kTile - 1) / kTile, splits);
+  dim3 grid(mt, nt, splits);
 #define GEMM_CASE(a, b, c)                                                   \
-  if (ta == a && tb == b && add == c) {                                      \
+  if (ta == a && tb == b && epi == c) {                                      \
     hipLaunchKernelGGL((k_gemm<a, b, c>), grid, dim3(256), 0, s, g);         \
     return;                                                                  \
   }
-  GEMM_CASE(false, false, false) GEMM_CASE(false, false, true)
-  GEMM_CASE(false, true, false) GEMM_CASE(false, true, true)
-  GEMM_CASE(true, false, false) GEMM_CASE(true, false, true)
-  GEMM_CASE(true, true, false) GEMM_CASE(true, true, true)
+  GEMM_CASE(false, false, kEpiStore) GEMM_CASE(false, false, kEpiAdd)
+  GEMM_CASE(false, true, kEpiStore) GEMM_CASE(false, true, kEpiAdd)
+  GEMM_CASE(true, false, kEpiStore) GEMM_CASE(true, false, kEpiAdd)
+  GEMM_CASE(true, true, kEpiStore) GEMM_CASE(true, true, kEpiAdd)
+  GEMM_CASE(false, false, kEpiSilu) GEMM_CASE(false, false, kEpiEdgeSilu)
+  GEMM_CASE(false, false, kEpiCast) GEMM_CASE(false, true, kEpiDsilu)
 #undef GEMM_CASE
+}
+
+// C = alpha op(A) op(B) [+ rowscale[m] * bias[n]], or added to C with `add`.
+void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
+          const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
+          const float* bias, const float* rowscale) {
+  GemmArgs g{};
+  g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = C, g.ldc = ldc;
+  g.M = M, g.N = N, g.K = K, g.alpha = alpha, g.bias = bias, g.rowscale = rowscale;
+  gemm(s, ta, tb, add ? kEpiAdd : kEpiStore, g);
+}
+
+// A weight gradient and its bias gradient: W (M x N) += A^T B, b (N) += the
+// column sums of B; A is K x M, B is K x N.
+void gemm_weight_grad(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+                      float* W, float* b, int M, int N, int K) {
+  GemmArgs g{};
+  g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = W, g.ldc = N;
+  g.M = M, g.N = N, g.K = K, g.alpha = 1.f, g.colsum = b;
+  gemm(s, true, false, kEpiAdd, g);
+}
+
+// Column sums (optionally row-weighted) of f32 rows, `cols` of them (a
+// multiple of 4, at most 128), added into out: 256 rows per work-group, 16
+// bytes per thread and row, joined through LDS.
+__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ x, int ldx, int rows,
+                                                int cols, const float* __restrict__ rowscale,
+                                                float* __restrict__ out) {
+  __shared__ float4 red[256];
+  const int quads = cols / 4, per = 256 / quads;  // threads per row, rows in flight
+  const int q = threadIdx.x % quads, r = threadIdx.x / quads;
+  const int r0 = blockIdx.x * 256, r1 = min(r0 + 256, rows);
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (r < per) {
+#pragma unroll 4
+    for (int k = r0 + r; k < r1; k += per) {
+      const float4 v = *(const float4*)(x + (size_t)k * ldx + 4 * q);
+      const float w = rowscale ? rowscale[k] : 1.f;
+      a.x += v.x * w, a.y += v.y * w, a.z += v.z * w, a.w += v.w * w;
+    }
+  }
+  red[threadIdx.x] = a;
+  __syncthreads();
+  if (r == 0) {
+    for (int k = 1; k < per; ++k) {
+      const float4 v = red[k * quads + q];
+      a.x += v.x, a.y += v.y, a.z += v.z, a.w += v.w;
+    }
+    atomicAdd(out + 4 * q, a.x);
+    atomicAdd(out + 4 * q + 1, a.y);
+    atomicAdd(out + 4 * q + 2, a.z);
+    atomicAdd(out + 4 * q + 3, a.w);
+  }
+}
+
+void colsum(hipStream_t s, const float* x, int ldx, int rows, int cols, const float* rowscale,
+            float* out) {
+  if (rows > 0)
+    hipLaunchKernelGGL(k_colsum, dim3((rows + 255) / 256), dim3(256), 0, s, x, ldx, rows, cols,
+                       rowscale, out);
+}
+
+// C = A B + bias and out16 = bf16(silu(C)).
+void gemm_silu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+               const float* bias, float* C, uint16_t* out16, int M, int N, int K) {
+  GemmArgs g{};
+  g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = C, g.ldc = N, g.out16 = out16;
+  g.M = M, g.N = N, g.K = K, g.alpha = 1.f, g.bias = bias;
+  gemm(s, false, false, kEpiSilu, g);
+}
+
+// out16 = bf16(A B^T silu'(pre)); out16 may be A itself when N fits one tile
+// (a work-group's rows are then read by no other).
+void gemm_dsilu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int ldb,
+                const float* pre, uint16_t* out16, int M, int N, int K) {
+  GemmArgs g{};
+  g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = const_cast<float*>(pre), g.ldc = N;
+  g.out16 = out16;
+  g.M = M, g.N = N, g.K = K, g.alpha = 1.f;
+  gemm(s, false, true, kEpiDsilu, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -234,7 +422,8 @@ __global__ __launch_bounds__(256) void k_scan_add(uint32_t* __restrict__ off,
 
 // ---------------------------------------------------------------------------
 
-// src / dst of every edge (dst-major, the density kernel's neighbour order).
+// src / dst of every edge (dst-major, the density kernel's neighbour order);
+// blockIdx.y of gridDim.y takes every gridDim.y-th group of four neighbours.
 __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
                                                const uint32_t* __restrict__ count,
                                                const uint32_t* __restrict__ off, uint32_t n,
@@ -244,7 +433,7 @@ __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
   uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   uint32_t deg = min(count[i], kMaxEdges), o = off[i];
-  for (uint32_t q = 0; q < deg; q += 4) {
+  for (uint32_t q = 4 * blockIdx.y; q < deg; q += 4 * gridDim.y) {
     uint4 js = nbr[(size_t)(q >> 2) * n + i];
     uint32_t jj[4] = {js.x, js.y, js.z, js.w};
     for (uint32_t t = 0; t < 4 && q + t < deg; ++t) {
@@ -252,7 +441,7 @@ __global__ __launch_bounds__(256) void k_graph(const uint4* __restrict__ nbr,
       dst[o + q + t] = i;
     }
   }
-  degc[i] = (float)deg / kAggC;
+  if (blockIdx.y == 0) degc[i] = (float)deg / kAggC;
 }
 
 // Constants of the edge inputs (one scene).
@@ -455,15 +644,6 @@ constexpr int kTileP = 16;                 // particles per tile (MFMA columns)
 constexpr int kSurWaves = 8;               // waves per work-group
 constexpr int kColBytes = 4 * 64 + 16;     // LDS bytes per particle column
 constexpr int kWaveLds = kTileP * kColBytes;
-
-// Eight floats to bf16 (round to nearest even), as one vector conversion so
-// that each pair becomes one two-operand v_cvt_pk_bf16_f32.
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-
-__device__ __attribute__((always_inline)) inline u32x4 pack8(const float v[8]) {
-  const f32x8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-  return __builtin_bit_cast(u32x4, __builtin_convertvector(x, bf16x8));
-}
 
 // Stages W (row-major, rows = inputs, ld = outputs) for k-steps
 // [ks0, ks0 + nks) of a layer with `ks_total` k-steps and `nob` 16-wide
@@ -737,98 +917,190 @@ __global__ __launch_bounds__(kSurWaves * 64) void k_surrogate(
 
 // ---------------------------------------------------------------------------
 // Training-path kernels (grid-stride loops unless noted).
-__global__ void k_silu_bf16(const float* __restrict__ z, uint16_t* __restrict__ s, size_t count) {
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x)
-    s[k] = to_bf16(silu(z[k]));
-}
-
-// dz = bf16(dy * silu'(p)); dy has row stride ldy, p and dz are dense.
-__global__ void k_dsilu(const float* __restrict__ dy, int ldy, const float* __restrict__ p,
-                        uint16_t* __restrict__ dz, size_t rows, int cols) {
-  size_t count = rows * cols;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t r = k / cols;
-    int c = (int)(k % cols);
-    dz[k] = to_bf16(dy[r * ldy + c] * dsilu(p[k]));
-  }
-}
-
-// S[i][c] = bf16(sum over i's edges of relu(z[e][c]) / C); thread per (i, c).
-__global__ __launch_bounds__(256) void k_segsum_relu(const float* __restrict__ z,
-                                                     const uint32_t* __restrict__ off, uint32_t n,
-                                                     uint16_t* __restrict__ S) {
-  const size_t count = (size_t)n * kEdgeW;
-  for (size_t t = blockIdx.x * (size_t)256 + threadIdx.x; t < count;
-       t += (size_t)gridDim.x * 256) {
-    uint32_t i = (uint32_t)(t / kEdgeW);
-    int c = (int)(t % kEdgeW);
-    float a = 0.f;
-    for (uint32_t k = off[i]; k < off[i + 1]; ++k) a += fmaxf(z[(size_t)k * kEdgeW + c], 0.f);
-    S[t] = to_bf16(a * (1.f / kAggC));
-  }
-}
-
-// u = bf16([S, nu, (a0 - g) / A, deg / C, 0...]) (64 wide).
-__global__ void k_pack_u(const uint16_t* __restrict__ S, const float* __restrict__ nu,
-                         const float4* __restrict__ acc0, const float* __restrict__ degc,
-                         uint32_t n, float gx, float gy, float gz, uint16_t* __restrict__ u) {
-  size_t count = (size_t)n * kIn;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t i = k / kIn;
-    int c = (int)(k % kIn);
-    if (c < kEdgeW) {
-      u[k] = S[i * kEdgeW + c];
-      continue;
+// The edge layer of the training forward pass and its neighbour sum:
+// z = e W1 + b1, S[i] = bf16(sum over i's edges of relu(z) / C), and for the
+// backward pass one bit per (edge, feature), z > 0. A work-group takes
+// kEdgeParts consecutive particles, whose edges are consecutive; 128 at a
+// time pass through the matrix cores into LDS, where 32 threads per particle
+// (one per feature) sum them in order. Reads the 64 bytes of each edge's
+// inputs and writes 4 (storing z and summing it in a second pass had moved
+// 64 + 128 + 128): 120 us for 5 million edges, 688 as the two passes.
+constexpr uint32_t kEdgeParts = 32;
+__global__ __launch_bounds__(256) void k_edge_layer(const uint16_t* __restrict__ E1,
+                                                    const uint16_t* __restrict__ W1,
+                                                    const float* __restrict__ b1,
+                                                    const uint32_t* __restrict__ off, uint32_t n,
+                                                    uint16_t* __restrict__ S,
+                                                    uint32_t* __restrict__ mask) {
+  static_assert(kEdgeW == 32 && kFeat == 32, "one 32x32 block per 32 edges");
+  constexpr uint32_t kChunk = 128;
+  __shared__ float zs[kChunk][kEdgeW + 1];
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6, col = lane & 31u, half = lane >> 5;
+  const uint32_t i0 = blockIdx.x * kEdgeParts, i1 = min(n, i0 + kEdgeParts);
+  const uint32_t e0 = off[i0], e1 = off[i1];
+  // W1's operands (k-steps of 16, lane: column `col`, 8 inputs from 8 half)
+  bf16x8 w[2];
+  for (int ks = 0; ks < 2; ++ks) {
+    uint32_t d[4];
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t k = 16 * ks + 8 * half + 2 * q;
+      d[q] = (uint32_t)W1[k * kEdgeW + col] | ((uint32_t)W1[(k + 1) * kEdgeW + col] << 16);
     }
-    float v = 0.f;
+    w[ks] = __builtin_bit_cast(bf16x8, u32x4{d[0], d[1], d[2], d[3]});
+  }
+  const float bias = b1[col];
+  // particle i0 + p is summed by the threads of group p % 8
+  const uint32_t grp = t >> 5, c = t & 31u;
+  uint32_t pe0[kEdgeParts / 8], pe1[kEdgeParts / 8];
+  float sum[kEdgeParts / 8];
+#pragma unroll
+  for (uint32_t q = 0; q < kEdgeParts / 8; ++q) {
+    const uint32_t i = i0 + 8 * q + grp;
+    pe0[q] = i < i1 ? off[i] : 0u;
+    pe1[q] = i < i1 ? off[i + 1] : 0u;
+    sum[q] = 0.f;
+  }
+  for (uint32_t c0 = e0; c0 < e1; c0 += kChunk) {
+    const uint32_t er = c0 + 32 * wave + col;
+    bf16x8 a[2];
+    for (int ks = 0; ks < 2; ++ks) {
+      u32x4 v = {0u, 0u, 0u, 0u};
+      if (er < e1) v = *(const u32x4*)(E1 + (size_t)er * kFeat + 16 * ks + 8 * half);
+      a[ks] = __builtin_bit_cast(bf16x8, v);
+    }
+    f32x16 z;
+    for (int r = 0; r < 16; ++r) z[r] = 0.f;
+    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], w[0], z, 0, 0, 0);
+    z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], w[1], z, 0, 0, 0);
+    // register r: edge 8 (r / 4) + 4 half + r % 4 of the wave's 32, feature col
+    uint32_t bits = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t row = 8 * (r >> 2) + (r & 3);
+      const float v = z[r] + bias;
+      const uint64_t on = __ballot(v > 0.f);
+      bits = col == row ? (uint32_t)on : (col == row + 4u ? (uint32_t)(on >> 32) : bits);
+      zs[32 * wave + row + 4 * half][col] = fmaxf(v, 0.f);
+    }
+    if (half == 0u && er < e1) mask[er] = bits;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kEdgeParts / 8; ++q) {
+      const uint32_t k0 = max(pe0[q], c0), k1 = min(pe1[q], c0 + kChunk);
+      for (uint32_t k = k0; k < k1; ++k) sum[q] += zs[k - c0][c];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < kEdgeParts / 8; ++q) {
+    const uint32_t i = i0 + 8 * q + grp;
+    if (i < i1) S[(size_t)i * kEdgeW + c] = to_bf16(sum[q] * (1.f / kAggC));
+  }
+}
+
+// The edge layer's gradients from d loss / d S (dY, row stride ldy):
+// dz[e] = bf16(dY[dst[e]] / C) where the forward pass found z > 0, else 0;
+// W += E1^T dz, b += the column sums of dz. A work-group takes `per`
+// consecutive edges, 256 at a time: both operands are turned in registers
+// into LDS rows of edges, and each wave multiplies a quarter of them. 193 us
+// for 5 million edges; as three passes (dz, the product, the column sums) 945.
+__global__ __launch_bounds__(256) void k_edge_grad(const uint16_t* __restrict__ E1,
+                                                   const float* __restrict__ dY, int ldy,
+                                                   const uint32_t* __restrict__ mask,
+                                                   const uint32_t* __restrict__ dst, uint32_t e,
+                                                   uint32_t per, float* __restrict__ W,
+                                                   float* __restrict__ b) {
+  static_assert(kEdgeW == 32 && kFeat == 32, "one 32x32 block");
+  constexpr int kRow = 256 + 8;  // u16 per LDS row of edges
+  __shared__ __attribute__((aligned(16))) uint16_t As[32 * kRow];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[32 * kRow];
+  __shared__ float red[3][32][33];
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const uint32_t b0 = blockIdx.x * per, b1 = min(e, b0 + per);
+  const uint32_t eq = (t >> 2) * 4u, f = (t & 3u) * 8u;  // 4 edges x 8 features per thread
+  f32x16 acc;
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  float csum = 0.f;
+  for (uint32_t c0 = b0; c0 < b1; c0 += 256u) {
+    u32x4 va[4], vb[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t ed = c0 + eq + u;
+      va[u] = vb[u] = u32x4{0u, 0u, 0u, 0u};
+      if (ed < b1) {
+        va[u] = *(const u32x4*)(E1 + (size_t)ed * kFeat + f);
+        const float4* dp = (const float4*)(dY + (size_t)dst[ed] * ldy + f);
+        const float4 x = dp[0], y = dp[1];
+        const float d[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        const uint32_t m = mask[ed] >> f;
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = (m >> q) & 1u ? d[q] * (1.f / kAggC) : 0.f;
+        vb[u] = pack8(v);
+      }
+    }
+    __syncthreads();  // the previous products have read LDS
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      uint16_t* ta = As + (f + 2 * p) * kRow + eq;
+      uint16_t* tb = Bs + (f + 2 * p) * kRow + eq;
+      *(uint2*)ta = make_uint2(__builtin_amdgcn_perm(va[1][p], va[0][p], 0x05040100u),
+                               __builtin_amdgcn_perm(va[3][p], va[2][p], 0x05040100u));
+      *(uint2*)(ta + kRow) = make_uint2(__builtin_amdgcn_perm(va[1][p], va[0][p], 0x07060302u),
+                                        __builtin_amdgcn_perm(va[3][p], va[2][p], 0x07060302u));
+      *(uint2*)tb = make_uint2(__builtin_amdgcn_perm(vb[1][p], vb[0][p], 0x05040100u),
+                               __builtin_amdgcn_perm(vb[3][p], vb[2][p], 0x05040100u));
+      *(uint2*)(tb + kRow) = make_uint2(__builtin_amdgcn_perm(vb[1][p], vb[0][p], 0x07060302u),
+                                        __builtin_amdgcn_perm(vb[3][p], vb[2][p], 0x07060302u));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < 64; ks += 16) {
+      const uint32_t at = (lane & 31u) * kRow + 64u * wave + ks + 8u * (lane >> 5);
+      const bf16x8 a = __builtin_bit_cast(bf16x8, *(const u32x4*)(As + at));
+      const bf16x8 bb = __builtin_bit_cast(bf16x8, *(const u32x4*)(Bs + at));
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, acc, 0, 0, 0);
+      const bf16x2 one = {(__bf16)1.f, (__bf16)1.f};
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        csum = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){bb[2 * q], bb[2 * q + 1]}, one, csum, false);
+    }
+  }
+  csum += __shfl_xor(csum, 32, 64);
+  if (lane < 32u) atomicAdd(b + lane, csum);
+  if (wave)
+    for (int r = 0; r < 16; ++r)
+      red[wave - 1][8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)][lane & 31u] = acc[r];
+  __syncthreads();
+  if (wave == 0)
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t row = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), cc = lane & 31u;
+      atomicAdd(W + row * kEdgeW + cc, acc[r] + red[0][row][cc] + red[1][row][cc] + red[2][row][cc]);
+    }
+}
+
+// u = bf16([S, nu, (a0 - g) / A, deg / C, 0...]) (64 wide), eight values per
+// thread.
+__global__ __launch_bounds__(256) void k_pack_u(const uint16_t* __restrict__ S,
+                                                const float* __restrict__ nu,
+                                                const float4* __restrict__ acc0,
+                                                const float* __restrict__ degc, uint32_t n,
+                                                float gx, float gy, float gz,
+                                                uint16_t* __restrict__ u) {
+  const size_t k = blockIdx.x * (size_t)256 + threadIdx.x;
+  if (k >= (size_t)n * (kIn / 8)) return;
+  const size_t i = k / (kIn / 8), c = 8 * (k % (kIn / 8));
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (c < kEdgeW) {
+    v = *(const u32x4*)(S + i * kEdgeW + c);
+  } else if (c == kEdgeW) {
     const float4 a = acc0[i];
-    switch (c - kEdgeW) {
-      case 0: v = nu[2 * i]; break;
-      case 1: v = nu[2 * i + 1]; break;
-      case 2: v = (a.x - gx) * (1.f / kAccScale); break;
-      case 3: v = (a.y - gy) * (1.f / kAccScale); break;
-      case 4: v = (a.z - gz) * (1.f / kAccScale); break;
-      case 5: v = degc[i]; break;
-      default: break;
-    }
-    u[k] = to_bf16(v);
+    const float x[8] = {nu[2 * i], nu[2 * i + 1], (a.x - gx) * (1.f / kAccScale),
+                        (a.y - gy) * (1.f / kAccScale), (a.z - gz) * (1.f / kAccScale), degc[i],
+                        0.f, 0.f};
+    v = pack8(x);
   }
-}
-
-// dz[e][c] = bf16(dY[dst[e]][c] / C) where z[e][c] > 0, else 0.
-__global__ void k_edge_dz(const float* __restrict__ dY, int ldy, const float* __restrict__ z,
-                          const uint32_t* __restrict__ dst, uint16_t* __restrict__ dz, size_t e) {
-  size_t count = e * kEdgeW;
-  for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < count;
-       k += (size_t)gridDim.x * blockDim.x) {
-    size_t ed = k / kEdgeW;
-    int c = (int)(k % kEdgeW);
-    float d = z[k] > 0.f ? dY[(size_t)dst[ed] * ldy + c] * (1.f / kAggC) : 0.f;
-    dz[k] = to_bf16(d);
-  }
-}
-
-// Column sums (optionally row-weighted) atomically added into out[0..cols).
-// One thread per column over a chunk of 512 rows.
-template <typename T>
-__device__ inline float load_val(const T* p);
-template <>
-__device__ inline float load_val<float>(const float* p) { return *p; }
-template <>
-__device__ inline float load_val<uint16_t>(const uint16_t* p) { return from_bf16(*p); }
-
-template <typename T>
-__global__ void k_colsum(const T* __restrict__ x, int ldx, size_t rows, int cols,
-                         float* __restrict__ out) {
-  int c = threadIdx.x;
-  if (c >= cols) return;
-  size_t r0 = (size_t)blockIdx.x * 512, r1 = r0 + 512 < rows ? r0 + 512 : rows;
-  float a = 0.f;
-  for (size_t r = r0; r < r1; ++r) a += load_val<T>(x + r * ldx + c);
-  atomicAdd(out + c, a);
+  *(u32x4*)(u + i * kIn + c) = v;
 }
 
 // Loss = sum over particles and the 3 used outputs of (out - target)^2 / n;
@@ -1036,7 +1308,7 @@ void launch_edge_inputs(clsph_nn* m, clsph_state* st) {
   hipStream_t s = st->ctx->stream;
   uint32_t n = m->n, e = m->e;
   const DevParams& d = st->host_dps[0];
-  hipLaunchKernelGGL(k_graph, grid_for(n), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
+  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
                      m->src, m->dst, m->degc);
   hipLaunchKernelGGL(k_node_inputs, grid_for(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
                      d.p.fluid_density, d.p.K, (float2*)m->nu);
@@ -1050,20 +1322,14 @@ static inline float* G(clsph_nn* m, int id) { return m->grad + param_offset(id);
 
 void forward(clsph_nn* m, const float4* acc0, float gx, float gy, float gz) {
   hipStream_t s = m->ctx->stream;
-  int n = (int)m->n, e = (int)m->e;
-  size_t nw = (size_t)n * kNodeW;
-  gemm(s, false, false, false, m->E1, kFeat, W(m, E_W1), kEdgeW, m->z, kEdgeW, e, kEdgeW, kFeat,
-       1.f, P(m, E_B1));
-  hipLaunchKernelGGL(k_segsum_relu, grid_for((size_t)n * kEdgeW), dim3(256), 0, s, m->z, m->off,
-                     m->n, m->S);
-  hipLaunchKernelGGL(k_pack_u, grid_for((size_t)n * kIn), dim3(256), 0, s, m->S, m->nu, acc0,
+  const int n = (int)m->n;
+  if (n)
+    hipLaunchKernelGGL(k_edge_layer, dim3((m->n + kEdgeParts - 1) / kEdgeParts), dim3(256), 0, s,
+                       m->E1, W(m, E_W1), P(m, E_B1), m->off, m->n, m->S, m->mask);
+  hipLaunchKernelGGL(k_pack_u, dim3((uint32_t)(((size_t)n * (kIn / 8) + 255) / 256)), dim3(256), 0, s, m->S, m->nu, acc0,
                      m->degc, m->n, gx, gy, gz, m->u);
-  gemm(s, false, false, false, m->u, kIn, W(m, N_W1), kNodeW, m->p1, kNodeW, n, kNodeW, kIn, 1.f,
-       P(m, N_B1));
-  hipLaunchKernelGGL(k_silu_bf16, grid_for(nw), dim3(256), 0, s, m->p1, m->y1, nw);
-  gemm(s, false, false, false, m->y1, kNodeW, W(m, N_W2), kNodeW, m->p2, kNodeW, n, kNodeW,
-       kNodeW, 1.f, P(m, N_B2));
-  hipLaunchKernelGGL(k_silu_bf16, grid_for(nw), dim3(256), 0, s, m->p2, m->y2, nw);
+  gemm_silu(s, m->u, kIn, W(m, N_W1), kNodeW, P(m, N_B1), m->p1, m->y1, n, kNodeW, kIn);
+  gemm_silu(s, m->y1, kNodeW, W(m, N_W2), kNodeW, P(m, N_B2), m->p2, m->y2, n, kNodeW, kNodeW);
   gemm(s, false, false, false, m->y2, kNodeW, W(m, N_W3), kOut, m->out, kOut, n, kOut, kNodeW,
        1.f, P(m, N_B3));
 }
@@ -1107,45 +1373,32 @@ void forward_fused(clsph_nn* m, clsph_state* st, float4* acc, float* out, bool o
 void backward(clsph_nn* m) {
   hipStream_t s = m->ctx->stream;
   int n = (int)m->n, e = (int)m->e;
-  size_t nw = (size_t)n * kNodeW;
   fill(m->grad, kParamTotal, 0.f, s);
   fill(m->loss, 1, 0.f, s);
   hipLaunchKernelGGL(k_loss, grid_for(n), dim3(256), 0, s, m->out, m->target, m->n, m->dout,
                      m->loss);
   hipLaunchKernelGGL(k_cast, grid_for((size_t)n * kOut), dim3(256), 0, s, m->dout, m->dout_b,
                      (size_t)n * kOut);
-  const dim3 nchunks((n + 511) / 512);
   // layer 3
   gemm(s, true, false, true, m->y2, kNodeW, m->dout_b, kOut, G(m, N_W3), kOut, kNodeW, kOut, n,
        1.f);
-  hipLaunchKernelGGL((k_colsum<float>), nchunks, dim3(kOut), 0, s, m->dout, kOut, (size_t)n, kOut,
-                     G(m, N_B3));
-  gemm(s, false, true, false, m->dout_b, kOut, W(m, N_W3), kOut, m->dY, kNodeW, n, kNodeW, kOut,
-       1.f);
-  hipLaunchKernelGGL(k_dsilu, grid_for(nw), dim3(256), 0, s, m->dY, kNodeW, m->p2, m->dpb,
-                     (size_t)n, kNodeW);
-  // layer 2
-  gemm(s, true, false, true, m->y1, kNodeW, m->dpb, kNodeW, G(m, N_W2), kNodeW, kNodeW, kNodeW, n,
-       1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), nchunks, dim3(kNodeW), 0, s, m->dpb, kNodeW, (size_t)n,
-                     kNodeW, G(m, N_B2));
-  gemm(s, false, true, false, m->dpb, kNodeW, W(m, N_W2), kNodeW, m->dY, kNodeW, n, kNodeW,
-       kNodeW, 1.f);
-  hipLaunchKernelGGL(k_dsilu, grid_for(nw), dim3(256), 0, s, m->dY, kNodeW, m->p1, m->dpb,
-                     (size_t)n, kNodeW);
+  colsum(s, m->dout, kOut, n, kOut, nullptr, G(m, N_B3));
+  gemm_dsilu(s, m->dout_b, kOut, W(m, N_W3), kOut, m->p2, m->dpb, n, kNodeW, kOut);
+  // layer 2; each work-group's rows of dpb are its own input and output
+  gemm_weight_grad(s, m->y1, kNodeW, m->dpb, kNodeW, G(m, N_W2), G(m, N_B2), kNodeW, kNodeW, n);
+  gemm_dsilu(s, m->dpb, kNodeW, W(m, N_W2), kNodeW, m->p1, m->dpb, n, kNodeW, kNodeW);
   // layer 1, and d loss / d S (the first 32 inputs) into dY
-  gemm(s, true, false, true, m->u, kIn, m->dpb, kNodeW, G(m, N_W1), kNodeW, kIn, kNodeW, n, 1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), nchunks, dim3(kNodeW), 0, s, m->dpb, kNodeW, (size_t)n,
-                     kNodeW, G(m, N_B1));
+  gemm_weight_grad(s, m->u, kIn, m->dpb, kNodeW, G(m, N_W1), G(m, N_B1), kIn, kNodeW, n);
   gemm(s, false, true, false, m->dpb, kNodeW, W(m, N_W1), kNodeW, m->dY, kNodeW, n, kEdgeW,
        kNodeW, 1.f);
   // edge layer
-  hipLaunchKernelGGL(k_edge_dz, grid_for((size_t)e * kEdgeW), dim3(256), 0, s, m->dY, kNodeW,
-                     m->z, m->dst, m->dz, (size_t)e);
-  gemm(s, true, false, true, m->E1, kFeat, m->dz, kEdgeW, G(m, E_W1), kEdgeW, kFeat, kEdgeW, e,
-       1.f);
-  hipLaunchKernelGGL((k_colsum<uint16_t>), dim3((e + 511) / 512), dim3(kEdgeW), 0, s, m->dz,
-                     kEdgeW, (size_t)e, kEdgeW, G(m, E_B1));
+  if (e > 0) {
+    // about two work-groups per compute unit, 1,024 edges each at least
+    uint32_t per = ((uint32_t)e + 511u) / 512u;
+    per = std::max(1024u, (per + 255u) & ~255u);
+    hipLaunchKernelGGL(k_edge_grad, dim3(((uint32_t)e + per - 1u) / per), dim3(256), 0, s, m->E1,
+                       m->dY, kNodeW, m->mask, m->dst, (uint32_t)e, per, G(m, E_W1), G(m, E_B1));
+  }
 }
 
 void adam(clsph_nn* m, float lr, float beta1, float beta2, float eps) {
@@ -1211,12 +1464,6 @@ hipError_t scratch_address(int device, void** ptr) {
   }
   *ptr = addr[device];
   return hipSuccess;
-}
-
-void gemm_public(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
-                 const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
-                 const float* bias, const float* rowscale) {
-  gemm(s, ta, tb, add, A, lda, B, ldb, C, ldc, M, N, K, alpha, bias, rowscale);
 }
 
 void launch_compare(clsph_nn* m, clsph_state* a, clsph_state* b, float res[2]) {

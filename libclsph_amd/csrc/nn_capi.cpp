@@ -21,10 +21,10 @@ namespace {
 void free_nn(clsph_nn* m) {
   dfree(m->params), dfree(m->wb), dfree(m->grad), dfree(m->adam_m), dfree(m->adam_v);
   dfree(m->off), dfree(m->src), dfree(m->dst), dfree(m->scan_part);
-  dfree(m->E1), dfree(m->nu), dfree(m->degc), dfree(m->z), dfree(m->S), dfree(m->u);
+  dfree(m->E1), dfree(m->nu), dfree(m->degc), dfree(m->mask), dfree(m->S), dfree(m->u);
   dfree(m->p1), dfree(m->y1), dfree(m->p2), dfree(m->y2), dfree(m->out);
   dfree(m->target), dfree(m->loss), dfree(m->dout), dfree(m->dout_b), dfree(m->dY);
-  dfree(m->dpb), dfree(m->dz), dfree(m->sum), dfree(m->loc), dfree(m->inv), dfree(m->cmp);
+  dfree(m->dpb), dfree(m->sum), dfree(m->loc), dfree(m->inv), dfree(m->cmp);
 }
 
 int check_state(clsph_nn* m, clsph_state* st) {
@@ -171,11 +171,11 @@ int clsph_nn_create(clsph_ctx* ctx, uint32_t n_cap, uint32_t e_cap, clsph_nn** o
   AL(m->off, N + 1); AL(m->src, E); AL(m->dst, E);
   AL(m->scan_part, N / 1024 + 2);
   AL(m->E1, E * nn::kFeat); AL(m->nu, 2 * N); AL(m->degc, N);
-  AL(m->z, E * EW); AL(m->S, N * EW); AL(m->u, N * nn::kIn);
+  AL(m->mask, E); AL(m->S, N * EW); AL(m->u, N * nn::kIn);
   AL(m->p1, N * NW); AL(m->y1, N * NW); AL(m->p2, N * NW); AL(m->y2, N * NW);
   AL(m->out, N * nn::kOut);
   AL(m->target, 3 * N); AL(m->loss, 1); AL(m->dout, N * nn::kOut); AL(m->dout_b, N * nn::kOut);
-  AL(m->dY, N * NW); AL(m->dpb, N * NW); AL(m->dz, E * EW); AL(m->sum, 3 * N);
+  AL(m->dY, N * NW); AL(m->dpb, N * NW); AL(m->sum, 3 * N);
   AL(m->loc, N); AL(m->inv, N); AL(m->cmp, 2);
 #undef AL
   if (rc) {
@@ -561,7 +561,7 @@ int gemm_staged(clsph_ctx* ctx, const char* who, int trans_a, int trans_b, int a
     return fail(ctx, CLSPH_EDEVICE, std::string(who) + ": copy failed");
   int lda = trans_a ? (int)m : (int)k, ldb = trans_b ? (int)k : (int)n;
   // a non-accumulating product over a long K runs as one chunk
-  nn::gemm_public(s, trans_a, trans_b, accumulate, da, lda, db, ldb, dc, (int)n, (int)m, (int)n,
+  nn::gemm(s, trans_a, trans_b, accumulate, da, lda, db, ldb, dc, (int)n, (int)m, (int)n,
                   (int)k, 1.f, bias ? dbias : nullptr, nullptr);
   int rc = check_launch(ctx);
   if (rc) return rc;
