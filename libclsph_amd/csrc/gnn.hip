@@ -180,170 +180,324 @@ __global__ __launch_bounds__(256) void k_edge_inputs(
   o[1] = u32x4{packed[4], packed[5], packed[6], packed[7]};
 }
 
-// ---------------------------------------------------------------------------
-// Fused edge round for inference: one wave per particle i walks its
-// neighbour list (the density kernel's, at most kMaxEdges) in tiles of 16
-// edges and computes S_i = bf16(sum_j silu(silu(e_ij W1 + b1 [+ PA_i + PB_j])
-// W2 + b2) / C) without storing per-edge values.
-//
-// Both layers run transposed on 16x16x32 bf16 matrix cores: z^T = W^T e^T,
-// so the output's columns are edges and a lane holds, for edge l % 16, the
-// features 16 ob + 4 (l / 16) + r of output block ob (r = 0..3). Layer 2's
-// B operand (lane: 8 consecutive K slots of its edge) is taken straight from
-// those registers by permuting the K order: slot t of k-step ks and lane
-// group g = l / 16 is feature 32 ks + 16 (t / 4) + 4 g + t % 4, and the
-// weights are staged in LDS in that order. Tiles accumulate per lane; the
-// 16 edge lanes are summed once per particle.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-__device__ inline u32x4 pack8(const float v[8]) {
-  u32x4 r;
-  for (int t = 0; t < 4; ++t)
-    r[t] = (uint32_t)to_bf16(v[2 * t]) | ((uint32_t)to_bf16(v[2 * t + 1]) << 16);
-  return r;
+// Eight floats to bf16 (round to nearest even).
+__device__ __attribute__((always_inline)) inline u32x4 pack8(const float v[8]) {
+  const f32x8 x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+  return __builtin_bit_cast(u32x4, __builtin_convertvector(x, bf16x8));
+}
+
+// Orders a wave's own LDS accesses (its lanes exchange data, no other wave is
+// involved).
+__device__ __attribute__((always_inline)) inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---------------------------------------------------------------------------
+// Fused edge round for inference: S_i = bf16(sum_j silu(silu(e_ij W1 + b1
+// [+ PA_i + PB_j]) W2 + b2) / C) over particle i's neighbour list (the density
+// kernel's, at most kMaxEdges) without storing per-edge values.
+//
+// A wave takes up to 16 consecutive particles at a time (a run).
+// The run's edges, each particle's padded to quads, are cut into four equal
+// streams, one per lane group g = l / 16, whichever particles that splits; a
+// tile is the next quad of each stream. (A tile of 16 edges per particle would
+// be 3/4 full at 30 neighbours.) 64 edges at a time, one per lane, compute
+// their inputs and pass them to the tiles through LDS as 32 bf16 K slots:
+//   0-11 the inputs, 12-14 ones, 16-31 one-hot of the edge's particle.
+// W1's rows 12-14 are b1 split into three bf16 (8 + 8 + 8 bits, exact) and its
+// rows 16-31 the particles' PA, so layer 1's bias and node terms cost no
+// instruction; PB_j is the product's starting value.
+//
+// Layer 1 runs transposed on 16x16x32 bf16 matrix cores, output row 4 g + r of
+// block ob being feature 32 g + 4 ob + r, so lane group g of edge l % 16 holds
+// 32 consecutive features. They are layer 2's A operand as they stand (slot t
+// of k-step ks: feature 32 g + 8 ks + t), whose output has edges as rows and
+// feature 8 (l % 16) + ob as column: register r of lane group g is edge r of
+// its stream's quad, and a particle's sum stays in the lane's registers until
+// its last quad. The up to three particles that the streams' ends split are
+// joined through LDS at the end of the run.
+//
+// An infinite or NaN PA would spread over its run through the one-hot product,
+// so a run with one is taken particle by particle.
+//
+// Bound by vector instructions: per tile and lane 64 SiLUs, of whose
+// instructions 128 (exp2, rcp) take twice the issue time of the other 320;
+// the matrix cores are busy for 640 of about 2,350 cycles. 131,072 particles of
+// 28 neighbours: 358 us without node terms, 400 with (a tile per particle,
+// node inputs recomputed per edge and 16-lane sums: 687 and 713). Four waves
+// per SIMD instead of three, products issued a block ahead and runs handed out
+// by a queue measured the same; sums by 16x16x4 float products with a 0/1
+// matrix 452 (those run on the vector units).
+constexpr int kRunMax = 16;
+// 16-byte unit u of edge e's record in LDS, on distinct banks for 16 edges
+__device__ inline int rec_at(int e, int u) { return 4 * e + (u ^ ((e >> 2) & 3)); }
+
+// Node inputs nu and scaled degrees.
+__global__ __launch_bounds__(256) void k_node_inputs(const float* __restrict__ rho,
+                                                     const float* __restrict__ prs,
+                                                     const uint32_t* __restrict__ count,
+                                                     uint32_t n, float rho0, float K,
+                                                     float2* __restrict__ nu,
+                                                     float* __restrict__ degc) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  nu[i] = node_in(rho[i], prs[i], rho0, K);
+  degc[i] = (float)min(count[i], kMaxEdges) / kAggC;
+}
+
+// The high 16 bits of b, as a float: b less it is exact and 8 bits shorter.
+__device__ inline float bf16_head(float b) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, b) & 0xFFFF0000u);
 }
 
 template <bool ROUND2>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_edge_fused(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_edge_fused(
     const float4* __restrict__ pos, const float4* __restrict__ vel,
-    const float* __restrict__ rho, const float* __restrict__ prs,
-    const uint4* __restrict__ nbr, const uint32_t* __restrict__ count, uint32_t n, float h,
-    float rho0, float K, const uint16_t* __restrict__ W1, const float* __restrict__ b1,
-    const uint16_t* __restrict__ W2, const float* __restrict__ b2,
+    const float2* __restrict__ nu, const uint32_t* __restrict__ nbr,
+    const uint32_t* __restrict__ count, uint32_t n, float h, const uint16_t* __restrict__ W1,
+    const float* __restrict__ b1, const uint16_t* __restrict__ W2, const float* __restrict__ b2,
     const uint16_t* __restrict__ PA, const uint16_t* __restrict__ PB,
-    uint16_t* __restrict__ S, float* __restrict__ degc, float* __restrict__ nu) {
-  __shared__ u32x4 w1s[8 * 64];       // [ob][lane]: W1^T rows 16 ob + l % 16, k 8 g + t
-  __shared__ u32x4 w2s[8 * 4 * 64];   // [ob][ks][lane]: W2^T in the permuted K order
-  __shared__ float bs[2 * kWidth];
-  for (int idx = threadIdx.x; idx < 8 * 64; idx += 256) {
-    int ob = idx >> 6, l = idx & 63, g = l >> 4, row = 16 * ob + (l & 15);
-    uint32_t w[4];
-    for (int t = 0; t < 4; ++t) {
-      int k0 = 8 * g + 2 * t;
-      uint32_t lo = k0 < kFeat ? W1[k0 * kWidth + row] : 0u;
-      uint32_t hi = k0 + 1 < kFeat ? W1[(k0 + 1) * kWidth + row] : 0u;
-      w[t] = lo | (hi << 16);
+    uint16_t* __restrict__ S) {
+  __shared__ u32x4 w2s[8 * 4 * 64];  // [ob][ks][lane]
+  __shared__ u32x4 recs[4][64 * 4];
+  __shared__ uint32_t js[4][64];
+  __shared__ uint32_t quads[4][16];  // slot, edges << 8, last of its particle << 16
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  {
+    // k-step `wave` of W2: eight rows of eight columns per lane, turned
+    u32x4 row[8];
+    for (int t = 0; t < 8; ++t)
+      row[t] = *(const u32x4*)(W2 + (size_t)(32 * g + 8 * wave + t) * kWidth + 8 * c);
+    for (int ob = 0; ob < 8; ++ob) {
+      u32x4 v;
+      for (int t = 0; t < 4; ++t)
+        v[t] = __builtin_amdgcn_perm(row[2 * t + 1][ob >> 1], row[2 * t][ob >> 1],
+                                     ob & 1 ? 0x07060302u : 0x05040100u);
+      w2s[(ob * 4 + wave) * 64 + lane] = v;
     }
-    w1s[idx] = u32x4{w[0], w[1], w[2], w[3]};
   }
-  for (int idx = threadIdx.x; idx < 8 * 4 * 64; idx += 256) {
-    int ob = idx >> 8, ks = (idx >> 6) & 3, l = idx & 63, g = l >> 4, row = 16 * ob + (l & 15);
-    uint32_t w[4];
-    for (int t = 0; t < 4; ++t) {
-      int ta = 2 * t, tb = 2 * t + 1;
-      int ka = 32 * ks + 16 * (ta >> 2) + 4 * g + (ta & 3);
-      int kb = 32 * ks + 16 * (tb >> 2) + 4 * g + (tb & 3);
-      w[t] = (uint32_t)W2[ka * kWidth + row] | ((uint32_t)W2[kb * kWidth + row] << 16);
+  // layer 1's weights: lane (c, g) holds feature 32 (c / 4) + 4 ob + c % 4 of K slots 8 g + t
+  u32x4 w1[8];
+  for (int ob = 0; ob < 8; ++ob) {
+    const int col = 32 * (c >> 2) + 4 * ob + (c & 3);
+    const float b = b1[col];
+    const bool finite = __builtin_fabsf(b) < __builtin_inff();
+    const float head = finite ? bf16_head(b) : b, rest = finite ? b - head : 0.f;
+    uint16_t v[8];
+    for (int t = 0; t < 8; ++t) {
+      const uint16_t row = W1[min(8 * g + t, kFeat - 1) * kWidth + col];
+      v[t] = 8 * g + t < 12 ? row : (uint16_t)0;
     }
-    w2s[idx] = u32x4{w[0], w[1], w[2], w[3]};
+    if (g == 1) {
+      v[4] = to_bf16(head);
+      v[5] = to_bf16(bf16_head(rest));
+      v[6] = to_bf16(rest - bf16_head(rest));
+    }
+    for (int t = 0; t < 4; ++t) w1[ob][t] = (uint32_t)v[2 * t] | ((uint32_t)v[2 * t + 1] << 16);
   }
-  for (int idx = threadIdx.x; idx < kWidth; idx += 256) {
-    bs[idx] = b1[idx];
-    bs[kWidth + idx] = b2[idx];
-  }
+  float bias2[8];
+  for (int ob = 0; ob < 8; ++ob) bias2[ob] = b2[8 * c + ob];
   __syncthreads();
 
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const uint32_t waves = gridDim.x * 4;
+  // this wave's particles; consecutive shares on the same XCD's L2
+  const uint32_t blocks = gridDim.x;
+  const uint32_t b = blocks % 8 ? blockIdx.x : (blockIdx.x % 8) * (blocks / 8) + blockIdx.x / 8;
+  const uint32_t w = b * 4 + wave;
+  const uint32_t last = (uint32_t)((uint64_t)n * (w + 1) / (blocks * 4));
   const float inv_h = 1.f / h;
-  for (uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += waves) {
-    const uint32_t deg = min(count[i], kMaxEdges);
-    const float4 xi = pos[i], vi = vel[i];
-    const float2 ni = node_in(rho[i], prs[i], rho0, K);
-    float pa[8][4];
-    for (int ob = 0; ob < 8; ++ob)
-      for (int r = 0; r < 4; ++r) pa[ob][r] = bs[16 * ob + 4 * g + r];
+  u32x4* rec = recs[wave];
+  uint32_t limit = kRunMax, redo_end = 0;
+  for (uint32_t i0 = (uint32_t)((uint64_t)n * w / (blocks * 4)); i0 < last;) {
+    const uint32_t parts = min(last - i0, limit);
     if (ROUND2) {
-      for (int ob = 0; ob < 8; ++ob) {
-        uint2 v = *(const uint2*)(PA + (size_t)i * kWidth + 16 * ob + 4 * g);
-        pa[ob][0] += from_bf16((uint16_t)(v.x & 0xFFFFu));
-        pa[ob][1] += from_bf16((uint16_t)(v.x >> 16));
-        pa[ob][2] += from_bf16((uint16_t)(v.y & 0xFFFFu));
-        pa[ob][3] += from_bf16((uint16_t)(v.y >> 16));
-      }
-    }
-    f32x4 acc[8];
-    for (int ob = 0; ob < 8; ++ob) acc[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t q0 = 0; q0 < deg; q0 += 16) {
-      const uint32_t q = q0 + c;
-      const bool valid = q < deg;
-      uint32_t j = i;
-      if (valid) {
-        uint4 js = nbr[(size_t)(q >> 2) * n + i];
-        uint32_t sel = q & 3u;
-        j = sel == 0 ? js.x : sel == 1 ? js.y : sel == 2 ? js.z : js.w;
-      }
-      // B operand of layer 1: features 8 g .. 8 g + 7 of this lane's edge
-      float f[kFeat];
-      edge_features(xi, pos[j], vi, vel[j], ni, node_in(rho[j], prs[j], rho0, K), inv_h, f);
-      float sel8[8];
-      for (int t = 0; t < 8; ++t) sel8[t] = g == 0 ? f[t] : (g == 1 ? f[8 + t] : 0.f);
-      const bf16x8 eb = __builtin_bit_cast(bf16x8, pack8(sel8));
-      // layer 1 (+ bias, node terms), SiLU, packed into layer 2's B operands
-      float pb[8][4];
-      if (ROUND2) {
+      bool odd = false;  // PA not finite
+      if (g >= 2)
         for (int ob = 0; ob < 8; ++ob) {
-          uint2 v = *(const uint2*)(PB + (size_t)j * kWidth + 16 * ob + 4 * g);
-          pb[ob][0] = from_bf16((uint16_t)(v.x & 0xFFFFu));
-          pb[ob][1] = from_bf16((uint16_t)(v.x >> 16));
-          pb[ob][2] = from_bf16((uint16_t)(v.y & 0xFFFFu));
-          pb[ob][3] = from_bf16((uint16_t)(v.y >> 16));
+          const int col = 32 * (c >> 2) + 4 * ob + (c & 3);
+          uint16_t v[8];
+          for (int t = 0; t < 8; ++t) {
+            const uint32_t p = 8 * (g - 2) + t;
+            const uint16_t pa = PA[(size_t)(i0 + min(p, parts - 1)) * kWidth + col];
+            v[t] = p < parts ? pa : (uint16_t)0;
+            odd |= (v[t] & 0x7F80u) == 0x7F80u;
+          }
+          for (int t = 0; t < 4; ++t)
+            w1[ob][t] = (uint32_t)v[2 * t] | ((uint32_t)v[2 * t + 1] << 16);
         }
-      }
-      float s1[8][4];
-      for (int ob = 0; ob < 8; ++ob) {
-        f32x4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, w1s[ob * 64 + lane]), eb, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
-            0, 0);
-        for (int r = 0; r < 4; ++r) {
-          float v = z[r] + pa[ob][r];
-          if (ROUND2) v += pb[ob][r];
-          s1[ob][r] = silu(v);
-        }
-      }
-      bf16x8 bop[4];
-      for (int ks = 0; ks < 4; ++ks) {
-        float v8[8];
-        for (int t = 0; t < 8; ++t) v8[t] = s1[2 * ks + (t >> 2)][t & 3];
-        bop[ks] = __builtin_bit_cast(bf16x8, pack8(v8));
-      }
-      // layer 2, SiLU, masked accumulation over the tile's edges
-      for (int ob = 0; ob < 8; ++ob) {
-        f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int ks = 0; ks < 4; ++ks)
-          y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, w2s[(ob * 4 + ks) * 64 + lane]), bop[ks], y, 0, 0, 0);
-        for (int r = 0; r < 4; ++r) {
-          float v = silu(y[r] + bs[kWidth + 16 * ob + 4 * g + r]);
-          acc[ob][r] += valid ? v : 0.f;
-        }
-        __builtin_amdgcn_sched_barrier(0);  // one output block's reads at a time
+      if (parts > 1 && __any(odd)) {
+        limit = 1, redo_end = i0 + parts;
+        continue;
       }
     }
-    // sum over the 16 edge lanes of each group
-    for (int ob = 0; ob < 8; ++ob)
-      for (int r = 0; r < 4; ++r) {
-        float v = acc[ob][r];
-        v += __shfl_xor(v, 1, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 8, 64);
-        acc[ob][r] = v;
-      }
-    // lane c < 8 of group g writes features 16 c + 4 g .. + 3
-    for (int ob = 0; ob < 8; ++ob)
-      if (c == ob) {
-        uint32_t lo = (uint32_t)to_bf16(acc[ob][0] * (1.f / kAggC)) |
-                      ((uint32_t)to_bf16(acc[ob][1] * (1.f / kAggC)) << 16);
-        uint32_t hi = (uint32_t)to_bf16(acc[ob][2] * (1.f / kAggC)) |
-                      ((uint32_t)to_bf16(acc[ob][3] * (1.f / kAggC)) << 16);
-        *(uint2*)(S + (size_t)i * kWidth + 16 * ob + 4 * g) = make_uint2(lo, hi);
-      }
-    if (lane == 0) {
-      degc[i] = (float)deg / kAggC;
-      nu[2 * i] = ni.x;
-      nu[2 * i + 1] = ni.y;
+    // lane p: degree and first quad of particle i0 + p
+    const uint32_t deg = (uint32_t)lane < parts ? min(count[i0 + lane], kMaxEdges) : 0u;
+    uint32_t start = (deg + 3) / 4;
+    for (int o = 1; o < kRunMax; o <<= 1) {
+      const uint32_t y = __shfl_up(start, o, 64);
+      if (lane >= o) start += y;
     }
+    const uint32_t total = __builtin_amdgcn_readlane(start, kRunMax - 1);
+    start -= (deg + 3) / 4;
+    uint32_t from[kRunMax];
+    for (int p = 1; p < kRunMax; ++p) from[p] = __builtin_amdgcn_readlane(start, p);
+    // the particle that owns a quad: the last to start at or before it (one
+    // without edges starts where the next does)
+    auto owner = [&](uint32_t quad) {
+      uint32_t slot = 0;
+      for (int p = 1; p < kRunMax; ++p) slot += quad >= from[p] ? 1u : 0u;
+      return quad < total ? slot : 0u;
+    };
+    for (uint64_t none = __ballot((uint32_t)lane < parts && deg == 0); none; none &= none - 1)
+      if (lane < 16)
+        *(u32x4*)(S + (size_t)(i0 + __builtin_ctzll(none)) * kWidth + 8 * c) =
+            u32x4{0u, 0u, 0u, 0u};
+    const uint32_t tiles = (total + 3) / 4;  // quads per stream
+    float acc[8], lead[8];
+    for (int ob = 0; ob < 8; ++ob) acc[ob] = lead[ob] = 0.f;
+    // this stream's first quad continues a particle of the stream before
+    const uint32_t slot0 = owner(g * tiles);
+    bool pending = g * tiles < total && g * tiles != (uint32_t)__shfl(start, slot0, 64);
+    bool led = false, open = false;
+    uint32_t slot = 0;
+    auto store = [&](const float* sum) {
+      float v[8];
+      for (int ob = 0; ob < 8; ++ob) v[ob] = sum[ob] * (1.f / kAggC);
+      *(u32x4*)(S + (size_t)(i0 + slot) * kWidth + 8 * c) = pack8(v);
+    };
+    for (uint32_t t0 = 0; t0 < tiles; t0 += 4) {
+      // the inputs of four tiles' edges
+      wave_fence();
+      {
+        const uint32_t t = t0 + g, quad = ((lane >> 2) & 3) * tiles + t, r = lane & 3;
+        const uint32_t p = owner(quad);
+        const uint32_t k = quad - (uint32_t)__shfl(start, p, 64);
+        const uint32_t d = (uint32_t)__shfl(deg, p, 64);
+        const bool on = t < tiles && quad < total;
+        const bool valid = on && 4 * k + r < d;
+        const uint32_t i = i0 + p;
+        uint32_t j = i0;
+        u32x4 lo = {0u, 0u, 0u, 0u}, hi = {0u, 0u, 0u, 0u};
+        if (valid) {
+          j = nbr[((size_t)k * n + i) * 4 + r];
+          float f[kFeat];
+          edge_features(pos[i], pos[j], vel[i], vel[j], nu[i], nu[j], inv_h, f);
+          f[12] = f[13] = f[14] = 1.f;
+          lo = pack8(f), hi = pack8(f + 8);
+        }
+        rec[rec_at(lane, 0)] = lo;
+        rec[rec_at(lane, 1)] = hi;
+        if (ROUND2) {
+          const uint32_t one = valid ? 0x3F80u << (16 * (p & 1)) : 0u, h = p >> 1;
+          rec[rec_at(lane, 2)] =
+              u32x4{h == 0 ? one : 0u, h == 1 ? one : 0u, h == 2 ? one : 0u, h == 3 ? one : 0u};
+          rec[rec_at(lane, 3)] =
+              u32x4{h == 4 ? one : 0u, h == 5 ? one : 0u, h == 6 ? one : 0u, h == 7 ? one : 0u};
+          js[wave][lane] = j;
+        }
+        if (r == 0)
+          quads[wave][lane >> 2] =
+              on ? p | (min(d - 4 * k, 4u) << 8) | (4 * k + 4 >= d ? 0x10000u : 0u) : 0u;
+      }
+      wave_fence();
+      // PB of the tile's edges, loaded a layer ahead
+      const uint32_t here = min(tiles - t0, 4u);
+      u32x4 pb[4];
+      auto load_pb = [&](uint32_t t) {
+        const u32x4* p = (const u32x4*)(PB + (size_t)js[wave][16 * t + c] * kWidth + 32 * g);
+        for (int q = 0; q < 4; ++q) pb[q] = p[q];
+      };
+      if (ROUND2) load_pb(0);
+#pragma unroll 1
+      for (uint32_t t = 0; t < here; ++t) {
+        u32x4 er = {0u, 0u, 0u, 0u};
+        if (ROUND2 || g < 2) er = rec[rec_at(16 * t + c, g)];
+        const bf16x8 eb = __builtin_bit_cast(bf16x8, er);
+        const uint32_t info = quads[wave][4 * t + g], edges = (info >> 8) & 0xFFu;
+        auto layer1 = [&](int ob) {
+          f32x4 z = {0.f, 0.f, 0.f, 0.f};
+          if (ROUND2) {
+            const uint32_t x = pb[ob >> 1][2 * (ob & 1)], y = pb[ob >> 1][2 * (ob & 1) + 1];
+            z = f32x4{__builtin_bit_cast(float, x << 16),
+                      __builtin_bit_cast(float, x & 0xFFFF0000u),
+                      __builtin_bit_cast(float, y << 16),
+                      __builtin_bit_cast(float, y & 0xFFFF0000u)};
+          }
+          return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w1[ob]), eb, z,
+                                                         0, 0, 0);
+        };
+        bf16x8 a2[4];
+        auto layer2 = [&](int ob) {
+          f32x4 y = {bias2[ob], bias2[ob], bias2[ob], bias2[ob]};
+          for (int ks = 0; ks < 4; ++ks)
+            y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a2[ks], __builtin_bit_cast(bf16x8, w2s[(ob * 4 + ks) * 64 + lane]), y, 0, 0, 0);
+          return y;
+        };
+        for (int ks = 0; ks < 4; ++ks) {
+          const f32x4 z0 = layer1(2 * ks), z1 = layer1(2 * ks + 1);
+          float v8[8];
+          for (int r = 0; r < 4; ++r) v8[r] = silu(z0[r]), v8[4 + r] = silu(z1[r]);
+          a2[ks] = __builtin_bit_cast(bf16x8, pack8(v8));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (ROUND2) load_pb(min(t + 1, here - 1));
+        // SiLU's 1 + exp2(..), or infinity (a factor of zero) past the quad's edges
+        float one[4];
+        for (uint32_t r = 0; r < 4; ++r) one[r] = r < edges ? 1.f : __builtin_inff();
+        for (int ob = 0; ob < 8; ++ob) {
+          const f32x4 y = layer2(ob);
+          for (int r = 0; r < 4; ++r)
+            acc[ob] = __builtin_fmaf(
+                y[r], __builtin_amdgcn_rcpf(one[r] + __builtin_amdgcn_exp2f(y[r] * -1.44269504f)),
+                acc[ob]);
+          __builtin_amdgcn_sched_barrier(0);  // one output block's reads at a time
+        }
+        if (edges) slot = info & 0xFFu, open = !(info >> 16);
+        if (__any(info >> 16)) {
+          if (info >> 16) {
+            if (pending) {
+              for (int ob = 0; ob < 8; ++ob) lead[ob] = acc[ob];
+              led = true, pending = false;
+            } else {
+              store(acc);
+            }
+            for (int ob = 0; ob < 8; ++ob) acc[ob] = 0.f;
+          }
+        }
+      }
+    }
+    if (__any(open)) {
+      // a particle that goes on in later streams: their leading sums, and
+      // whole streams of it
+      wave_fence();
+      float4* rows = (float4*)rec;  // [g][acc, lead][128]
+      for (int q = 0; q < 2; ++q) {
+        rows[(2 * g) * 32 + 2 * c + q] =
+            make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+        rows[(2 * g + 1) * 32 + 2 * c + q] =
+            make_float4(lead[4 * q], lead[4 * q + 1], lead[4 * q + 2], lead[4 * q + 3]);
+      }
+      wave_fence();
+      for (int h = 1; h < 4; ++h) {
+        const bool whole = __shfl((int)(open && pending), 16 * h, 64);
+        const bool part = __shfl((int)led, 16 * h, 64);
+        const uint32_t of = __shfl(slot0, 16 * h, 64);
+        if (h > g && open && of == slot && (whole || part))
+          for (int q = 0; q < 2; ++q) {
+            const float4 v = rows[(2 * h + (whole ? 0 : 1)) * 32 + 2 * c + q];
+            acc[4 * q] += v.x, acc[4 * q + 1] += v.y;
+            acc[4 * q + 2] += v.z, acc[4 * q + 3] += v.w;
+          }
+      }
+      if (open && !pending) store(acc);
+    }
+    i0 += parts;
+    if (i0 >= redo_end) limit = kRunMax;
   }
 }
 
@@ -950,10 +1104,12 @@ void forward_fused(clsph_gnn* m, clsph_state* st, float4* acc, float gx, float g
   if (blocks * 4 > n) blocks = (n + 3) / 4;
   if (blocks == 0) blocks = 1;
   if (ev) (void)hipEventRecord(ev[0], s);
+  hipLaunchKernelGGL(k_node_inputs, grid_for(n), dim3(256), 0, s, st->rho_s, st->prs_s,
+                     st->nbr_count, n, d.p.fluid_density, d.p.K, (float2*)m->nu, m->degc);
   hipLaunchKernelGGL((k_edge_fused<false>), dim3(blocks), dim3(256), 0, s, st->pos_s, st->vel_s,
-                     st->rho_s, st->prs_s, st->nbr, st->nbr_count, n, d.p.h, d.p.fluid_density,
-                     d.p.K, W(m, E1_W1), P(m, E1_B1), W(m, E1_W2), P(m, E1_B2),
-                     (const uint16_t*)nullptr, (const uint16_t*)nullptr, m->S[0], m->degc, m->nu);
+                     (const float2*)m->nu, (const uint32_t*)st->nbr, st->nbr_count, n, d.p.h, W(m, E1_W1),
+                     P(m, E1_B1), W(m, E1_W2), P(m, E1_B2), (const uint16_t*)nullptr,
+                     (const uint16_t*)nullptr, m->S[0]);
   if (ev) (void)hipEventRecord(ev[1], s);
   // node part of round 1 (fused)
   constexpr size_t kLdsNode1 = (size_t)(8 * 4 + 8 * 5 + 8 * 4 + 8 * 4) * 64 * 16 + 4 * kWidth * 4;
@@ -980,9 +1136,8 @@ void forward_fused(clsph_gnn* m, clsph_state* st, float4* acc, float gx, float g
                      m->PB);
   if (ev) (void)hipEventRecord(ev[2], s);
   hipLaunchKernelGGL((k_edge_fused<true>), dim3(blocks), dim3(256), 0, s, st->pos_s, st->vel_s,
-                     st->rho_s, st->prs_s, st->nbr, st->nbr_count, n, d.p.h, d.p.fluid_density,
-                     d.p.K, W(m, E2_W1), P(m, E2_B1), W(m, E2_W2), P(m, E2_B2), m->PA, m->PB,
-                     m->S[1], m->degc, m->nu);
+                     (const float2*)m->nu, (const uint32_t*)st->nbr, st->nbr_count, n, d.p.h, W(m, E2_W1),
+                     P(m, E2_B1), W(m, E2_W2), P(m, E2_B2), m->PA, m->PB, m->S[1]);
   if (ev) (void)hipEventRecord(ev[3], s);
   hipLaunchKernelGGL(k_node2, dim3(nblocks), dim3(512), kLdsNode2, s, m->S[1], m->Hb, m->degc, n,
                      m->wb, m->params, m->out, acc, gx, gy, gz);
