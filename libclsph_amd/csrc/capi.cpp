@@ -28,6 +28,17 @@ int read_dps(clsph_state* st, std::vector<DevParams>& out, BatchParams* bp = nul
   return CLSPH_OK;
 }
 
+void free_ctx(clsph_ctx* ctx) {
+  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  for (int k = 0; k < 2; ++k) {
+    if (ctx->transfer_done[k]) (void)hipEventDestroy(ctx->transfer_done[k]);
+    if (ctx->transfer[k]) (void)hipHostFree(ctx->transfer[k]);
+  }
+  if (ctx->transfer_status) (void)hipHostFree(ctx->transfer_status);
+  if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+  delete ctx;
+}
+
 void free_state_buffers(clsph_state* st) {
   dfree(st->pos), dfree(st->vel), dfree(st->vh);
   dfree(st->pos_s), dfree(st->vel_s), dfree(st->vh_s), dfree(st->acc_s);
@@ -405,37 +416,22 @@ int upload(clsph_state* st, uint32_t scene, const clsph_particle* p, uint32_t n)
   if (n > st->scene_cap[scene]) return fail(st->ctx, CLSPH_EINVAL, "more particles than the scene holds");
   if (st->fixed_counts && n != st->scene_n[scene])
     return fail(st->ctx, CLSPH_EINVAL, "a batch scene takes exactly its allocated count");
-  std::vector<float4> pos(n), vel(n), vh(n), acc(n);
-  std::vector<float> rho(n), prs(n);
-  std::vector<uint32_t> key(n);
-  for (uint32_t i = 0; i < n; ++i) {
-    const float* a = p[i].position.s;
-    const float* b = p[i].velocity.s;
-    const float* c = p[i].intermediate_velocity.s;
-    const float* d = p[i].acceleration.s;
-    pos[i] = make_float4(a[0], a[1], a[2], 0.f);
-    vel[i] = make_float4(b[0], b[1], b[2], 0.f);
-    vh[i] = make_float4(c[0], c[1], c[2], 0.f);
-    acc[i] = make_float4(d[0], d[1], d[2], 0.f);
-    rho[i] = p[i].density;
-    prs[i] = p[i].pressure;
-    key[i] = p[i].grid_index;
+  const uint32_t b0 = st->scene_begin[scene];
+  clsph_ctx* c = st->ctx;
+  hipStream_t s = c->stream;
+  std::lock_guard<std::mutex> hold(c->transfer_lock);
+  for (uint32_t r = 0, k = 0; r < n; r += kTransferRecords, k ^= 1u) {
+    const uint32_t count = std::min(n - r, kTransferRecords);
+    // the buffer is free once the kernel that read it before has ended
+    if (r >= 2u * kTransferRecords) HIPCK(c, hipEventSynchronize(c->transfer_done[k]));
+    memcpy(c->transfer[k], p + r, sizeof(clsph_particle) * (size_t)count);
+    launch_unpack_records(st, b0 + r, count, c->transfer[k]);
+    HIPCK(c, hipEventRecord(c->transfer_done[k], s));
   }
-  uint32_t b0 = st->scene_begin[scene];
-  hipStream_t s = st->ctx->stream;
-  auto put = [&](void* dst, const void* src, size_t bytes) -> int {
-    if (bytes) HIPCK(st->ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-    return CLSPH_OK;
-  };
-  int rc = put(st->pos + b0, pos.data(), sizeof(float4) * n);
-  if (!rc) rc = put(st->vel + b0, vel.data(), sizeof(float4) * n);
-  if (!rc) rc = put(st->vh + b0, vh.data(), sizeof(float4) * n);
-  if (!rc) rc = put(st->acc_s + b0, acc.data(), sizeof(float4) * n);
-  if (!rc) rc = put(st->rho_s + b0, rho.data(), sizeof(float) * n);
-  if (!rc) rc = put(st->prs_s + b0, prs.data(), sizeof(float) * n);
-  if (!rc) rc = put(st->key_b + b0, key.data(), sizeof(uint32_t) * n);
+  int rc = check_launch(c);
   if (rc) return rc;
   if (n != st->scene_n[scene]) {
+    HIPCK(c, hipStreamSynchronize(s));
     st->scene_n[scene] = n;
     st->n = n;  // single-scene states only (batches keep their counts)
     rc = build_blocks(st);
@@ -463,55 +459,30 @@ int download(clsph_state* st, uint32_t scene, clsph_particle* out, uint32_t n, b
   if (n == 0) return device_errors(st);
   if (n != sn && !st->fields_canonical)
     return fail(st->ctx, CLSPH_EINVAL, "partial downloads need the whole particle count");
-  uint32_t b0 = st->scene_begin[scene];
-  uint32_t cnt = n;
-  std::vector<float4> pos(cnt), vel(cnt), vh(cnt), acc(cnt);
-  std::vector<float> rho(cnt), prs(cnt);
-  std::vector<uint32_t> key(cnt), slot(cnt);
-  hipStream_t s = st->ctx->stream;
-  const float4* P = (sorted ? st->pos_s : st->pos) + b0;
-  const float4* V = (sorted ? st->vel_s : st->vel) + b0;
-  const float4* H = (sorted ? st->vh_s : st->vh) + b0;
-  auto get = [&](void* dst, const void* src, size_t bytes) -> int {
-    HIPCK(st->ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+  clsph_ctx* c = st->ctx;
+  std::lock_guard<std::mutex> hold(c->transfer_lock);
+  TransferStatus* status = c->transfer_status;
+  *status = {};
+  if (!st->fields_canonical) launch_invert_slots(st, scene);
+  auto begin = [&](uint32_t r, uint32_t k) -> int {
+    launch_pack_records(st, scene, n, r, std::min(n - r, kTransferRecords), sorted, c->transfer[k],
+                        status);
+    HIPCK(c, hipEventRecord(c->transfer_done[k], c->stream));
     return CLSPH_OK;
   };
-  int rc = get(pos.data(), P, sizeof(float4) * cnt);
-  if (!rc) rc = get(vel.data(), V, sizeof(float4) * cnt);
-  if (!rc) rc = get(vh.data(), H, sizeof(float4) * cnt);
-  bool want_acc = sorted || !st->acc_zero;
-  if (!rc && want_acc) rc = get(acc.data(), st->acc_s + b0, sizeof(float4) * cnt);
-  if (!rc) rc = get(rho.data(), st->rho_s + b0, sizeof(float) * cnt);
-  if (!rc) rc = get(prs.data(), st->prs_s + b0, sizeof(float) * cnt);
-  if (!rc) rc = get(key.data(), st->key_b + b0, sizeof(uint32_t) * cnt);
-  bool reorder = !st->fields_canonical;
-  if (!rc && reorder) rc = get(slot.data(), st->slot + b0, sizeof(uint32_t) * cnt);
-  if (rc) return rc;
-  std::vector<DevParams> d;
-  rc = read_dps(st, d);  // also waits for the copies above
-  if (rc) return rc;
-  uint32_t kbase = reorder ? d[scene].key_base : 0;
-  for (uint32_t k = 0; k < cnt; ++k) {
-    uint32_t o = reorder ? slot[k] - b0 : k;
-    if (o >= n) return fail(st->ctx, CLSPH_EDEVICE, "canonical slots are not a permutation");
-    clsph_particle& q = out[o];
-    memset(&q, 0, sizeof(q));
-    q.density = rho[k];
-    q.pressure = prs[k];
-    q.grid_index = reorder ? (key[k] - kbase) >> 3 : key[k];
-    if (want_acc && (sorted || !reorder)) {
-      q.acceleration.s[0] = acc[k].x, q.acceleration.s[1] = acc[k].y, q.acceleration.s[2] = acc[k].z;
-    }
+  int rc = begin(0, 0);
+  if (!rc && n > kTransferRecords) rc = begin(kTransferRecords, 1);
+  if (!rc) rc = check_launch(c);
+  for (uint32_t r = 0, k = 0; !rc && r < n; r += kTransferRecords, k ^= 1u) {
+    HIPCK(c, hipEventSynchronize(c->transfer_done[k]));
+    memcpy(out + r, c->transfer[k],
+           sizeof(clsph_particle) * (size_t)std::min(n - r, kTransferRecords));
+    if (n - r > 2u * kTransferRecords) rc = begin(r + 2u * kTransferRecords, k);
   }
-  for (uint32_t k = 0; k < cnt; ++k) {
-    uint32_t o = (sorted && reorder) ? slot[k] - b0 : k;
-    clsph_particle& q = out[o];
-    q.position.s[0] = pos[k].x, q.position.s[1] = pos[k].y, q.position.s[2] = pos[k].z;
-    q.velocity.s[0] = vel[k].x, q.velocity.s[1] = vel[k].y, q.velocity.s[2] = vel[k].z;
-    q.intermediate_velocity.s[0] = vh[k].x, q.intermediate_velocity.s[1] = vh[k].y,
-    q.intermediate_velocity.s[2] = vh[k].z;
-  }
-  return device_errors(st);
+  if (rc) return rc;
+  if (status->bad_slots)
+    return fail(c, CLSPH_EDEVICE, "canonical slots are not a permutation");
+  return error_code(st, status->err);
 }
 
 int scene_upload(clsph_state* st, uint32_t scene, const float* face_normals,
@@ -574,13 +545,7 @@ int ensure_graph(clsph_state* st) {
 namespace clsph {
 namespace host {
 
-int device_errors(clsph_state* st) {
-  std::vector<DevParams> d;
-  BatchParams b;
-  int rc = read_dps(st, d, &b);
-  if (rc) return rc;
-  uint32_t err = b.err;
-  for (const DevParams& x : d) err |= x.err;
+int error_code(clsph_state* st, uint32_t err) {
   if (err & kErrGridDim)
     return fail(st->ctx, CLSPH_EGRID,
                 "grid dimension >= 1024 cells on an axis (particles spread too far)");
@@ -589,6 +554,16 @@ int device_errors(clsph_state* st) {
   if (err & kErrFineKey)
     return fail(st->ctx, CLSPH_ETABLE, "grid_cell_count reached 2^29 cells");
   return CLSPH_OK;
+}
+
+int device_errors(clsph_state* st) {
+  std::vector<DevParams> d;
+  BatchParams b;
+  int rc = read_dps(st, d, &b);
+  if (rc) return rc;
+  uint32_t err = b.err;
+  for (const DevParams& x : d) err |= x.err;
+  return error_code(st, err);
 }
 
 int resize_single(clsph_state* st, uint32_t n) {
@@ -625,10 +600,22 @@ int clsph_init(int device, clsph_ctx** out) {
   }
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cus = prop.multiProcessorCount;
+  hipError_t te = hipHostMalloc((void**)&ctx->transfer_status, sizeof(TransferStatus),
+                                hipHostMallocDefault);
+  for (int k = 0; k < 2 && te == hipSuccess; ++k) {
+    te = hipHostMalloc((void**)&ctx->transfer[k], sizeof(clsph_particle) * kTransferRecords,
+                       hipHostMallocDefault);
+    if (te == hipSuccess)
+      te = hipEventCreateWithFlags(&ctx->transfer_done[k], hipEventDisableTiming);
+  }
+  if (te != hipSuccess) {
+    free_ctx(ctx);
+    return fail(nullptr, CLSPH_EDEVICE,
+                std::string("transfer buffers: ") + hipGetErrorString(te));
+  }
   hipError_t se = clsph::nn::scratch_address(device, &ctx->scratch);
   if (se != hipSuccess) {
-    (void)hipStreamDestroy(ctx->stream);
-    delete ctx;
+    free_ctx(ctx);
     return fail(nullptr, CLSPH_EDEVICE,
                 std::string("device workspace address: ") + hipGetErrorString(se));
   }
@@ -639,8 +626,7 @@ int clsph_init(int device, clsph_ctx** out) {
 int clsph_free(clsph_ctx* ctx) {
   if (!ctx) return CLSPH_OK;
   (void)hipSetDevice(ctx->device);
-  if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-  delete ctx;
+  free_ctx(ctx);
   return CLSPH_OK;
 }
 

@@ -57,6 +57,8 @@ inline int check_launch(clsph_ctx* ctx) {
   return CLSPH_OK;
 }
 
+// The return code of device error bits (defined in capi.cpp).
+int error_code(clsph_state* st, uint32_t err);
 // Reads the device error bits of every scene and turns them into a return
 // code (defined in capi.cpp).
 int device_errors(clsph_state* st);

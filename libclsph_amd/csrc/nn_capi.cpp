@@ -424,10 +424,9 @@ int clsph_track_ids(clsph_state* st, int enable) {
     }
     st->graph_dirty = st->lgraph_dirty = true;
   }
-  std::vector<uint32_t> iota(st->n_cap);
-  for (uint32_t k = 0; k < st->n_cap; ++k) iota[k] = k;
-  HIPCK(c, hipMemcpyAsync(st->ids, iota.data(), sizeof(uint32_t) * st->n_cap,
-                          hipMemcpyHostToDevice, c->stream));
+  launch_reset_ids(st);
+  int rc = check_launch(c);
+  if (rc) return rc;
   HIPCK(c, hipStreamSynchronize(c->stream));
   return CLSPH_OK;
 }

@@ -8,10 +8,21 @@
 // each inside one scene.
 #pragma once
 
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "common.h"
+
+namespace clsph {
+// Records per page-locked transfer buffer (1 MB: a buffer's copy by the host
+// overlaps the next one's transfer, and stays in its cache).
+constexpr uint32_t kTransferRecords = 13056;
+struct TransferStatus {
+  uint32_t err;        // kErr* bits of every scene and of the batch
+  uint32_t bad_slots;  // the canonical slots are not a permutation
+};
+}  // namespace clsph
 
 struct clsph_ctx {
   int device = 0;
@@ -21,6 +32,13 @@ struct clsph_ctx {
   // Device address of the static workspace of clsph_nn_gemm_noalloc on this
   // context's device (shared by every context on the device).
   void* scratch = nullptr;
+  // Two page-locked buffers of particle records for synchronous transfers of
+  // any of the context's states, an event each (its last kernel ended) and
+  // their status; held by one transfer at a time.
+  std::mutex transfer_lock;
+  clsph_particle* transfer[2] = {};
+  hipEvent_t transfer_done[2] = {};
+  clsph::TransferStatus* transfer_status = nullptr;
 };
 
 // Stage indices (clsph_time_stage order).
@@ -168,9 +186,18 @@ void launch_aabb(clsph_state* s);
 void launch_grid_params(clsph_state* s);
 void launch_hash(clsph_state* s);
 void launch_track_ids(clsph_state* s);
+// Identities of all n_cap particles back to the canonical index.
+void launch_reset_ids(clsph_state* s);
 // Particle records (reference layout, canonical order) of a single-scene
 // state into out (device, n records), as the host download assembles them.
 void launch_pack_aos(clsph_state* s, clsph_particle* out);
+// Synchronous transfers: the inverse of a scene's canonical slots (into the
+// sort's scratch), records [r0, r0 + count) of a scene's n into a page-locked
+// buffer, and `count` records from one into the arrays at particle `first`.
+void launch_invert_slots(clsph_state* s, uint32_t scene);
+void launch_pack_records(clsph_state* s, uint32_t scene, uint32_t n, uint32_t r0, uint32_t count,
+                         bool sorted, void* out, TransferStatus* status);
+void launch_unpack_records(clsph_state* s, uint32_t first, uint32_t count, const void* in);
 // sort.hip
 // The sort: sorted keys and permutation, the half-cell table, the canonical
 // slots and the state gathered into sorted order.

@@ -272,12 +272,12 @@ class State:
         self.n = len(parts)
 
     def download(self):
-        out = layout.particles(self.n)
+        out = np.empty(self.n, dtype=layout.PARTICLE)
         self.ctx.check(lib.clsph_download_aos(self.h, _ptr(out), self.n))
         return out
 
     def download_sorted(self):
-        out = layout.particles(self.n)
+        out = np.empty(self.n, dtype=layout.PARTICLE)
         self.ctx.check(lib.clsph_download_sorted_aos(self.h, _ptr(out), self.n))
         return out
 
@@ -634,7 +634,7 @@ class Batch(State):
         self.ctx.check(lib.clsph_batch_upload(self.h, scene, _ptr(parts), len(parts)))
 
     def download_scene(self, scene):
-        out = layout.particles(self.counts[scene])
+        out = np.empty(self.counts[scene], dtype=layout.PARTICLE)
         self.ctx.check(lib.clsph_batch_download(self.h, scene, _ptr(out), len(out)))
         return out
 
