@@ -625,31 +625,201 @@ struct ForceConsts {
   float h, h2, m, c_spiky, c_visc, c_grad, c_lap, spiky0;
 };
 
-__device__ inline void force_pair(ForceSums& f, const ForceConsts& k, float4 ai, float4 bi,
-                                  float4 aj, float4 bj) {
+// Every rounding of the sums is written out, so that both kernels below (and
+// any inlining) compute the same bits.
+__device__ inline float length2(float x, float y, float z) {
+  return __builtin_fmaf(z, z, __builtin_fmaf(x, x, y * y));
+}
+
+// A pair's terms: each sum adds a weight times a value.
+struct PairTerms {
+  float g, vw, gw, lw;     // weights: pressure, viscosity, colour-field gradient and laplacian
+  float3 dir, dv, dx;      // values of the first three
+  float lv;
+};
+
+__device__ inline PairTerms pair_terms(const ForceConsts& k, float4 ai, float4 bi, float4 aj,
+                                       float4 bj) {
+#pragma clang fp contract(off)
+  PairTerms p;
   float dx = ai.x - aj.x, dy = ai.y - aj.y, dz = ai.z - aj.z;
-  float d2 = dx * dx + dy * dy + dz * dz;
+  float d2 = length2(dx, dy, dz);
   float r = __builtin_amdgcn_sqrtf(d2);
   float t = k.h2 - d2;
   float hr = k.h - r;
   // pressure (forces.cl:66-73): (p_j/rho_j^2 + p_i/rho_i^2) m grad W_spiky
   float ps = (aj.w + ai.w) * k.m;
   const bool coincident = r < 1e-7f;
-  float g = coincident ? ps * k.spiky0 : ps * k.c_spiky * hr * hr * __builtin_amdgcn_rcpf(r);
-  f.pt.x += g * (coincident ? 1.f : dx);
-  f.pt.y += g * (coincident ? 1.f : dy);
-  f.pt.z += g * (coincident ? 1.f : dz);
+  p.g = coincident ? ps * k.spiky0 : ps * k.c_spiky * hr * hr * __builtin_amdgcn_rcpf(r);
+  p.dir = make_float3(coincident ? 1.f : dx, coincident ? 1.f : dy, coincident ? 1.f : dz);
   // viscosity (forces.cl:75-80): (v_j - v_i) (m/rho_j) lap W_visc
-  float vw = bj.w * k.c_visc * hr;
-  f.vt.x += (bj.x - bi.x) * vw;
-  f.vt.y += (bj.y - bi.y) * vw;
-  f.vt.z += (bj.z - bi.z) * vw;
+  p.vw = bj.w * k.c_visc * hr;
+  p.dv = make_float3(bj.x - bi.x, bj.y - bi.y, bj.z - bi.z);
   // colour field gradient and laplacian (forces.cl:83-91)
-  float gw = bj.w * k.c_grad * t * t;
-  f.nrm.x += gw * dx;
-  f.nrm.y += gw * dy;
-  f.nrm.z += gw * dz;
-  f.lap += bj.w * k.c_lap * t * (3.f * k.h2 - 7.f * d2);
+  p.gw = bj.w * k.c_grad * t * t;
+  p.dx = make_float3(dx, dy, dz);
+  p.lw = bj.w * k.c_lap * t;
+  p.lv = __builtin_fmaf(-7.f, d2, 3.f * k.h2);
+  return p;
+}
+
+__device__ inline void force_pair(ForceSums& f, const ForceConsts& k, float4 ai, float4 bi,
+                                  float4 aj, float4 bj) {
+  const PairTerms p = pair_terms(k, ai, bi, aj, bj);
+  f.pt.x = __builtin_fmaf(p.g, p.dir.x, f.pt.x);
+  f.pt.y = __builtin_fmaf(p.g, p.dir.y, f.pt.y);
+  f.pt.z = __builtin_fmaf(p.g, p.dir.z, f.pt.z);
+  f.vt.x = __builtin_fmaf(p.vw, p.dv.x, f.vt.x);
+  f.vt.y = __builtin_fmaf(p.vw, p.dv.y, f.vt.y);
+  f.vt.z = __builtin_fmaf(p.vw, p.dv.z, f.vt.z);
+  f.nrm.x = __builtin_fmaf(p.gw, p.dx.x, f.nrm.x);
+  f.nrm.y = __builtin_fmaf(p.gw, p.dx.y, f.nrm.y);
+  f.nrm.z = __builtin_fmaf(p.gw, p.dx.z, f.nrm.z);
+  f.lap = __builtin_fmaf(p.lw, p.lv, f.lap);
+}
+
+__device__ inline ForceConsts force_consts(const DevParams* __restrict__ dp) {
+  ForceConsts k;
+  k.h = dp->p.h;
+  k.h2 = k.h * k.h;
+  k.m = dp->p.particle_mass;
+  k.c_spiky = dp->t.spiky;
+  k.c_visc = dp->t.viscosity;
+  k.c_grad = dp->t.poly_6_gradient;
+  k.c_lap = dp->t.poly_6_laplacian;
+  // Coincident-particle branch of spiky_gradient (smoothing.cl:23-25).
+  const float h3 = k.h2 * k.h;
+  k.spiky0 = -45.f / (3.14159274f * (h3 * h3));
+  return k;
+}
+
+// The sums before the first pair: the self term of the colour-field
+// laplacian, (m/rho_i) poly6_lap h^2 (3 h^2).
+__device__ inline ForceSums force_start(const ForceConsts& k, float4 bi) {
+  ForceSums fs;
+  fs.pt = make_float3(0.f, 0.f, 0.f);
+  fs.vt = fs.pt;
+  fs.nrm = fs.pt;
+  fs.lap = bi.w * k.c_lap * k.h2 * (3.f * k.h2);
+  return fs;
+}
+
+// More neighbours than the list holds: walks the half-cells again.
+__device__ inline void force_walk(ForceSums& fs, const ForceConsts& k, uint32_t i, float4 ai,
+                                  float4 bi, const float4* __restrict__ fab,
+                                  const uint32_t* __restrict__ table,
+                                  const DevParams* __restrict__ dp, uint32_t F, uint32_t n) {
+  uint32_t hc[3];
+  half_cell(ai, dp, hc);
+  const float h2 = k.h2;
+  for_each_candidate(hc, dp->key_base, table, F, n, [&](uint32_t j) {
+    float4 aj = fab[2u * j];
+    float d2 = length2(ai.x - aj.x, ai.y - aj.y, ai.z - aj.z);
+    if (!(d2 < h2) || j == i) return;
+    force_pair(fs, k, ai, bi, aj, fab[2u * j + 1u]);
+  });
+}
+
+// Acceleration from the sums (forces.cl:95-111 and sph.cl:53-58).
+__device__ inline float4 force_close(const ForceSums& fs, float rho_i,
+                                     const DevParams* __restrict__ dp) {
+#pragma clang fp contract(off)
+  const float3 pt = fs.pt, vt = fs.vt, nrm = fs.nrm;
+  const float mu = dp->p.dynamic_viscosity;
+  float3 f = make_float3(__builtin_fmaf(vt.x, mu, -(rho_i * pt.x)),
+                         __builtin_fmaf(vt.y, mu, -(rho_i * pt.y)),
+                         __builtin_fmaf(vt.z, mu, -(rho_i * pt.z)));
+  const float nl = sqrtf(length2(nrm.x, nrm.y, nrm.z));
+  if (nl > dp->p.surface_tension_threshold) {
+    const float kk = -dp->p.surface_tension * fs.lap / nl;
+    f.x = __builtin_fmaf(kk, nrm.x, f.x);
+    f.y = __builtin_fmaf(kk, nrm.y, f.y);
+    f.z = __builtin_fmaf(kk, nrm.z, f.z);
+  }
+  const clsph_float3& g = dp->p.constant_acceleration;
+  return make_float4(f.x / rho_i + g.s[0], f.y / rho_i + g.s[1], f.z / rho_i + g.s[2], 0.f);
+}
+
+// The forces stage by sixteen lanes per particle, for states too small to
+// fill the chip with one particle per lane (rule in launch_forces): a round
+// takes the next sixteen neighbours of the list, one per lane, and leaves
+// their terms in LDS; ten lanes then each add one sum's terms in list order,
+// so that every sum is the one lane's of k_forces to the bit. Bound by the
+// latency of the list, the two gathers and the serial sums; the next round's
+// gathers are in flight meanwhile (4,096 particles: 4.3 us, a lane each 10.5).
+constexpr int kForceLanes = 16, kForceLanesBlock = 256;
+constexpr uint32_t kForceLanesMax = 57344;  // particles up to which they do
+constexpr uint32_t kForceTerms = 14;  // PairTerms' floats, in order
+constexpr uint32_t kForcePitch = 20;  // floats between terms: 16-byte reads, spread over banks
+__global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
+    const float4* __restrict__ fab, const float* __restrict__ rho,
+    const uint32_t* __restrict__ table, const uint4* __restrict__ nbr,
+    const uint32_t* __restrict__ nbr_count, const BlockDesc* __restrict__ blocks,
+    const DevParams* __restrict__ dps, const BatchParams* __restrict__ bp,
+    float4* __restrict__ acc_out, uint32_t n) {
+  constexpr uint32_t L = kForceLanes, kParts = kForceLanesBlock / L, kShare = 64u / kParts;
+  __shared__ __attribute__((aligned(16))) float terms[kParts][kForceTerms * kForcePitch];
+  // a 64-particle entry of the work list is shared by kShare work-groups
+  const BlockDesc b = blocks[blockIdx.x / kShare];
+  const DevParams* dp = dps + b.scene;
+  const uint32_t part = threadIdx.x / L, sub = threadIdx.x % L;
+  const uint32_t p = b.first + (blockIdx.x % kShare) * kParts + part;
+  const uint32_t se = dp->begin + dp->n;
+  const bool live = p < se;
+  if (!__any(live)) return;
+  const uint32_t i = live ? p : se - 1u;
+  const ForceConsts k = force_consts(dp);
+  const float4 ai = fab[2u * i], bi = fab[2u * i + 1u];
+  const uint32_t all = nbr_count[i];
+  const uint32_t cnt = live && all <= kMaxNeighbours ? all : 0u;
+  float* w = terms[part];
+  auto index = [&](uint32_t q) {  // past the end: the particle itself
+    return q < cnt ? reinterpret_cast<const uint32_t*>(nbr)[4u * ((size_t)(q >> 2) * n + i) + (q & 3u)]
+                   : i;
+  };
+  // the sum this lane adds: its weight's and value's rows of the terms
+  const uint32_t sum = sub < 10u ? sub : 9u, kind = sum / 3u;
+  const uint32_t wrow = kind, vrow = 4u + sum;
+  float acc = kind == 3u ? force_start(k, bi).lap : 0.f;
+  uint32_t j = index(sub), jn = index(L + sub);
+  float4 aj = fab[2u * j], bj = fab[2u * j + 1u];
+  for (uint32_t q0 = 0; __any(q0 < cnt); q0 += L) {
+    const float4 na = fab[2u * jn], nb = fab[2u * jn + 1u];
+    jn = index(q0 + 2u * L + sub);
+    const PairTerms t = pair_terms(k, ai, bi, aj, bj);
+    const float v[kForceTerms] = {t.g,    t.vw,   t.gw,   t.lw,   t.dir.x, t.dir.y, t.dir.z,
+                                  t.dv.x, t.dv.y, t.dv.z, t.dx.x, t.dx.y,  t.dx.z,  t.lv};
+#pragma unroll
+    for (uint32_t r = 0; r < kForceTerms; ++r) w[r * kForcePitch + sub] = v[r];
+    wave_lds_fence();
+    const uint32_t left = cnt > q0 ? cnt - q0 : 0u, take = left < L ? left : L;
+#pragma unroll
+    for (uint32_t g = 0; g < L; g += 4u) {
+      const float4 wt = *(const float4*)(w + wrow * kForcePitch + g);
+      const float4 va = *(const float4*)(w + vrow * kForcePitch + g);
+      if (g < take) acc = __builtin_fmaf(wt.x, va.x, acc);
+      if (g + 1u < take) acc = __builtin_fmaf(wt.y, va.y, acc);
+      if (g + 2u < take) acc = __builtin_fmaf(wt.z, va.z, acc);
+      if (g + 3u < take) acc = __builtin_fmaf(wt.w, va.w, acc);
+    }
+    wave_lds_fence();
+    aj = na;
+    bj = nb;
+  }
+  w[sub] = acc;  // sub >= 10 repeats the last sum, past the ten
+  wave_lds_fence();
+  if (!live || sub != 0u) return;
+  ForceSums fs;
+  if (all <= kMaxNeighbours) {
+    fs.pt = make_float3(w[0], w[1], w[2]);
+    fs.vt = make_float3(w[3], w[4], w[5]);
+    fs.nrm = make_float3(w[6], w[7], w[8]);
+    fs.lap = w[9];
+  } else {
+    fs = force_start(k, bi);
+    force_walk(fs, k, i, ai, bi, fab, table, dp, usable_key_end(dp, bp), n);
+  }
+  acc_out[i] = force_close(fs, rho[i], dp);
 }
 
 // OVERFLOW_ONLY: only the particles whose neighbours overflow the list
@@ -671,26 +841,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__
   if (i == 0xFFFFFFFFu) return;
   if (OVERFLOW_ONLY && nbr_count[i] <= kMaxNeighbours) return;
   const DevParams* dp = dps + scene;
-  ForceConsts k;
-  k.h = dp->p.h;
-  k.h2 = k.h * k.h;
-  k.m = dp->p.particle_mass;
-  k.c_spiky = dp->t.spiky;
-  k.c_visc = dp->t.viscosity;
-  k.c_grad = dp->t.poly_6_gradient;
-  k.c_lap = dp->t.poly_6_laplacian;
-  // Coincident-particle branch of spiky_gradient (smoothing.cl:23-25).
-  const float h3 = k.h2 * k.h;
-  k.spiky0 = -45.f / (3.14159274f * (h3 * h3));
+  const ForceConsts k = force_consts(dp);
   const uint32_t F = usable_key_end(dp, bp);
   float4 ai = fab[2u * i], bi = fab[2u * i + 1u];
   float rho_i = rho[i];
-  ForceSums fs;
-  fs.pt = make_float3(0.f, 0.f, 0.f);
-  fs.vt = fs.pt;
-  fs.nrm = fs.pt;
-  // Self term of the colour-field laplacian: (m/rho_i) poly6_lap h^2 (3 h^2).
-  fs.lap = bi.w * k.c_lap * k.h2 * (3.f * k.h2);
+  ForceSums fs = force_start(k, bi);
   uint32_t cnt = nbr_count[i];
   if (cnt <= kMaxNeighbours) {
     // groups of four neighbours, software-pipelined: while a group's pair
@@ -731,33 +886,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__
       if (r > 2) force_pair(fs, k, ai, bi, fab[2u * js.z], fab[2u * js.z + 1u]);
     }
   } else {
-    // More neighbours than the list holds: walk the half-cells again.
-    uint32_t hc[3];
-    half_cell(ai, dp, hc);
-    const float h2 = k.h2;
-    for_each_candidate(hc, dp->key_base, table, F, n, [&](uint32_t j) {
-      float4 aj = fab[2u * j];
-      float dx = ai.x - aj.x, dy = ai.y - aj.y, dz = ai.z - aj.z;
-      float d2 = dx * dx + dy * dy + dz * dz;
-      if (!(d2 < h2) || j == i) return;
-      force_pair(fs, k, ai, bi, aj, fab[2u * j + 1u]);
-    });
+    force_walk(fs, k, i, ai, bi, fab, table, dp, F, n);
   }
-  float3 pt = fs.pt, vt = fs.vt, nrm = fs.nrm;
-  float lap = fs.lap;
-  // forces.cl:95-111 and sph.cl:53-58
-  float mu = dp->p.dynamic_viscosity;
-  float3 f = make_float3(-rho_i * pt.x + vt.x * mu, -rho_i * pt.y + vt.y * mu,
-                         -rho_i * pt.z + vt.z * mu);
-  float nl = sqrtf(nrm.x * nrm.x + nrm.y * nrm.y + nrm.z * nrm.z);
-  if (nl > dp->p.surface_tension_threshold) {
-    float kk = -dp->p.surface_tension * lap / nl;
-    f.x += kk * nrm.x;
-    f.y += kk * nrm.y;
-    f.z += kk * nrm.z;
-  }
-  const clsph_float3& g = dp->p.constant_acceleration;
-  acc_out[i] = make_float4(f.x / rho_i + g.s[0], f.y / rho_i + g.s[1], f.z / rho_i + g.s[2], 0.f);
+  acc_out[i] = force_close(fs, rho_i, dp);
 }
 
 void launch_density(clsph_state* s, float2* nu) {
@@ -794,6 +925,19 @@ void launch_density(clsph_state* s, float2* nu) {
 
 void launch_forces(clsph_state* s) {
   if (s->n == 0) return;
+  // One lane per particle does half the work, but takes at least a lane's
+  // whole list: 10.5 us with 35 neighbours, 24-29 us with the up to 128 of a
+  // settled dam break. Stage times with 1 / 16 lanes, early and settled: 4,096
+  // particles 10.5 / 4.3 and 15.5 / 5.6 us, 16,384 11.6 / 6.3 and 22.7 / 8.9,
+  // 50,021 12.1 / 13.4 and 28.1 / 20.4, 65,536 12.1 / 15.6 and 28.9 / 24.3,
+  // 98,304 12.2 / 22.1 and 28.2 / 32.4.
+  if (s->n <= kForceLanesMax) {
+    constexpr uint32_t kShare = 64u * kForceLanes / kForceLanesBlock;
+    hipLaunchKernelGGL(k_forces_lanes, dim3(s->nblocks[0] * kShare), dim3(kForceLanesBlock), 0,
+                       s->ctx->stream, s->fab, s->rho_s, s->table, s->nbr, s->nbr_count,
+                       s->blocks[0], s->dps, s->bp, s->acc_s, s->n);
+    return;
+  }
   hipLaunchKernelGGL((k_forces<false>), dim3(s->nblocks_of(kStageForces)),
                      dim3(s->bs_of(kStageForces)), 0, s->ctx->stream, s->fab, s->rho_s,
                      s->table, s->nbr, s->nbr_count, s->table_of(kStageForces), s->dps, s->bp,
