@@ -46,7 +46,7 @@ void free_state_buffers(clsph_state* st) {
   dfree(st->nbr), dfree(st->nbr_count);
   dfree(st->key_a), dfree(st->key_t), dfree(st->val_t), dfree(st->key_u), dfree(st->val_u);
   dfree(st->key_b), dfree(st->val_b);
-  dfree(st->sort_hist), dfree(st->sort_totals), dfree(st->sort_runs), dfree(st->sort_runs_ctl);
+  dfree(st->sort_hist), dfree(st->sort_totals);
   dfree(st->table), dfree(st->slot);
   dfree(st->ids), dfree(st->ids_tmp);
   dfree(st->aabb_partial);
@@ -262,9 +262,7 @@ int rebuild_meshes(clsph_state* st) {
 
 // Launches the kernels of one whole substep on the context stream.
 void enqueue_step(clsph_state* st) {
-  launch_grid_params(st);
-  launch_hash(st);
-  launch_sort(st);
+  launch_grid_to_sort(st);
   launch_density(st);
   launch_forces(st);
   launch_advect(st);
@@ -369,10 +367,6 @@ int alloc_state(clsph_ctx* ctx, uint32_t n_scenes, const uint32_t* caps, bool fi
     if (rc == CLSPH_OK) rc = dalloc(ctx, p, n_cap);
   if (rc == CLSPH_OK) rc = dalloc(ctx, &st->sort_hist, (size_t)st->n_tiles_cap * kMaxBins);
   if (rc == CLSPH_OK) rc = dalloc(ctx, &st->sort_totals, (size_t)kMaxBins);
-  st->sort_runs_cap = sort_runs_cap_for(st->table_cap);
-  if (rc == CLSPH_OK) rc = dalloc(ctx, &st->sort_runs, (size_t)st->sort_runs_cap);
-  if (rc == CLSPH_OK) rc = dalloc(ctx, &st->sort_runs_ctl, 2);
-  if (rc == CLSPH_OK) HIPCK(ctx, hipMemset(st->sort_runs_ctl, 0, 2 * sizeof(uint32_t)));
   if (rc == CLSPH_OK) rc = dalloc(ctx, &st->table, (size_t)st->table_cap + 1);
   st->aabb_stride = (uint32_t)(blocks64 + 1);
   if (rc == CLSPH_OK) rc = dalloc(ctx, &st->aabb_partial, (size_t)st->aabb_stride * 6);

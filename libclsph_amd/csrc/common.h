@@ -109,17 +109,19 @@ __host__ __device__ inline uint32_t bitlen(uint32_t v) {
 // locate_in_grid (grid.cl:43-67): the reference's cell id is
 // Morton((uint)((x - min) / (h * 2))); the half-cell key adds the octant and
 // the scene's key base.
-__device__ inline uint32_t hash_key(float4 p, const DevParams* __restrict__ dp) {
+__device__ inline uint32_t hash_key(float4 p, float h, const float mn[3], uint32_t key_base) {
 #pragma clang fp contract(off)
-  float L = dp->p.h * 2;
-  float u[3] = {(p.x - dp->p.min_point.s[0]) / L, (p.y - dp->p.min_point.s[1]) / L,
-                (p.z - dp->p.min_point.s[2]) / L};
+  float L = h * 2;
+  float u[3] = {(p.x - mn[0]) / L, (p.y - mn[1]) / L, (p.z - mn[2]) / L};
   uint32_t c[3], oct = 0;
   for (int a = 0; a < 3; ++a) {
     c[a] = (uint32_t)u[a];
     oct |= (((uint32_t)(2.f * u[a])) & 1u) << a;
   }
-  return dp->key_base + ((morton3(c[0], c[1], c[2]) << 3) | oct);
+  return key_base + ((morton3(c[0], c[1], c[2]) << 3) | oct);
+}
+__device__ inline uint32_t hash_key(float4 p, const DevParams* __restrict__ dp) {
+  return hash_key(p, dp->p.h, dp->p.min_point.s, dp->key_base);
 }
 
 // The learned surrogate's node inputs of a particle: nu = [rho / rho0 - 1,

@@ -13,6 +13,7 @@
 // (reference key << 3) | octant, so sorting by it keeps the reference's cells
 // contiguous and in order, each grouped by octant. A scene's keys are offset
 // by its key_base.
+#include "grid_params.h"
 #include "reduce.h"
 #include "state.h"
 
@@ -29,25 +30,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_aabb(const float4* __restrict__ p
   bool valid = i != 0xFFFFFFFFu;
   float4 p = valid ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   block_aabb_partial(p, valid, partial, stride);
-}
-
-// The batch's key total, key width and sort digit width for `base` keys in
-// all (one thread); `err` holds the error bits raised while laying them out.
-__device__ void batch_layout(BatchParams* __restrict__ bp, uint64_t base, uint32_t err,
-                             uint32_t table_cap, uint32_t sort_passes) {
-  if (base > table_cap) err |= kErrTableCap;
-  bp->key_total = (uint32_t)base;
-  uint32_t kb = bitlen((uint32_t)base);
-  bp->key_bits = kb;
-  // the sort orders by cell id (key >> 3) in sort_passes LSD passes; a state
-  // sized for three runs two while the cell ids fit them
-  uint32_t cb = kb > 3u ? kb - 3u : 1u;
-  uint32_t passes = sort_passes ? sort_passes : 1u;
-  if (passes > 2u && cb <= 2u * (uint32_t)kMaxDigitBits) passes = 2u;
-  bp->lsd_passes = passes;
-  uint32_t db = (cb + passes - 1u) / passes;
-  bp->digit_bits = db < 1u ? 1u : (db > (uint32_t)kMaxDigitBits ? (uint32_t)kMaxDigitBits : db);
-  if (err) atomicOr(&bp->err, err);
 }
 
 // Lays the scenes' half-cell key ranges end to end (each scene gets
@@ -91,9 +73,6 @@ __device__ void batch_keys(DevParams* __restrict__ dps, BatchParams* __restrict_
 // the batch's keys (batch_keys); a single scene does so from the values in
 // its registers. The parameters thread 0 needs are loaded before the
 // reduction, so that their latency overlaps it.
-__device__ uint32_t scene_grid(DevParams* __restrict__ dp, const float v[6], float h, uint32_t n,
-                               uint32_t& G);
-
 __global__ __launch_bounds__(1024) void k_grid_params(DevParams* __restrict__ dps,
                                                       const float* __restrict__ partial,
                                                       uint32_t stride,
@@ -103,60 +82,16 @@ __global__ __launch_bounds__(1024) void k_grid_params(DevParams* __restrict__ dp
   const float h = dp->p.h;
   const uint32_t np = dp->n, err0 = dp->err;
   const uint32_t table_cap = bp->table_cap, sort_passes = bp->sort_passes;
-  const float inf = __builtin_huge_valf();
-  float v[6] = {inf, inf, inf, -inf, -inf, -inf};
-  // eight partial boxes per thread in flight at a time
-  const uint32_t b0 = dp->block_begin, b1 = dp->block_end;
-  for (uint32_t b = b0 + threadIdx.x; b < b1; b += 8u * blockDim.x) {
-    float q[8][6];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const uint32_t bu = b + (uint32_t)u * blockDim.x;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) q[u][k] = bu < b1 ? partial[k * stride + bu] : (k < 3 ? inf : -inf);
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      for (int k = 0; k < 3; ++k) v[k] = fminf(v[k], q[u][k]);
-      for (int k = 3; k < 6; ++k) v[k] = fmaxf(v[k], q[u][k]);
-    }
-  }
-  for (int k = 0; k < 3; ++k) v[k] = wave_min(v[k]);
-  for (int k = 3; k < 6; ++k) v[k] = wave_max(v[k]);
-  int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  if (l == 0)
-    for (int k = 0; k < 6; ++k) red[k][w] = v[k];
-  __syncthreads();
-  if (threadIdx.x >= 64u) return;  // the first wave joins the waves' boxes
-  // lanes 0-15 take one wave's box each; a butterfly over 16 lanes leaves
-  // the scene's box in every lane
-  static_assert(sizeof(red[0]) / sizeof(float) == 16, "16 waves per work-group");
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    float r = red[k][l & 15];
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) {
-      const float y = __shfl_xor(r, o, 64);
-      r = (k < 3) ? fminf(r, y) : fmaxf(r, y);
-    }
-    v[k] = r;
-  }
+  float v[6];
+  if (!scene_box<16>(dp, partial, stride, red, v)) return;
   if (threadIdx.x != 0 && gridDim.x == 1u) return;
-  uint32_t G = 0, err = 0;
-  if (threadIdx.x == 0) err = scene_grid(dp, v, h, np, G);
-  if (gridDim.x == 1u) {
-    // one scene: batch_keys with the scene's values in registers
-    const uint64_t Gk = ((err0 | err) & kErrFineKey) ? 0u : G;
-    dp->key_base = 0;
-    dp->key_end = (uint32_t)(8ull * Gk);
-    uint64_t base = 8ull * (Gk + 1);
-    uint32_t berr = 0;
-    if (base > 0xFFFFFFF0ull) {
-      berr = kErrFineKey;
-      base = 0xFFFFFFF0ull;
+  if (threadIdx.x == 0) {
+    const GridOf g = grid_of(v, h, np);
+    store_grid(dp, g, np);
+    if (gridDim.x == 1u) {
+      single_layout(dp, bp, g.cells, err0 | g.err, table_cap, sort_passes);
+      return;
     }
-    batch_layout(bp, base, berr, table_cap, sort_passes);
-    return;
   }
   // the scenes' grids are in place once every work-group has passed here
   uint32_t last = 0;
@@ -168,46 +103,6 @@ __global__ __launch_bounds__(1024) void k_grid_params(DevParams* __restrict__ dp
   __threadfence();
   if (threadIdx.x == 0) bp->ticket = 0;
   batch_keys(dps, bp);
-}
-
-// The grid of one scene from its bounding box v = (min xyz, max xyz), its
-// smoothing length h and particle count n; returns the error bits it raised
-// and the cell count in G.
-__device__ uint32_t scene_grid(DevParams* __restrict__ dp, const float v[6], float h, uint32_t n,
-                               uint32_t& G) {
-  dp->capped = 0;
-  G = 0;
-  if (n == 0) {
-    dp->p.grid_cell_count = 0;
-    return 0u;
-  }
-  // Initial values are numeric_limits<cl_int>::max()/min() as float; a
-  // position replaces them only when strictly smaller / larger.
-  const float init_min = 2147483648.0f, init_max = -2147483648.0f;
-  float L = h * 2;
-  float mn[3], mx[3];
-  uint32_t gs[3];
-  uint32_t err = 0;
-  for (int a = 0; a < 3; ++a) {
-    mn[a] = (v[a] < init_min) ? v[a] : init_min;
-    mx[a] = (v[3 + a] > init_max) ? v[3 + a] : init_max;
-    mn[a] -= L * 2;
-    mx[a] += L * 2;
-    gs[a] = (uint32_t)((mx[a] - mn[a]) / L);
-    if (gs[a] >= 1024u) err |= kErrGridDim;
-    dp->p.min_point.s[a] = mn[a];
-    dp->p.max_point.s[a] = mx[a];
-  }
-  dp->p.min_point.s[3] = 0.f;
-  dp->p.max_point.s[3] = 0.f;
-  dp->p.grid_size_x = (int32_t)gs[0];
-  dp->p.grid_size_y = (int32_t)gs[1];
-  dp->p.grid_size_z = (int32_t)gs[2];
-  G = morton3(gs[0], gs[1], gs[2]);
-  dp->p.grid_cell_count = G;
-  if (G >= (1u << 29)) err |= kErrFineKey;
-  if (err) atomicOr(&dp->err, err);
-  return err;
 }
 
 // Half-cell keys of every particle (hash_key).

@@ -94,9 +94,7 @@ int copy_state_async(clsph_state* dst, clsph_state* src) {
 
 // The stages of a substep up to density, as clsph_grid .. clsph_density_pressure.
 void enqueue_density_stages(clsph_state* st) {
-  launch_grid_params(st);
-  launch_hash(st);
-  launch_sort(st);
+  launch_grid_to_sort(st);
   launch_density(st);
   st->acc_learned = false;
   st->fields_canonical = false;
@@ -119,9 +117,7 @@ int ensure_learned_graph(clsph_state* st, clsph_nn* m) {
   }
   hipGraph_t graph = nullptr;
   HIPCK(st->ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  launch_grid_params(st);
-  launch_hash(st);
-  launch_sort(st);
+  launch_grid_to_sort(st);
   launch_density(st, (float2*)m->nu);
   launch_forces_overflow(st);
   nn::forward_fused(m, st, st->acc_s, nullptr, true, nullptr, true);

@@ -12,9 +12,11 @@
 //     keys), k_lsd_scan (each digit's counts scanned over the tiles) and
 //     k_lsd_scatter (keys ranked in registers with wave64 ballot matching,
 //     the tile reordered digit-major in LDS, each digit run written to
-//     consecutive addresses). After the passes the particles are in the
-//     reference's order, with their canonical indices. A state whose table
-//     capacity needs three passes launches three, and its third pass does
+//     consecutive addresses). With few tiles the scatter does the scan's
+//     part itself, and a substep's first count also does the grid stage and
+//     the hash (k_grid_count): a launch costs 3-5 us whatever its size. After
+//     the passes the particles are in the reference's order, with their
+//     canonical indices. A state whose table capacity needs three passes launches three, and its third pass does
 //     nothing in a substep whose cell ids fit two (22 bits): the pass count
 //     of the substep is set on the device with the digit width.
 //  2. k_cells: each cell's particles are contiguous in that order; a
@@ -24,6 +26,9 @@
 //     position its position in the reference's order (the canonical slot,
 //     where advection writes the particle back). It gathers the state into
 //     sorted order on the way.
+#include <algorithm>
+
+#include "grid_params.h"
 #include "state.h"
 
 namespace clsph {
@@ -79,27 +84,14 @@ __device__ inline uint32_t pass_digit(uint32_t key, uint32_t db, uint32_t pass) 
 
 // ---- 1. LSD passes ----------------------------------------------------------
 
-// Digit counts of each tile: hist[tile * nb + d].
-__global__ __launch_bounds__(kLsdBlock) void k_lsd_count(const uint32_t* __restrict__ keys,
-                                                         uint32_t n,
-                                                         const BatchParams* __restrict__ bp,
-                                                         uint32_t pass,
-                                                         uint32_t* __restrict__ hist,
-                                                         uint32_t* __restrict__ runs_ctl) {
-  __shared__ uint32_t bins[kMaxBins];
-  // the first pass also empties the cell pass's list of long runs
-  if (pass == 0 && blockIdx.x == 0 && threadIdx.x == 0) runs_ctl[0] = 0;
-  if (pass >= lsd_passes_of(bp)) return;
-  const uint32_t db = bp->digit_bits, nb = 1u << db;
-  for (uint32_t d = threadIdx.x; d < nb; d += kLsdBlock) bins[d] = 0;
+// Digit counts of one tile's keys (kk: key t of the thread at base +
+// t * kLsdBlock + threadIdx.x) into row[d]. Every thread calls it.
+__device__ inline void count_tile(const uint32_t kk[kLsdItems], uint32_t base, uint32_t n,
+                                  uint32_t db, uint32_t pass, uint32_t (&bins)[kMaxBins],
+                                  uint32_t* __restrict__ row) {
+  const uint32_t nb = 1u << db;
   const int lane = threadIdx.x & 63;
-  const uint32_t base = blockIdx.x * kLsdTile;
-  uint32_t kk[kLsdItems];
-#pragma unroll
-  for (int t = 0; t < kLsdItems; ++t) {
-    const uint32_t i = base + t * kLsdBlock + threadIdx.x;
-    kk[t] = i < n ? keys[i] : 0u;
-  }
+  for (uint32_t d = threadIdx.x; d < nb; d += kLsdBlock) bins[d] = 0;
   __syncthreads();
 #pragma unroll
   for (int t = 0; t < kLsdItems; ++t) {
@@ -117,7 +109,71 @@ __global__ __launch_bounds__(kLsdBlock) void k_lsd_count(const uint32_t* __restr
     if (head) atomicAdd(&bins[d], next - (uint32_t)lane);
   }
   __syncthreads();
-  for (uint32_t d = threadIdx.x; d < nb; d += kLsdBlock) hist[(size_t)blockIdx.x * nb + d] = bins[d];
+  for (uint32_t d = threadIdx.x; d < nb; d += kLsdBlock) row[d] = bins[d];
+}
+
+// Digit counts of each tile: hist[tile * nb + d].
+__global__ __launch_bounds__(kLsdBlock) void k_lsd_count(const uint32_t* __restrict__ keys,
+                                                         uint32_t n,
+                                                         const BatchParams* __restrict__ bp,
+                                                         uint32_t pass,
+                                                         uint32_t* __restrict__ hist) {
+  __shared__ uint32_t bins[kMaxBins];
+  if (pass >= lsd_passes_of(bp)) return;
+  const uint32_t db = bp->digit_bits;
+  const uint32_t base = blockIdx.x * kLsdTile;
+  uint32_t kk[kLsdItems];
+#pragma unroll
+  for (int t = 0; t < kLsdItems; ++t) {
+    const uint32_t i = base + t * kLsdBlock + threadIdx.x;
+    kk[t] = i < n ? keys[i] : 0u;
+  }
+  count_tile(kk, base, n, db, pass, bins, hist + ((size_t)blockIdx.x << db));
+}
+
+// Grid parameters, keys and the first pass's digit counts of a single scene in
+// one launch, for states whose launches cost more than their work: every
+// work-group reduces the scene's boxes for itself (24 bytes per 256 particles,
+// from L2) and computes the grid; the first one stores it.
+__global__ __launch_bounds__(kLsdBlock) void k_grid_count(
+    const float4* __restrict__ pos, uint32_t n, DevParams* __restrict__ dp,
+    BatchParams* __restrict__ bp, const float* __restrict__ partial, uint32_t stride,
+    uint32_t* __restrict__ key, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t bins[kMaxBins];
+  __shared__ float red[6][kLsdBlock / 64];
+  __shared__ float g_min[3];
+  __shared__ uint32_t g_db;
+  const uint32_t base = blockIdx.x * kLsdTile;
+  float4 x[kLsdItems];
+#pragma unroll
+  for (int t = 0; t < kLsdItems; ++t) {
+    const uint32_t i = base + t * kLsdBlock + threadIdx.x;
+    x[t] = i < n ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const float h = dp->p.h;
+  const uint32_t np = dp->n, err0 = dp->err, table_cap = bp->table_cap, passes = bp->sort_passes;
+  float v[6];
+  if (scene_box<kLsdBlock / 64>(dp, partial, stride, red, v) && threadIdx.x == 0) {
+    const GridOf g = grid_of(v, h, np);
+    const uint32_t err = err0 | g.err;  // the same in every work-group, stored by now or not
+    for (int a = 0; a < 3; ++a) g_min[a] = g.mn[a];
+    g_db = key_layout(single_total(single_keys(g.cells, err)), passes).digit_bits;
+    if (blockIdx.x == 0) {
+      store_grid(dp, g, np);
+      single_layout(dp, bp, g.cells, err, table_cap, passes);
+    }
+  }
+  __syncthreads();
+  const float mn[3] = {g_min[0], g_min[1], g_min[2]};
+  uint32_t kk[kLsdItems];
+#pragma unroll
+  for (int t = 0; t < kLsdItems; ++t) {
+    const uint32_t i = base + t * kLsdBlock + threadIdx.x;
+    kk[t] = hash_key(x[t], h, mn, 0u);
+    if (i < n) key[i] = kk[t];
+  }
+  const uint32_t db = g_db;
+  count_tile(kk, base, n, db, 0u, bins, hist + ((size_t)blockIdx.x << db));
 }
 
 // Each digit's counts scanned over the tiles, in place (exclusive), and the
@@ -196,10 +252,15 @@ __global__ __launch_bounds__(kScanBlock) void k_lsd_scan(uint32_t* __restrict__ 
 // counts while the keys are ranked, the first half of the same bytes then
 // holding the tile's keys and values in digit order; each digit's run start
 // in that copy (16-bit), and its output start minus that run start.
+//
+// FOLD: `offsets` holds the tiles' counts as k_lsd_count left them, and the
+// work-group adds up each digit's counts over the tiles for itself, for few
+// tiles (rule in launch_sort).
 constexpr int kScatBlock = 512;                         // scatter threads per tile
 constexpr int kScatItems = kLsdTile / kScatBlock;       // keys per thread
 constexpr int kScatWaves = kScatBlock / 64;
 constexpr int kScatWaveKeys = kLsdTile / kScatWaves;    // consecutive keys per wave
+template <bool FOLD>
 __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, uint32_t n,
     const BatchParams* __restrict__ bp, uint32_t pass, const uint32_t* __restrict__ offsets,
@@ -211,6 +272,7 @@ __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
   __shared__ uint4 stage[kStageQ];
   __shared__ uint16_t tile_start[kMaxBins];   // digit runs in the LDS copy of the tile
   __shared__ uint32_t dshift[kMaxBins];       // output start of a digit's run - tile_start
+  __shared__ uint32_t tot[FOLD ? kMaxBins : 1];  // digit totals
   uint16_t(*wcnt)[kMaxBins] = reinterpret_cast<uint16_t(*)[kMaxBins]>(stage);
   uint32_t* skey = reinterpret_cast<uint32_t*>(stage);
   uint32_t* sval = skey + kLsdTile;
@@ -227,6 +289,31 @@ __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
   }
   for (uint32_t q = threadIdx.x; q < kStageQ; q += kScatBlock)
     stage[q] = make_uint4(0u, 0u, 0u, 0u);
+  if constexpr (FOLD) {
+    // totals and counts of the tiles before this one: for few digits, several
+    // threads share one and take every S-th tile
+    for (uint32_t d = threadIdx.x; d < nb; d += kScatBlock) tot[d] = dshift[d] = 0u;
+    __syncthreads();
+    const uint32_t S = nb < (uint32_t)kScatBlock ? (uint32_t)kScatBlock >> db : 1u;
+    const uint32_t first = nb < (uint32_t)kScatBlock ? threadIdx.x >> db : 0u;
+    for (uint32_t d = S > 1u ? threadIdx.x & (nb - 1u) : threadIdx.x; d < nb; d += kScatBlock) {
+      uint32_t all = 0, before = 0;
+#pragma unroll 8
+      for (uint32_t q = first; q < gridDim.x; q += S) {
+        const uint32_t c = offsets[((size_t)q << db) + d];
+        all += c;
+        before += q < blockIdx.x ? c : 0u;
+      }
+      if (S > 1u) {
+        atomicAdd(&tot[d], all);
+        atomicAdd(&dshift[d], before);
+      } else {
+        tot[d] = all;
+        dshift[d] = before;
+      }
+    }
+    __syncthreads();
+  }
   // where each digit's run of this tile starts in the output: the digit's
   // start (exclusive scan of the totals) plus the tiles before this one
   constexpr int per = kMaxBins / kScatBlock;
@@ -236,8 +323,13 @@ __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
 #pragma unroll
     for (int k = 0; k < per; ++k) {
       const uint32_t d = threadIdx.x * per + k;
-      v[k] = d < nb ? totals[d] : 0u;
-      o[k] = d < nb ? offsets[(size_t)blockIdx.x * nb + d] : 0u;
+      if constexpr (FOLD) {
+        v[k] = d < nb ? tot[d] : 0u;
+        o[k] = d < nb ? dshift[d] : 0u;
+      } else {
+        v[k] = d < nb ? totals[d] : 0u;
+        o[k] = d < nb ? offsets[(size_t)blockIdx.x * nb + d] : 0u;
+      }
       local += v[k];
     }
     uint32_t run = block_exclusive_scan<kScatBlock>(local);
@@ -350,8 +442,7 @@ __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
 constexpr int kCellRange = 256;                     // positions whose cells a work-group owns
 constexpr int kCellAhead = 256;                     // positions past them staged for the last cell
 constexpr int kCellSpan = kCellRange + kCellAhead;  // [a, b) inverted in LDS up to this
-constexpr int kLongRun = 4096;  // empty keys a work-group writes itself; longer runs are listed
-constexpr int kFillBlocks = 512;
+constexpr int kLongRun = 4096;  // empty keys a work-group writes itself
 
 // Writes the particle at reference position k (key, canonical index src) to
 // sorted position dst.
@@ -376,9 +467,7 @@ __device__ __forceinline__ void cells_place(
     const uint32_t* stk, const uint32_t* __restrict__ sk, const uint32_t* __restrict__ sv,
     uint32_t n, uint32_t r0, uint32_t a, uint32_t b, uint32_t total, bool table_ok, uint32_t* inv,
     uint32_t* c_start, uint32_t* c_id, uint32_t (*c_oct)[8], uint32_t (*wtot)[9],
-    uint32_t (*pre)[9], uint32_t* carry, uint4* __restrict__ runs, uint32_t* __restrict__ runs_ctl,
-    uint32_t runs_cap,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t* __restrict__ slot,
+    uint32_t (*pre)[9], uint32_t* carry, uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t* __restrict__ slot,
     uint32_t* __restrict__ table, const float4* __restrict__ pos, const float4* __restrict__ vel,
     const float4* __restrict__ vh, float4* __restrict__ pos_s, float4* __restrict__ vel_s,
     float4* __restrict__ vh_s) {
@@ -451,7 +540,7 @@ __device__ __forceinline__ void cells_place(
   // keys after each cell. A key of an owned cell holds the start of its
   // octant run; an empty key the start of the next cell. Runs of more than
   // kLongRun empty keys (the sparse Morton range leaves a few of hundreds of
-  // thousands) are listed for k_fill_runs, which spreads them over the chip.
+  // thousands) are left to fill_long_runs, which spreads them over the chip.
   if (table_ok) {
     // the eight keys of every owned cell, one (cell, octant) per thread: the
     // cell's start plus its particles of lower octants
@@ -474,17 +563,8 @@ __device__ __forceinline__ void cells_place(
         f1 = j + 1 < (int)ncells ? (c_id[j + 1] << 3) : kend;
         v = c_start[j + 1];
       }
-      if (f1 - f0 > (uint32_t)kLongRun && f1 > f0) {
-        if (threadIdx.x == 0) {
-          const uint32_t i = atomicAdd(&runs_ctl[0], 1u);
-          if (i < runs_cap)
-            runs[i] = make_uint4(f0, f1, v, 0u);
-          else
-            for (uint32_t f = f0; f < f1; ++f) table[f] = v;  // list full: written here
-        }
-      } else {
-        for (uint32_t f = f0 + threadIdx.x; f < f1; f += kCellBlock) table[f] = v;
-      }
+      if (f1 > f0 && f1 - f0 > (uint32_t)kLongRun) continue;
+      for (uint32_t f = f0 + threadIdx.x; f < f1; f += kCellBlock) table[f] = v;
     }
   }
   __syncthreads();
@@ -550,11 +630,59 @@ __device__ __forceinline__ void cells_place(
 #undef KEY_AT
 }
 
+// First position whose cell id (key >> 3) is at least `cell` in the n keys of
+// sk, by a wave: 64 probes a round.
+__device__ inline uint32_t first_at_cell(const uint32_t* __restrict__ sk, uint32_t n,
+                                         uint32_t cell) {
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t step = (hi - lo + 63u) >> 6;
+    const uint32_t p = lo + ((threadIdx.x & 63u) + 1u) * step - 1u;
+    const bool below = p < hi && (sk[p] >> 3) < cell;
+    const uint32_t c = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(below));
+    lo += c * step;
+    if (lo > hi) lo = hi;
+    const uint32_t top = lo + step - 1u;
+    hi = top < hi ? top : hi;
+  }
+  return lo;
+}
+
+// The table's runs of more than kLongRun empty keys, by the waves of the
+// launch's first `fillers` work-groups, kLongRun keys at a time: such a run
+// covers a multiple of kLongRun, so a wave finds what lies in its keys
+// [x, x + kLongRun) from the cells around either end, whatever else is in
+// between. (A kernel of its own over a list left by the owners took 4.5 us at
+// every size: 7 % of a substep of 16,384 particles, 1.3 % at 1,048,576.)
+__device__ inline void fill_long_runs(const uint32_t* __restrict__ sk, uint32_t n, uint32_t total,
+                                      uint32_t fillers, uint32_t* __restrict__ table) {
+  constexpr uint32_t kWaves = kCellBlock / 64, kRun = kLongRun;
+  const uint32_t lane = threadIdx.x & 63u;
+  // the long run that holds key x (a multiple of kRun), or an empty one
+  auto run_at = [&](uint32_t x, uint32_t& f0, uint32_t& f1, uint32_t& v) {
+    v = first_at_cell(sk, n, x >> 3);
+    f0 = v > 0u ? (sk[v - 1u] & ~7u) + 8u : 0u;
+    f1 = v < n ? sk[v] & ~7u : total + 1u;
+    if (f0 > x || f1 <= x || f1 - f0 <= kRun) f0 = f1 = x;
+  };
+  for (uint32_t c = blockIdx.x * kWaves + (threadIdx.x >> 6); c <= total / kRun;
+       c += fillers * kWaves) {
+    const uint32_t x = c * kRun, end = total - x < kRun ? total + 1u : x + kRun;
+    uint32_t f0, f1, v;
+    run_at(x, f0, f1, v);
+    f1 = f1 < end ? f1 : end;
+    for (uint32_t f = x + lane; f < f1; f += 64u) table[f] = v;
+    if (end > total) continue;
+    run_at(end, f0, f1, v);
+    if (f0 <= x) continue;  // the same run
+    for (uint32_t f = f0 + lane; f < end; f += 64u) table[f] = v;
+  }
+}
+
 __global__ __launch_bounds__(kCellBlock) void k_cells(
     const uint32_t* __restrict__ sk_odd, const uint32_t* __restrict__ sv_odd,
     const uint32_t* __restrict__ sk_even, const uint32_t* __restrict__ sv_even, uint32_t n,
-    const BatchParams* __restrict__ bp, uint4* __restrict__ runs, uint32_t* __restrict__ runs_ctl,
-    uint32_t runs_cap, uint32_t* __restrict__ keys_out,
+    const BatchParams* __restrict__ bp, uint32_t fillers, uint32_t* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, uint32_t* __restrict__ slot, uint32_t* __restrict__ table,
     const float4* __restrict__ pos, const float4* __restrict__ vel, const float4* __restrict__ vh,
     float4* __restrict__ pos_s, float4* __restrict__ vel_s, float4* __restrict__ vh_s) {
@@ -576,7 +704,12 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(
   const uint32_t* __restrict__ sv = odd ? sv_odd : sv_even;
   const uint32_t total = bp->key_total;
   const bool table_ok = total <= bp->table_cap && !(bp->err & kErrFineKey);
-  const uint32_t r0 = blockIdx.x * kCellRange;
+  // the first work-groups fill the table's long runs of empty keys
+  if (blockIdx.x < fillers) {
+    if (table_ok) fill_long_runs(sk, n, total, fillers, table);
+    return;
+  }
+  const uint32_t r0 = (blockIdx.x - fillers) * kCellRange;
   if (r0 >= n) return;
   const uint32_t r1 = min(n, r0 + kCellRange);
   const uint32_t hi = min(n, r1 + kCellAhead);  // staged: positions [r0 - 1, hi)
@@ -627,61 +760,41 @@ __global__ __launch_bounds__(kCellBlock) void k_cells(
   // keys at a - 1 .. b - 1, and the key at b unless b = n
   if (b < hi || (b == n && hi == n))
     cells_place<true>(stk, sk, sv, n, r0, a, b, total, table_ok, inv, c_start, c_id, c_oct, wtot,
-                      pre, carry, runs, runs_ctl, runs_cap, keys_out, vals_out, slot, table, pos, vel, vh,
+                      pre, carry, keys_out, vals_out, slot, table, pos, vel, vh,
                       pos_s, vel_s, vh_s);
   else
     cells_place<false>(stk, sk, sv, n, r0, a, b, total, table_ok, inv, c_start, c_id, c_oct, wtot,
-                       pre, carry, runs, runs_ctl, runs_cap, keys_out, vals_out, slot, table, pos, vel, vh,
+                       pre, carry, keys_out, vals_out, slot, table, pos, vel, vh,
                        pos_s, vel_s, vh_s);
 #undef CELLS_STARTS_LDS
 #undef CELLS_STARTS_HBM
 }
 
-// The long runs of empty keys k_cells listed (runs_ctl[0] of them, at most
-// runs_cap): table[f] = value for f in [f0, f1), every work-group taking a
-// share of every run.
-__global__ __launch_bounds__(256) void k_fill_runs(const uint4* __restrict__ runs,
-                                                   uint32_t* __restrict__ runs_ctl,
-                                                   uint32_t runs_cap,
-                                                   uint32_t* __restrict__ table) {
-  __shared__ uint4 lr[256];
-  const uint32_t count = min(runs_ctl[0], runs_cap);
-  const uint32_t stride = gridDim.x * 256u;
-  for (uint32_t i0 = 0; i0 < count; i0 += 256) {
-    if (i0 + threadIdx.x < count) lr[threadIdx.x] = runs[i0 + threadIdx.x];
-    __syncthreads();
-    const uint32_t m = min(count - i0, 256u);
-    for (uint32_t i = 0; i < m; ++i) {
-      const uint4 r = lr[i];
-      for (uint32_t f = r.x + blockIdx.x * 256u + threadIdx.x; f < r.y; f += stride) table[f] = r.z;
-    }
-    __syncthreads();
-  }
-}
-
-// Empties the list of long runs (before a cell pass run on its own; the sort
-// empties it in its first kernel).
-__global__ void k_clear_runs(uint32_t* __restrict__ runs_ctl) { runs_ctl[0] = 0; }
-
 void cell_pass(clsph_state* s) {
-  hipLaunchKernelGGL(k_cells, dim3((s->n + kCellRange - 1) / kCellRange), dim3(kCellBlock), 0,
-                     s->ctx->stream, s->key_t, s->val_t, s->key_u, s->val_u, s->n, s->bp, s->sort_runs, s->sort_runs_ctl,
-                     s->sort_runs_cap, s->key_b, s->val_b, s->slot, s->table, s->pos, s->vel,
-                     s->vh, s->pos_s, s->vel_s, s->vh_s);
-  hipLaunchKernelGGL(k_fill_runs, dim3(kFillBlocks), dim3(256), 0, s->ctx->stream, s->sort_runs,
-                     s->sort_runs_ctl, s->sort_runs_cap, s->table);
+  const uint32_t cells = (s->n + kCellRange - 1) / kCellRange;
+  const uint32_t fillers = std::min(512u, std::max(128u, cells / 8u));
+  hipLaunchKernelGGL(k_cells, dim3(fillers + cells), dim3(kCellBlock), 0, s->ctx->stream, s->key_t,
+                     s->val_t, s->key_u, s->val_u, s->n, s->bp, fillers, s->key_b, s->val_b,
+                     s->slot, s->table, s->pos, s->vel, s->vh, s->pos_s, s->vel_s, s->vh_s);
 }
 
 void launch_cell_table(clsph_state* s) {
-  if (s->n == 0) return;
-  hipLaunchKernelGGL(k_clear_runs, dim3(1), dim3(1), 0, s->ctx->stream, s->sort_runs_ctl);
-  cell_pass(s);
+  if (s->n != 0) cell_pass(s);
 }
 
-uint32_t sort_runs_cap_for(uint32_t table_cap) { return table_cap / kLongRun + 64u; }
+// Tiles up to which the scatter adds up the tiles' counts itself instead of
+// a scan kernel before it, and particles up to which one kernel does the grid
+// stage, the hash and the first counts. Substeps of the dam break, scan and
+// separate kernels / scan folded / both: 4,096 particles 66.3 / 60.5 / 57.9 us,
+// 16,384 70.9 / 65.3 / 62.1, 50,021 (25 tiles) 98.0 / 95.1 / 91.8, 98,304 (48)
+// 105.2 / 104.9 / 101.3, 131,071 (64) 118.6 / 119.5 / 116.2 (115.2 with the
+// scan); 524,288 213.8 and with the one kernel 210.5, 1,048,576 364.3 and 364.8.
+constexpr uint32_t kFoldTiles = 48;
+constexpr uint32_t kFusedMax = 655360;
 
-void launch_sort(clsph_state* s) {
-  if (s->n == 0) return;
+// The LSD passes and the cell pass; `counted`: the keys and the first pass's
+// counts are there.
+static void sort_keys(clsph_state* s, bool counted) {
   hipStream_t st = s->ctx->stream;
   const uint32_t tiles = sort_tiles_for(s->n);
   // pass p reads the previous pass's output: key_a (identity values), then
@@ -700,18 +813,41 @@ void launch_sort(clsph_state* s) {
     else if (per <= 32) go(k_lsd_scan<32>);
     else go(k_lsd_scan<0>);
   };
+  const bool fold = tiles <= kFoldTiles;
   for (uint32_t p = 0; p < s->sort_passes; ++p) {
     uint32_t* kout = (p & 1) ? s->key_u : s->key_t;
     uint32_t* vout = (p & 1) ? s->val_u : s->val_t;
-    hipLaunchKernelGGL(k_lsd_count, dim3(tiles), dim3(kLsdBlock), 0, st, kin, s->n, s->bp, p,
-                       s->sort_hist, s->sort_runs_ctl);
-    scan(p);
-    hipLaunchKernelGGL(k_lsd_scatter, dim3(tiles), dim3(kScatBlock), 0, st, kin, vin, s->n, s->bp,
-                       p, s->sort_hist, s->sort_totals, kout, vout);
+    if (p != 0 || !counted)
+      hipLaunchKernelGGL(k_lsd_count, dim3(tiles), dim3(kLsdBlock), 0, st, kin, s->n, s->bp, p,
+                         s->sort_hist);
+    if (!fold) scan(p);
+    auto scatter = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kScatBlock), 0, st, kin, vin, s->n, s->bp, p,
+                         s->sort_hist, s->sort_totals, kout, vout);
+    };
+    if (fold) scatter(k_lsd_scatter<true>);
+    else scatter(k_lsd_scatter<false>);
     kin = kout;
     vin = vout;
   }
   cell_pass(s);
+}
+
+void launch_sort(clsph_state* s) {
+  if (s->n != 0) sort_keys(s, false);
+}
+
+void launch_grid_to_sort(clsph_state* s) {
+  if (s->n_scenes != 1 || s->n == 0 || s->n > kFusedMax) {
+    launch_grid_params(s);
+    launch_hash(s);
+    launch_sort(s);
+  } else {
+    hipLaunchKernelGGL(k_grid_count, dim3(sort_tiles_for(s->n)), dim3(kLsdBlock), 0,
+                       s->ctx->stream, s->pos, s->n, s->dps, s->bp, s->aabb_partial,
+                       s->aabb_stride, s->key_a, s->sort_hist);
+    sort_keys(s, true);
+  }
 }
 
 }  // namespace clsph

@@ -87,12 +87,6 @@ struct clsph_state {
   uint32_t sort_passes = 2;           // LSD passes, from the table capacity
   uint32_t* sort_hist = nullptr;      // per-tile digit counts, then offsets (tiles x kMaxBins)
   uint32_t* sort_totals = nullptr;    // digit totals of the current pass (kMaxBins)
-  // long runs of empty keys of the half-cell table, listed by the cell pass
-  // and written by the fill pass ({first key, end key, value, 0}); the list's
-  // length (emptied before each cell pass) and a spare word
-  uint4* sort_runs = nullptr;
-  uint32_t* sort_runs_ctl = nullptr;
-  uint32_t sort_runs_cap = 0;
   uint32_t n_tiles_cap = 0;
 
   // Half-cell table (table_cap + 1 entries): table[f] = #{keys < f}; the
@@ -202,10 +196,11 @@ void launch_unpack_records(clsph_state* s, uint32_t first, uint32_t count, const
 // The sort: sorted keys and permutation, the half-cell table, the canonical
 // slots and the state gathered into sorted order.
 void launch_sort(clsph_state* s);
+// Grid parameters, keys and the sort, as the three launches above.
+void launch_grid_to_sort(clsph_state* s);
 // Its last pass alone (table, slots and gather again from the same grouping).
 void launch_cell_table(clsph_state* s);
 uint32_t sort_tiles_for(uint32_t n);
-uint32_t sort_runs_cap_for(uint32_t table_cap);
 // sph.hip
 // With `nu`, also the learned surrogate's node inputs of every particle.
 void launch_density(clsph_state* s, float2* nu = nullptr);
