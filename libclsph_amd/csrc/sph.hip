@@ -168,18 +168,19 @@ struct DensityWalk {
   }
 };
 
-// One lane's walk over its cell's halo staged in LDS: the 4x4x4 half-cells
-// around the particle's cell (side 2h), half-cell q = x + 4y + 16z at
-// cand[off[q], off[q + 1]) in sorted order, each entry (x, y, z, sorted
-// index). The particle sits at local coordinates 1 + (hc & 1), so each row
-// (dy, dz) of its 3x3x3 block is one contiguous range. A row is skipped when
+// One lane's walk over its unit's halo staged in LDS: the half-cells of the
+// unit (a cell, side 4, or a quad of 2x2 cells, side 6) with one half-cell
+// around them, half-cell q = x + side y + side^2 z at cand[off[q], off[q + 1])
+// in sorted order, each entry (x, y, z, sorted index). Each row (dy, dz) of
+// the particle's 3x3x3 block is one contiguous range. A row is skipped when
 // its nearest face is out of reach, and its x-range keeps the half-cells on
 // either side only when they are in reach. Candidates are visited in z, y, x
 // order, four loaded at a time.
 __device__ inline void density_walk_halo(DensityWalk& w, uint32_t i, float4 xi,
-                                         const uint32_t hc[3], const float fr[3],
+                                         const uint32_t hc[3], const float fr[3], uint32_t side,
                                          const float4* cand, const uint32_t* off, float h2) {
-  const uint32_t lx = 1u + (hc[0] & 1u), ly = 1u + (hc[1] & 1u), lz = 1u + (hc[2] & 1u);
+  const uint32_t lx = 1u + (hc[0] & (side - 3u)), ly = 1u + (hc[1] & (side - 3u)),
+                 lz = 1u + (hc[2] & 1u);
   const float lo_x = fr[0] * fr[0], hi_x = (1.f - fr[0]) * (1.f - fr[0]);
   for (int dz = -1; dz <= 1; ++dz) {
     const float az = dz < 0 ? fr[2] : (dz > 0 ? 1.f - fr[2] : 0.f);
@@ -187,7 +188,7 @@ __device__ inline void density_walk_halo(DensityWalk& w, uint32_t i, float4 xi,
       const float ay = dy < 0 ? fr[1] : (dy > 0 ? 1.f - fr[1] : 0.f);
       const float ryz = az * az + ay * ay;
       if (ryz >= kReach2) continue;
-      const uint32_t row = 4u * (ly + (uint32_t)dy) + 16u * (lz + (uint32_t)dz);
+      const uint32_t row = side * (ly + (uint32_t)dy + side * (lz + (uint32_t)dz));
       const uint32_t xa = lo_x + ryz < kReach2 ? lx - 1u : lx;
       const uint32_t xb = hi_x + ryz < kReach2 ? lx + 1u : lx;
       // byte offsets into cand: the group at a holds entry u inside the
@@ -386,7 +387,7 @@ __device__ inline void density_walk_lanes(LaneWalk<L>& w, bool live, uint32_t i,
 // the ordered sum: 12 us at 4,096 particles, where one lane's walk took 66.
 constexpr int kLanesBlock = 256;
 constexpr uint32_t kLanes16Max = 40960;   // particles up to which 16 lanes take one
-constexpr uint32_t kLanes4Max = 147456;   // and up to which 4 lanes do
+constexpr uint32_t kLanes4Max = 180224;   // and up to which 4 lanes do
 template <int L>
 __global__ __launch_bounds__(kLanesBlock) void k_density_lanes(
     const float4* __restrict__ pos, const float4* __restrict__ vel,
@@ -426,22 +427,27 @@ __device__ inline uint32_t compact10(uint32_t v) {
   return v;
 }
 
-// Halo staging of the density kernel, per work-group of WAVES waves: up to
-// kHalos cells (their 4x4x4 half-cell halos) and kCap candidates (x, y, z,
-// index: 16 B each). A bulk cell holds about 64 particles, so the
-// work-group's particles span about WAVES + 1 cells of about 512 halo
-// candidates each. Up to 4 waves, 768 candidates per wave (three 4-wave
-// work-groups per CU); at 8 waves, 12 cells and 4860 candidates keep a
-// work-group within 80 KB, so that two fit per CU.
+// Halo staging of the density kernel, per work-group of WAVES waves: the
+// half-cells around a unit of its particles' cells, kCap candidates (x, y, z,
+// index: 16 B each) in all. A unit is a quad of 2x2 cells in x and y (one run
+// of the Morton order; 6x6x4 half-cells, about 1,152 candidates at rest for
+// 256 particles) where all the work-group's quads fit, otherwise a cell
+// (4x4x4, 512 for 64): quads stage a quarter fewer candidates for the same
+// particles, but when dense the first ones that fit hold fewer of them. At 8
+// waves 4,820 candidates keep a work-group within 80 KB, so that two fit per
+// CU; below, 768 per wave.
+constexpr uint32_t kQuadBox = 144, kCellBox = 64;  // half-cells of a halo
 template <int WAVES>
 struct DensityHalos {
-  static constexpr uint32_t kHalos = WAVES < 8 ? 2u * WAVES : 12u;
-  static constexpr uint32_t kCap = WAVES < 8 ? 768u * WAVES - 4u : 4860u;
+  static constexpr uint32_t kQuads = WAVES < 8 ? (WAVES < 4 ? 1u : 3u) : 6u;  // staged at most
+  static constexpr uint32_t kEntries = kQuads * kQuadBox;
+  static constexpr uint32_t kCells = kEntries / kCellBox;
+  static constexpr uint32_t kCap = WAVES < 8 ? 768u * WAVES - 4u : 4820u;
   float4 cand[kCap + 4];               // + the padding of a group of four
-  uint32_t off[kHalos * 64u + 1u];     // halo h, half-cell q: off[64 h + q]
-  uint32_t cell[kHalos];               // first key of each cell (a multiple of 8)
+  uint32_t off[kEntries + 1u];         // halo by halo, half-cell by half-cell
+  uint32_t unit[kCells];               // the units' Morton codes
   uint32_t wave_sum[WAVES];
-  uint32_t wave_cells[WAVES];
+  uint32_t wave_units[WAVES];
 };
 // Lanes per particle outside the staged halos, and what their walks keep in
 // the candidates' bytes (two 80 KB work-groups per CU leave no others).
@@ -455,14 +461,16 @@ struct DensityRest {
 // Density and pressure (sph.cl:9-40, forces.cl:15-43) of the particles
 // [first, first + 64 WAVES) of one scene, with each particle's neighbour
 // list (self excluded) in visiting order into nbr[q * n + i]. The work-group
-// first stages, for each distinct cell (side 2h) its particles fall in, the
-// cell's 4x4x4 half-cell halo in LDS (coalesced runs of the sorted
-// positions); particles then walk their 3x3x3 half-cells there, one to a
-// lane. Those of cells beyond the staging capacity, and every particle when
+// first stages the halos of the units its particles fall in (DensityHalos) in
+// LDS (coalesced runs of the sorted positions); particles then walk their
+// 3x3x3 half-cells there, one to a lane. Those of units beyond the staging
+// capacity, and every particle when
 // the table is unusable, are then walked from HBM by four lanes each, with
 // the same visiting order: a lane's walk of HBM by itself took 30-50 us, in
-// some work-group of every launch (with four lanes 262,144 particles take 70
-// instead of 80 us, 1,048,576 after 1,000 substeps 211 instead of 223).
+// some work-group of every launch. With cells only, whose halos overlap more,
+// 207,000 particles took 65 us instead of 41 after 20 substeps, 1,048,576 209,
+// 149 and 219 instead of 198, 147 and 203 after 20, 200 and 1,000, 2,097,152
+// 389, 339 and 446 instead of 376, 325 and 398.
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict__ pos,
                                                         const float4* __restrict__ vel,
@@ -478,7 +486,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
                                                         uint32_t* __restrict__ nbr_count,
                                                         float2* __restrict__ nu, uint32_t n) {
   using Halos = DensityHalos<WAVES>;
-  static_assert(Halos::kHalos <= 2u * WAVES, "at most two (halo, half-cell) entries per thread");
+  static_assert(Halos::kEntries < (WAVES == 1 ? 192u : 128u * WAVES), "kPer entries per thread");
   __shared__ Halos sh;
   // runs of 16 work-groups per XCD: neighbouring halos share an L2
   const BlockDesc b = blocks[xcd_block<16>(blockIdx.x, gridDim.x)];
@@ -490,100 +498,120 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
   const float h = dp->p.h, h2 = h * h;
   const uint32_t F = usable_key_end(dp, bp);
 
-  // Cells of the work-group's particles, in order: a particle starts one
-  // when it is the first particle or its cell differs from its predecessor's.
-  const uint32_t key = live ? keys[i] : 0u;
-  const uint32_t prev = (live && t > 0) ? keys[i - 1] : 0u;
-  const bool starts = live && (t == 0 || (key >> 3) != (prev >> 3));
-  const uint64_t mask = __ballot(starts);
-  if (lane == 0) sh.wave_cells[wv] = (uint32_t)__popcll(mask);
-  __syncthreads();
-  uint32_t before = 0, cells = 0;
-  for (int q = 0; q < WAVES; ++q) {
-    const uint32_t c = sh.wave_cells[q];
-    before += (uint32_t)q < wv ? c : 0u;
-    cells += c;
-  }
-  // index of the particle's cell among the work-group's cells
-  const uint32_t ci = before + (uint32_t)__popcll(mask & (~0ull >> (63u - lane))) - 1u;
-  if (starts && ci < Halos::kHalos) sh.cell[ci] = key & ~7u;
-  const uint32_t halos = F == 0u ? 0u : (cells < Halos::kHalos ? cells : Halos::kHalos);
-  __syncthreads();
-
-  // Halo half-cell runs: thread t takes the entries 2t and 2t + 1 of the
-  // (halo, half-cell) list.
-  uint32_t rs[2] = {0u, 0u}, rc[2] = {0u, 0u};
+  // Units of the work-group's particles, in order: a particle starts one
+  // when it is the first particle or its unit differs from its predecessor's.
+  const uint32_t key = live ? keys[i] - dp->key_base : 0u;
+  const uint32_t prev = (live && t > 0) ? keys[i - 1] - dp->key_base : 0u;
+  uint32_t units, ui, side = 6u;
+  auto find_units = [&](uint32_t bits) {
+    const bool starts = live && (t == 0 || (key >> bits) != (prev >> bits));
+    const uint64_t mask = __ballot(starts);
+    if (lane == 0) sh.wave_units[wv] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    uint32_t before = 0;
+    units = 0;
+    for (int q = 0; q < WAVES; ++q) {
+      const uint32_t c = sh.wave_units[q];
+      before += (uint32_t)q < wv ? c : 0u;
+      units += c;
+    }
+    // index of the particle's unit among the work-group's units
+    ui = before + (uint32_t)__popcll(mask & (~0ull >> (63u - lane))) - 1u;
+    if (starts && ui < Halos::kCells) sh.unit[ui] = key >> bits;
+  };
+  find_units(5u);
+  constexpr int kPer = WAVES == 1 ? 3 : 2;  // half-cells per thread
+  uint32_t rs[kPer], rc[kPer], ex[kPer], staged, box;
+  for (;;) {
+    const uint32_t most = F == 0u ? 0u : (side == 6u ? Halos::kQuads : Halos::kCells);
+    const uint32_t halos = units < most ? units : most;
+    box = side == 6u ? kQuadBox : kCellBox;
+    __syncthreads();
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const uint32_t q = 2u * t + (uint32_t)u, hh = q >> 6, l = q & 63u;
-    if (hh < halos) {
-      const uint32_t c8 = sh.cell[hh];
-      const uint32_t cl = (c8 - dp->key_base) >> 3;
-      const uint32_t hx = 2u * compact10(cl) - 1u + (l & 3u);
-      const uint32_t hy = 2u * compact10(cl >> 1) - 1u + ((l >> 2) & 3u);
-      const uint32_t hz = 2u * compact10(cl >> 2) - 1u + (l >> 4);
-      if (hx < 2048u && hy < 2048u && hz < 2048u) {
-        const uint32_t f = dp->key_base + half_key(hx, hy, hz);
-        if (f < F) {
-          uint32_t e = table[f + 1u];
-          e = e < n ? e : n;
-          uint32_t s = table[f];
-          s = s < e ? s : e;
-          rs[u] = s;
-          rc[u] = e - s;
+    for (int u = 0; u < kPer; ++u) {
+      const uint32_t q = (uint32_t)kPer * t + (uint32_t)u;
+      rs[u] = rc[u] = 0u;
+      const uint32_t hh = side == 6u ? q / kQuadBox : q / kCellBox;
+      if (hh < halos) {
+        const uint32_t un = sh.unit[hh], l = q - hh * box;
+        const uint32_t r = side == 6u ? l / 6u : l >> 2, x = l - r * side;
+        const uint32_t z = side == 6u ? r / 6u : r >> 2, y = r - z * side;
+        // a cell's Morton code is un; a quad's (2x2 cells in x and y) lacks
+        // their last bits
+        const uint32_t hx = side == 6u ? 4u * compact10(un >> 1) : 2u * compact10(un);
+        const uint32_t hy = side == 6u ? 4u * compact10(un >> 2) : 2u * compact10(un >> 1);
+        const uint32_t hz = 2u * compact10(side == 6u ? un : un >> 2);
+        const uint32_t gx = hx - 1u + x, gy = hy - 1u + y, gz = hz - 1u + z;
+        if (gx < 2048u && gy < 2048u && gz < 2048u) {
+          const uint32_t f = dp->key_base + half_key(gx, gy, gz);
+          if (f < F) {
+            uint32_t e = table[f + 1u];
+            e = e < n ? e : n;
+            uint32_t s = table[f];
+            s = s < e ? s : e;
+            rs[u] = s;
+            rc[u] = e - s;
+          }
         }
       }
     }
-  }
-  // exclusive scan of the run lengths over the work-group
-  const uint32_t mine = rc[0] + rc[1];
-  uint32_t incl = mine;
+    // exclusive scan of the run lengths over the work-group
+    uint32_t mine = 0;
 #pragma unroll
-  for (uint32_t o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += y;
-  }
-  if (lane == 63) sh.wave_sum[wv] = incl;
-  __syncthreads();
-  uint32_t base = 0;
-  for (int q = 0; q < WAVES; ++q) base += (uint32_t)q < wv ? sh.wave_sum[q] : 0u;
-  const uint32_t ex = base + incl - mine;
-  if (2u * t < Halos::kHalos * 64u) {  // threads past the last halo hold no runs
-    sh.off[2u * t] = ex;
-    sh.off[2u * t + 1u] = ex + rc[0];
-  }
-  if (t == WAVES * 64 - 1) sh.off[Halos::kHalos * 64u] = ex + mine;
-  __syncthreads();
-  // halos staged: the leading ones whose candidates fit
-  uint32_t staged = 0;
-  while (staged < halos && sh.off[64u * (staged + 1u)] <= Halos::kCap) ++staged;
+    for (int u = 0; u < kPer; ++u) mine += rc[u];
+    uint32_t incl = mine;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const uint32_t q = 2u * t + (uint32_t)u;
-    if ((q >> 6) < staged) {
-      const uint32_t o = u ? ex + rc[0] : ex;
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) sh.wave_sum[wv] = incl;
+    __syncthreads();
+    uint32_t base = 0;
+    for (int q = 0; q < WAVES; ++q) base += (uint32_t)q < wv ? sh.wave_sum[q] : 0u;
+    uint32_t at = base + incl - mine;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const uint32_t q = (uint32_t)kPer * t + (uint32_t)u;
+      if (q <= Halos::kEntries) sh.off[q] = at;
+      ex[u] = at;
+      at += rc[u];
+    }
+    __syncthreads();
+    // halos staged: the leading ones whose candidates fit
+    staged = 0;
+    while (staged < halos && sh.off[box * (staged + 1u)] <= Halos::kCap) ++staged;
+    if (staged == units || side == 4u || F == 0u) break;
+    // not all quads fit: cell by cell
+    side = 4u;
+    find_units(3u);
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint32_t q = (uint32_t)kPer * t + (uint32_t)u;
+    if ((side == 6u ? q / kQuadBox : q / kCellBox) < staged) {
       for (uint32_t k = 0; k < rc[u]; ++k) {
         const uint32_t j = rs[u] + k;
         const float4 p = pos[j];
-        sh.cand[o + k] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
+        sh.cand[ex[u] + k] = make_float4(p.x, p.y, p.z, __uint_as_float(j));
       }
     }
   }
   __syncthreads();
 
-  if (live && ci < staged) {
+  if (live && ui < staged) {
     const float4 xi = pos[i];
     uint32_t hc[3];
     float fr[3];
     half_cell_frac(xi, dp, hc, fr);
     DensityWalk w(nbr, i, n, h2);
-    density_walk_halo(w, i, xi, hc, fr, sh.cand, sh.off + 64u * ci, h2);
+    density_walk_halo(w, i, xi, hc, fr, side, sh.cand, sh.off + box * ui, h2);
     w.finish();
     density_store(dp, i, xi, w.acc, w.cnt, vel, rho, prs, fab, nbr_count, nu);
   }
-  if (staged == cells) return;  // uniform: every cell was staged
+  if (staged == units) return;  // uniform: every unit was staged
   // the rest, in the order of their threads
-  const bool left = live && ci >= staged;
+  const bool left = live && ui >= staged;
   const uint64_t lm = __ballot(left);
   if (lane == 0) sh.wave_sum[wv] = (uint32_t)__popcll(lm);
   __syncthreads();  // also: the staged walks are done with cand
@@ -897,7 +925,11 @@ void launch_density(clsph_state* s, float2* nu) {
   // at least a wave's walk, 30-50 us; below that many particles the chip has
   // lanes to spare. Stage time on evolved dam breaks, 1 / 4 / 16 lanes:
   // 16,384 particles 86 / 25 / 15 us, 50,021 49 / 31 / 30, 65,536
-  // 48 / 34 / 36, 131,071 62 / 49 / 58, 180,000 47 / 58 / 77.
+  // 48 / 34 / 36, 131,071 62 / 49 / 58. 1 / 4 lanes after 20, 200, 1,000 and
+  // 1,800 substeps: 160,000 39, 64, 59, 85 / 48, 47, 51, 62 us, 180,225 73, 41,
+  // 62, 98 / 53, 50, 57, 72, 207,000 41, 42, 63, 145 / 62, 58, 59, 77, 262,144
+  // 42, 58, 64, 135 / 73, 67, 71, 94, 524,288 77, 85, 124, 165 / 133, 122, 129,
+  // 180 (settled fluid is two to three times as dense).
   if (s->n <= kLanes4Max) {
     // 64-particle entries of the work list, whatever the stage's block size
     auto lanes = [&](auto kernel, uint32_t share) {
