@@ -107,8 +107,8 @@ int clsph_density_pressure(clsph_state* st);
 int clsph_forces(clsph_state* st);
 /* advection_collision: sph.cl:64-112, launched at sph_simulation.cpp:330-337 */
 int clsph_advect_collide(clsph_state* st);
-/* `nsteps` whole substeps (all stages above), replayed from one captured
- * HIP graph; replaces simulate_single_frame's body. */
+/* `nsteps` whole substeps (all stages above), replayed from captured HIP
+ * graphs; replaces simulate_single_frame's body. */
 int clsph_step(clsph_state* st, uint32_t nsteps);
 
 /* ---- batches: many independent scenes advanced together. No counterpart

@@ -18,6 +18,11 @@ namespace clsph {
 // Records per page-locked transfer buffer (1 MB: a buffer's copy by the host
 // overlaps the next one's transfer, and stays in its cache).
 constexpr uint32_t kTransferRecords = 13056;
+// Substeps per captured graph, and substeps after which a state captures those
+// of more than one.
+constexpr int kNumGraphs = 3;
+constexpr uint32_t kGraphSteps[kNumGraphs] = {1, 4, 16};
+constexpr uint32_t kGraphAfter = 64;
 struct TransferStatus {
   uint32_t err;        // kErr* bits of every scene and of the batch
   uint32_t bad_slots;  // the canonical slots are not a permutation
@@ -135,8 +140,10 @@ struct clsph_state {
   clsph::BatchParams* bp = nullptr;  // device batch parameters
   std::vector<clsph::DevParams> host_dps;
 
-  hipGraphExec_t graph = nullptr;  // one captured substep
+  // Captured substeps: graphs[k] holds clsph::kGraphSteps[k] of them.
+  hipGraphExec_t graphs[clsph::kNumGraphs] = {};
   bool graph_dirty = true;
+  uint32_t graph_steps = 0;  // substeps replayed from them, up to kGraphAfter
   // One captured learned macro step (clsph_learned_step), for the network
   // with serial lgraph_serial at lgraph_n particles; parameters are baked in.
   hipGraphExec_t lgraph = nullptr;
