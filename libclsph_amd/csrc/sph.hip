@@ -53,13 +53,13 @@ __device__ inline uint32_t usable_key_end(const DevParams* __restrict__ dp,
   return (bp->err & (kErrTableCap | kErrFineKey)) ? 0u : dp->key_end;
 }
 
-// Visits the particles of the 3x3x3 half-cells around hc in z, y, x order.
-// Along x the three cells form two Morton-contiguous runs: the pair starting
-// at the even coordinate, and the remaining one.
+// Visits the runs [s, e) of particles of the 3x3x3 half-cells around hc in
+// z, y, x order. Along x the three cells form two Morton-contiguous runs: the
+// pair starting at the even coordinate, and the remaining one.
 template <typename F>
-__device__ inline void for_each_candidate(const uint32_t hc[3], uint32_t base,
-                                          const uint32_t* __restrict__ ht, uint32_t Fc,
-                                          uint32_t n, F&& fn) {
+__device__ inline void for_each_run(const uint32_t hc[3], uint32_t base,
+                                    const uint32_t* __restrict__ ht, uint32_t Fc, uint32_t n,
+                                    F&& fn) {
   const uint32_t x0 = hc[0] - 1u;
   const bool even = (x0 & 1u) == 0u;
   for (uint32_t dz = 0; dz < 3; ++dz)
@@ -69,9 +69,9 @@ __device__ inline void for_each_candidate(const uint32_t hc[3], uint32_t base,
       uint32_t b = base + half_key(even ? x0 + 2u : x0 + 1u, y, z);
       uint32_t s, e;
       half_range(a, even ? 2u : 1u, ht, Fc, n, s, e);
-      for (uint32_t j = s; j < e; ++j) fn(j);
+      fn(s, e);
       half_range(b, even ? 1u : 2u, ht, Fc, n, s, e);
-      for (uint32_t j = s; j < e; ++j) fn(j);
+      fn(s, e);
     }
 }
 
@@ -732,20 +732,42 @@ __device__ inline ForceSums force_start(const ForceConsts& k, float4 bi) {
   return fs;
 }
 
-// More neighbours than the list holds: walks the half-cells again.
+// The neighbours past those the list holds, of which `last` is the final one:
+// walks the half-cells again from there, in density's order and with its test,
+// W candidates' loads in flight (one where registers are short).
+// (Walking them all from the start, one candidate after another, took the
+// stage from 35 to 123 us once some lists overflowed, 131,071 particles.)
+template <uint32_t W>
 __device__ inline void force_walk(ForceSums& fs, const ForceConsts& k, uint32_t i, float4 ai,
-                                  float4 bi, const float4* __restrict__ fab,
+                                  float4 bi, uint32_t last, const float4* __restrict__ fab,
                                   const uint32_t* __restrict__ table,
                                   const DevParams* __restrict__ dp, uint32_t F, uint32_t n) {
   uint32_t hc[3];
   half_cell(ai, dp, hc);
-  const float h2 = k.h2;
-  for_each_candidate(hc, dp->key_base, table, F, n, [&](uint32_t j) {
-    float4 aj = fab[2u * j];
-    float d2 = length2(ai.x - aj.x, ai.y - aj.y, ai.z - aj.z);
-    if (!(d2 < h2) || j == i) return;
-    force_pair(fs, k, ai, bi, aj, fab[2u * j + 1u]);
+  bool past = false;
+  for_each_run(hc, dp->key_base, table, F, n, [&](uint32_t s, uint32_t e) {
+    if (!past) {
+      if (last < s || last >= e) return;
+      past = true;
+      s = last + 1u;
+    }
+    for (uint32_t j0 = s; j0 < e; j0 += W) {
+      float4 aj[W];
+#pragma unroll
+      for (uint32_t u = 0; u < W; ++u) aj[u] = fab[2u * (j0 + u < e ? j0 + u : j0)];
+#pragma unroll
+      for (uint32_t u = 0; u < W; ++u) {
+        const uint32_t j = j0 + u;
+        if (j < e && dist2(ai, aj[u]) < k.h2 && j != i)
+          force_pair(fs, k, ai, bi, aj[u], fab[2u * j + 1u]);
+      }
+    }
   });
+}
+
+// The last entry of particle i's full list.
+__device__ inline uint32_t last_listed(const uint4* __restrict__ nbr, uint32_t i, uint32_t n) {
+  return nbr[(size_t)(kMaxNeighbours / 4u - 1u) * n + i].w;
 }
 
 // Acceleration from the sums (forces.cl:95-111 and sph.cl:53-58).
@@ -799,7 +821,7 @@ __global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
   const ForceConsts k = force_consts(dp);
   const float4 ai = fab[2u * i], bi = fab[2u * i + 1u];
   const uint32_t all = nbr_count[i];
-  const uint32_t cnt = live && all <= kMaxNeighbours ? all : 0u;
+  const uint32_t cnt = live ? (all < kMaxNeighbours ? all : kMaxNeighbours) : 0u;
   float* w = terms[part];
   auto index = [&](uint32_t q) {  // past the end: the particle itself
     return q < cnt ? reinterpret_cast<const uint32_t*>(nbr)[4u * ((size_t)(q >> 2) * n + i) + (q & 3u)]
@@ -838,15 +860,13 @@ __global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
   wave_lds_fence();
   if (!live || sub != 0u) return;
   ForceSums fs;
-  if (all <= kMaxNeighbours) {
-    fs.pt = make_float3(w[0], w[1], w[2]);
-    fs.vt = make_float3(w[3], w[4], w[5]);
-    fs.nrm = make_float3(w[6], w[7], w[8]);
-    fs.lap = w[9];
-  } else {
-    fs = force_start(k, bi);
-    force_walk(fs, k, i, ai, bi, fab, table, dp, usable_key_end(dp, bp), n);
-  }
+  fs.pt = make_float3(w[0], w[1], w[2]);
+  fs.vt = make_float3(w[3], w[4], w[5]);
+  fs.nrm = make_float3(w[6], w[7], w[8]);
+  fs.lap = w[9];
+  if (all > kMaxNeighbours)
+    force_walk<1>(fs, k, i, ai, bi, last_listed(nbr, i, n), fab, table, dp,
+                  usable_key_end(dp, bp), n);
   acc_out[i] = force_close(fs, rho[i], dp);
 }
 
@@ -874,48 +894,46 @@ __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__
   float4 ai = fab[2u * i], bi = fab[2u * i + 1u];
   float rho_i = rho[i];
   ForceSums fs = force_start(k, bi);
-  uint32_t cnt = nbr_count[i];
-  if (cnt <= kMaxNeighbours) {
-    // groups of four neighbours, software-pipelined: while a group's pair
-    // terms are summed, the next group's records and the indices of the one
-    // after it are in flight
-    const uint32_t groups = cnt >> 2;
-    auto gather = [&](uint4 js, float4 ra[4], float4 rb[4]) {
-      const uint32_t jj[4] = {js.x, js.y, js.z, js.w};
+  const uint32_t all = nbr_count[i], cnt = all < kMaxNeighbours ? all : kMaxNeighbours;
+  // groups of four neighbours, software-pipelined: while a group's pair
+  // terms are summed, the next group's records and the indices of the one
+  // after it are in flight
+  const uint32_t groups = cnt >> 2;
+  auto gather = [&](uint4 js, float4 ra[4], float4 rb[4]) {
+    const uint32_t jj[4] = {js.x, js.y, js.z, js.w};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        ra[u] = fab[2u * jj[u]];
-        rb[u] = fab[2u * jj[u] + 1u];
-      }
-    };
-    float4 ca[4], cb[4];
-    uint4 jn = make_uint4(0u, 0u, 0u, 0u);
-    if (groups) {
-      gather(nbr[i], ca, cb);
-      if (groups > 1) jn = nbr[(size_t)n + i];
+    for (int u = 0; u < 4; ++u) {
+      ra[u] = fab[2u * jj[u]];
+      rb[u] = fab[2u * jj[u] + 1u];
     }
-    for (uint32_t gq = 0; gq < groups; ++gq) {
-      float4 na[4], nb[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) na[u] = ca[u], nb[u] = cb[u];
-      if (gq + 1 < groups) gather(jn, na, nb);
-      if (gq + 2 < groups) jn = nbr[(size_t)(gq + 2) * n + i];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) force_pair(fs, k, ai, bi, ca[u], cb[u]);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) ca[u] = na[u], cb[u] = nb[u];
-    }
-    const uint32_t q = groups << 2;
-    if (q < cnt) {
-      uint4 js = nbr[(size_t)(q >> 2) * n + i];
-      uint32_t r = cnt - q;
-      force_pair(fs, k, ai, bi, fab[2u * js.x], fab[2u * js.x + 1u]);
-      if (r > 1) force_pair(fs, k, ai, bi, fab[2u * js.y], fab[2u * js.y + 1u]);
-      if (r > 2) force_pair(fs, k, ai, bi, fab[2u * js.z], fab[2u * js.z + 1u]);
-    }
-  } else {
-    force_walk(fs, k, i, ai, bi, fab, table, dp, F, n);
+  };
+  float4 ca[4], cb[4];
+  uint4 jn = make_uint4(0u, 0u, 0u, 0u);
+  if (groups) {
+    gather(nbr[i], ca, cb);
+    if (groups > 1) jn = nbr[(size_t)n + i];
   }
+  for (uint32_t gq = 0; gq < groups; ++gq) {
+    float4 na[4], nb[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) na[u] = ca[u], nb[u] = cb[u];
+    if (gq + 1 < groups) gather(jn, na, nb);
+    if (gq + 2 < groups) jn = nbr[(size_t)(gq + 2) * n + i];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) force_pair(fs, k, ai, bi, ca[u], cb[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) ca[u] = na[u], cb[u] = nb[u];
+  }
+  const uint32_t q = groups << 2;
+  if (q < cnt) {
+    uint4 js = nbr[(size_t)(q >> 2) * n + i];
+    uint32_t r = cnt - q;
+    force_pair(fs, k, ai, bi, fab[2u * js.x], fab[2u * js.x + 1u]);
+    if (r > 1) force_pair(fs, k, ai, bi, fab[2u * js.y], fab[2u * js.y + 1u]);
+    if (r > 2) force_pair(fs, k, ai, bi, fab[2u * js.z], fab[2u * js.z + 1u]);
+  }
+  if (all > kMaxNeighbours)
+    force_walk<4>(fs, k, i, ai, bi, last_listed(nbr, i, n), fab, table, dp, F, n);
   acc_out[i] = force_close(fs, rho_i, dp);
 }
 
