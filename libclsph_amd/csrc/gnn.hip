@@ -202,7 +202,11 @@ __device__ __attribute__((always_inline)) inline void wave_fence() {
 // [+ PA_i + PB_j]) W2 + b2) / C) over particle i's neighbour list (the density
 // kernel's, at most kMaxEdges) without storing per-edge values.
 //
-// A wave takes up to 16 consecutive particles at a time (a run).
+// A wave takes up to 16 particles at a time (a run), every R-th of R runs, so
+// that particles with many neighbours, which lie together, are shared by all
+// waves (an evaluation of 131,072 particles in a macro step 902 us at 29
+// neighbours on average and 1,367 at 34, with consecutive particles; now 892
+// and 1,006. 14,000 at 37: 304 and 265).
 // The run's edges, each particle's padded to quads, are cut into four equal
 // streams, one per lane group g = l / 16, whichever particles that splits; a
 // tile is the next quad of each stream. (A tile of 16 edges per particle would
@@ -304,16 +308,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   for (int ob = 0; ob < 8; ++ob) bias2[ob] = b2[8 * c + ob];
   __syncthreads();
 
-  // this wave's particles; consecutive shares on the same XCD's L2
-  const uint32_t blocks = gridDim.x;
+  // this wave's runs; consecutive ones on the same XCD's L2
+  const uint32_t blocks = gridDim.x, waves = blocks * 4;
   const uint32_t b = blocks % 8 ? blockIdx.x : (blockIdx.x % 8) * (blocks / 8) + blockIdx.x / 8;
   const uint32_t w = b * 4 + wave;
-  const uint32_t last = (uint32_t)((uint64_t)n * (w + 1) / (blocks * 4));
+  const uint32_t rounds = (n + kRunMax * waves - 1) / (kRunMax * waves);
+  const uint32_t stride = waves * rounds;
   const float inv_h = 1.f / h;
   u32x4* rec = recs[wave];
   uint32_t limit = kRunMax, redo_end = 0;
-  for (uint32_t i0 = (uint32_t)((uint64_t)n * w / (blocks * 4)); i0 < last;) {
-    const uint32_t parts = min(last - i0, limit);
+  for (uint32_t q = 0, o0 = 0; q < rounds;) {
+    // run q of the wave: `size` particles from `first`, every stride-th
+    const uint32_t first = w + waves * q, size = first < n ? (n - 1 - first) / stride + 1 : 0u;
+    if (o0 >= size) {
+      ++q, o0 = 0, limit = kRunMax, redo_end = 0;
+      continue;
+    }
+    const uint32_t parts = min(size - o0, limit), i0 = first + o0 * stride;
     if (ROUND2) {
       bool odd = false;  // PA not finite
       if (g >= 2)
@@ -322,7 +333,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
           uint16_t v[8];
           for (int t = 0; t < 8; ++t) {
             const uint32_t p = 8 * (g - 2) + t;
-            const uint16_t pa = PA[(size_t)(i0 + min(p, parts - 1)) * kWidth + col];
+            const uint16_t pa = PA[(size_t)(i0 + min(p, parts - 1) * stride) * kWidth + col];
             v[t] = p < parts ? pa : (uint16_t)0;
             odd |= (v[t] & 0x7F80u) == 0x7F80u;
           }
@@ -330,12 +341,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             w1[ob][t] = (uint32_t)v[2 * t] | ((uint32_t)v[2 * t + 1] << 16);
         }
       if (parts > 1 && __any(odd)) {
-        limit = 1, redo_end = i0 + parts;
+        limit = 1, redo_end = o0 + parts;
         continue;
       }
     }
-    // lane p: degree and first quad of particle i0 + p
-    const uint32_t deg = (uint32_t)lane < parts ? min(count[i0 + lane], kMaxEdges) : 0u;
+    // lane p: degree and first quad of particle p of the run
+    const uint32_t deg = (uint32_t)lane < parts ? min(count[i0 + lane * stride], kMaxEdges) : 0u;
     uint32_t start = (deg + 3) / 4;
     for (int o = 1; o < kRunMax; o <<= 1) {
       const uint32_t y = __shfl_up(start, o, 64);
@@ -354,7 +365,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     };
     for (uint64_t none = __ballot((uint32_t)lane < parts && deg == 0); none; none &= none - 1)
       if (lane < 16)
-        *(u32x4*)(S + (size_t)(i0 + __builtin_ctzll(none)) * kWidth + 8 * c) =
+        *(u32x4*)(S + (size_t)(i0 + __builtin_ctzll(none) * stride) * kWidth + 8 * c) =
             u32x4{0u, 0u, 0u, 0u};
     const uint32_t tiles = (total + 3) / 4;  // quads per stream
     float acc[8], lead[8];
@@ -367,7 +378,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     auto store = [&](const float* sum) {
       float v[8];
       for (int ob = 0; ob < 8; ++ob) v[ob] = sum[ob] * (1.f / kAggC);
-      *(u32x4*)(S + (size_t)(i0 + slot) * kWidth + 8 * c) = pack8(v);
+      *(u32x4*)(S + (size_t)(i0 + slot * stride) * kWidth + 8 * c) = pack8(v);
     };
     for (uint32_t t0 = 0; t0 < tiles; t0 += 4) {
       // the inputs of four tiles' edges
@@ -379,7 +390,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         const uint32_t d = (uint32_t)__shfl(deg, p, 64);
         const bool on = t < tiles && quad < total;
         const bool valid = on && 4 * k + r < d;
-        const uint32_t i = i0 + p;
+        const uint32_t i = i0 + p * stride;
         uint32_t j = i0;
         u32x4 lo = {0u, 0u, 0u, 0u}, hi = {0u, 0u, 0u, 0u};
         if (valid) {
@@ -496,8 +507,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
       }
       if (open && !pending) store(acc);
     }
-    i0 += parts;
-    if (i0 >= redo_end) limit = kRunMax;
+    o0 += parts;
+    if (o0 >= redo_end) limit = kRunMax;
   }
 }
 
