@@ -993,11 +993,18 @@ __global__ void k_write_acc(const float* __restrict__ out, uint32_t n, float gx,
 }
 
 // ---------------------------------------------------------------------------
+// Work-groups of a grid-stride kernel over `count` items.
 inline dim3 grid_for(size_t count, size_t per_block = 256) {
   size_t b = (count + per_block - 1) / per_block;
   if (b > 65536) b = 65536;
   if (b == 0) b = 1;
   return dim3((uint32_t)b);
+}
+
+// Work-groups of a kernel whose threads take one item each, all of them.
+inline dim3 grid_of_all(size_t count, size_t per_block = 256) {
+  const size_t b = (count + per_block - 1) / per_block;
+  return dim3((uint32_t)(b ? b : 1));
 }
 
 void fill(float* x, size_t count, float v, hipStream_t s) {
@@ -1064,7 +1071,7 @@ static void mlp2(clsph_gnn* m, const uint16_t* u, int kin, int w1, float* pre1, 
 static void node_round1(clsph_gnn* m, hipStream_t s) {
   int n = (int)m->n;
   gemm_cast(s, m->S[0], W(m, E1_W3), m->u1, kIn1, n, P(m, E1_B3), m->degc);
-  hipLaunchKernelGGL(k_tail_u1, grid_for(n), dim3(256), 0, s, m->nu, m->n, m->u1);
+  hipLaunchKernelGGL(k_tail_u1, grid_of_all(n), dim3(256), 0, s, m->nu, m->n, m->u1);
   mlp2(m, m->u1, kIn1, N1_W1, m->p1, m->y1, m->p2, m->y2, s);
   gemm_cast(s, m->y2, W(m, N1_W3), m->Hb, kWidth, n, P(m, N1_B3));
   gemm_cast(s, m->Hb, W(m, E2_WA), m->PA, kWidth, n);
@@ -1075,7 +1082,7 @@ static void node_round1(clsph_gnn* m, hipStream_t s) {
 static void node_round2(clsph_gnn* m, float4* acc, float gx, float gy, float gz, hipStream_t s) {
   int n = (int)m->n;
   gemm_cast(s, m->S[1], W(m, E2_W3), m->u2 + kWidth, kIn2, n, P(m, E2_B3), m->degc);
-  hipLaunchKernelGGL(k_head_u2, grid_for((size_t)n * (kWidth / 8)), dim3(256), 0, s, m->Hb, m->n,
+  hipLaunchKernelGGL(k_head_u2, grid_of_all((size_t)n * (kWidth / 8)), dim3(256), 0, s, m->Hb, m->n,
                      m->u2);
   mlp2(m, m->u2, kIn2, N2_W1, m->q1, m->w1, m->q2, m->w2, s);
   gemm(s, false, false, false, m->w2, kWidth, W(m, N2_W3), kOut, m->out, kOut, n, kOut, kWidth,
@@ -1115,7 +1122,7 @@ void forward_fused(clsph_gnn* m, clsph_state* st, float4* acc, float gx, float g
   if (blocks * 4 > n) blocks = (n + 3) / 4;
   if (blocks == 0) blocks = 1;
   if (ev) (void)hipEventRecord(ev[0], s);
-  hipLaunchKernelGGL(k_node_inputs, grid_for(n), dim3(256), 0, s, st->rho_s, st->prs_s,
+  hipLaunchKernelGGL(k_node_inputs, grid_of_all(n), dim3(256), 0, s, st->rho_s, st->prs_s,
                      st->nbr_count, n, d.p.fluid_density, d.p.K, (float2*)m->nu, m->degc);
   hipLaunchKernelGGL((k_edge_fused<false>), dim3(blocks), dim3(256), 0, s, st->pos_s, st->vel_s,
                      (const float2*)m->nu, (const uint32_t*)st->nbr, st->nbr_count, n, d.p.h, W(m, E1_W1),
