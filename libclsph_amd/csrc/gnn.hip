@@ -1021,7 +1021,7 @@ void launch_graph(clsph_gnn* m, clsph_state* st) {
                      m->scan_part);
   hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanBlock), 0, s, m->scan_part, chunks,
                      m->off + n);
-  hipLaunchKernelGGL(k_scan_add, grid_for(n), dim3(256), 0, s, m->off, m->scan_part, n);
+  hipLaunchKernelGGL(k_scan_add, grid_of_all(n), dim3(256), 0, s, m->off, m->scan_part, n);
 }
 
 void launch_edge_inputs(clsph_gnn* m, clsph_state* st) {
@@ -1031,7 +1031,7 @@ void launch_edge_inputs(clsph_gnn* m, clsph_state* st) {
   hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
                      m->src, m->dst, m->degc);
   uint32_t cnt = e > n ? e : n;
-  hipLaunchKernelGGL(k_edge_inputs, grid_for(cnt), dim3(256), 0, s, st->pos_s, st->vel_s,
+  hipLaunchKernelGGL(k_edge_inputs, grid_of_all(cnt), dim3(256), 0, s, st->pos_s, st->vel_s,
                      st->rho_s, st->prs_s, m->src, m->dst, e, n, d.p.h, d.p.fluid_density,
                      d.p.K, m->E1, m->nu);
 }
@@ -1088,7 +1088,7 @@ static void node_round2(clsph_gnn* m, float4* acc, float gx, float gy, float gz,
   gemm(s, false, false, false, m->w2, kWidth, W(m, N2_W3), kOut, m->out, kOut, n, kOut, kWidth,
        1.f, P(m, N2_B3));
   if (acc)
-    hipLaunchKernelGGL(k_write_acc, grid_for(n), dim3(256), 0, s, m->out, m->n, gx, gy, gz, acc);
+    hipLaunchKernelGGL(k_write_acc, grid_of_all(n), dim3(256), 0, s, m->out, m->n, gx, gy, gz, acc);
 }
 
 void forward(clsph_gnn* m, const DevParams* dp, float4* acc, float gx, float gy, float gz) {
@@ -1209,7 +1209,7 @@ void backward(clsph_gnn* m) {
   size_t nw = (size_t)n * kWidth;
   fill(m->grad, kParamTotal, 0.f, s);
   fill(m->loss, 1, 0.f, s);
-  hipLaunchKernelGGL(k_loss, grid_for(n), dim3(256), 0, s, m->out, m->target, m->n, m->dout,
+  hipLaunchKernelGGL(k_loss, grid_of_all(n), dim3(256), 0, s, m->out, m->target, m->n, m->dout,
                      m->loss);
   // dpb (n x 256 bf16): the first half is mlp3_back's scratch, the second
   // half holds the bf16 gradient fed into it.

@@ -1280,11 +1280,18 @@ __global__ void k_target_mean(const uint32_t* __restrict__ perm, const float* __
 }
 
 // ---------------------------------------------------------------------------
+// Work-groups of a grid-stride kernel over `count` items.
 inline dim3 grid_for(size_t count, size_t per_block = 256) {
   size_t b = (count + per_block - 1) / per_block;
   if (b > 65536) b = 65536;
   if (b == 0) b = 1;
   return dim3((uint32_t)b);
+}
+
+// Work-groups of a kernel whose threads take one item each, all of them.
+inline dim3 grid_of_all(size_t count, size_t per_block = 256) {
+  const size_t b = (count + per_block - 1) / per_block;
+  return dim3((uint32_t)(b ? b : 1));
 }
 
 void fill(float* x, size_t count, float v, hipStream_t s) {
@@ -1301,7 +1308,7 @@ void launch_graph(clsph_nn* m, clsph_state* st) {
                      m->scan_part);
   hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanBlock), 0, s, m->scan_part, chunks,
                      m->off + n);
-  hipLaunchKernelGGL(k_scan_add, grid_for(n), dim3(256), 0, s, m->off, m->scan_part, n);
+  hipLaunchKernelGGL(k_scan_add, grid_of_all(n), dim3(256), 0, s, m->off, m->scan_part, n);
 }
 
 void launch_edge_inputs(clsph_nn* m, clsph_state* st) {
@@ -1310,7 +1317,7 @@ void launch_edge_inputs(clsph_nn* m, clsph_state* st) {
   const DevParams& d = st->host_dps[0];
   hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
                      m->src, m->dst, m->degc);
-  hipLaunchKernelGGL(k_node_inputs, grid_for(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
+  hipLaunchKernelGGL(k_node_inputs, grid_of_all(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
                      d.p.fluid_density, d.p.K, (float2*)m->nu);
   hipLaunchKernelGGL(k_edge_inputs, grid_for(e), dim3(256), 0, s, st->fab,
                      (const float2*)m->nu, m->src, m->dst, e, edge_consts(d), m->E1);
@@ -1342,7 +1349,7 @@ void forward_fused(clsph_nn* m, clsph_state* st, float4* acc, float* out, bool o
   const DevParams& d = st->host_dps[0];
   if (ev) (void)hipEventRecord(ev[0], s);
   if (!nu_ready)
-    hipLaunchKernelGGL(k_node_inputs, grid_for(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
+    hipLaunchKernelGGL(k_node_inputs, grid_of_all(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
                        d.p.fluid_density, d.p.K, (float2*)m->nu);
   // persistent grid: the work-groups that fit on the device at once (the
   // kernel's registers and LDS allow two per compute unit) stage the weights
@@ -1375,7 +1382,7 @@ void backward(clsph_nn* m) {
   int n = (int)m->n, e = (int)m->e;
   fill(m->grad, kParamTotal, 0.f, s);
   fill(m->loss, 1, 0.f, s);
-  hipLaunchKernelGGL(k_loss, grid_for(n), dim3(256), 0, s, m->out, m->target, m->n, m->dout,
+  hipLaunchKernelGGL(k_loss, grid_of_all(n), dim3(256), 0, s, m->out, m->target, m->n, m->dout,
                      m->loss);
   hipLaunchKernelGGL(k_cast, grid_for((size_t)n * kOut), dim3(256), 0, s, m->dout, m->dout_b,
                      (size_t)n * kOut);
@@ -1425,20 +1432,20 @@ void launch_target_mean(clsph_nn* m, clsph_state* learner, clsph_state* teacher,
     launch_sort(teacher);
     launch_density(teacher);
     launch_forces(teacher);
-    hipLaunchKernelGGL(k_accum_acc, grid_for(n), dim3(256), 0, s, teacher->acc_s, teacher->val_b,
+    hipLaunchKernelGGL(k_accum_acc, grid_of_all(n), dim3(256), 0, s, teacher->acc_s, teacher->val_b,
                        teacher->ids, n, m->sum);
     launch_advect(teacher);
     launch_track_ids(teacher);
   }
-  hipLaunchKernelGGL(k_target_mean, grid_for(n), dim3(256), 0, s, learner->val_b, m->sum,
+  hipLaunchKernelGGL(k_target_mean, grid_of_all(n), dim3(256), 0, s, learner->val_b, m->sum,
                      learner->acc_s, n, 1.f / (float)nsub, m->target);
 }
 
 void launch_target(clsph_nn* m, clsph_state* a, clsph_state* t, float dt) {
   hipStream_t s = m->ctx->stream;
   uint32_t n = a->n;
-  hipLaunchKernelGGL(k_invert, grid_for(n), dim3(256), 0, s, t->ids, n, m->loc);
-  hipLaunchKernelGGL(k_target, grid_for(n), dim3(256), 0, s, a->val_b, a->vh, m->loc, t->vh,
+  hipLaunchKernelGGL(k_invert, grid_of_all(n), dim3(256), 0, s, t->ids, n, m->loc);
+  hipLaunchKernelGGL(k_target, grid_of_all(n), dim3(256), 0, s, a->val_b, a->vh, m->loc, t->vh,
                      a->acc_s, n, 1.f / dt, m->target);
 }
 
@@ -1469,8 +1476,8 @@ hipError_t scratch_address(int device, void** ptr) {
 void launch_compare(clsph_nn* m, clsph_state* a, clsph_state* b, float res[2]) {
   hipStream_t s = m->ctx->stream;
   uint32_t n = a->n;
-  hipLaunchKernelGGL(k_invert, grid_for(n), dim3(256), 0, s, b->ids, n, m->loc);
-  hipLaunchKernelGGL(k_invert_perm, grid_for(n), dim3(256), 0, s, b->val_b, n, m->inv);
+  hipLaunchKernelGGL(k_invert, grid_of_all(n), dim3(256), 0, s, b->ids, n, m->loc);
+  hipLaunchKernelGGL(k_invert_perm, grid_of_all(n), dim3(256), 0, s, b->val_b, n, m->inv);
   uint32_t blocks = (n + 255) / 256;
   if (blocks > (uint32_t)kCmpBlocks) blocks = kCmpBlocks;
   if (blocks == 0) blocks = 1;

@@ -24,6 +24,7 @@ def compare(ctx, n, spread, e_cap):
     the same comparison at small sizes."""
     sc = scenes.dam_break(n, seed=5, jitter=0.1)
     parts = sc.particles.copy()
+    parts["velocity"][:, :3] = np.random.default_rng(6).normal(0.0, 0.5, (n, 3))
     if spread > 1.0:
         shake = np.random.default_rng(5).normal(0.0, 0.25 * float(sc.params["h"]), (n, 3))
         parts["position"][:, :3] = parts["position"][:, :3] * spread + shake
@@ -33,14 +34,19 @@ def compare(ctx, n, spread, e_cap):
     for name in ("grid", "hash", "sort", "density"):
         st.stage(name)
     net = native.TwoRoundNetwork(ctx, n, e_cap=e_cap)
-    net.set_params(L.random_params(11).astype(np.float32))
+    flat = L.random_params(11)
+    weights = L.unpack(flat)
+    for name in ("e1.w1", "e2.w1"):  # outputs that depend on the edges' inputs
+        weights[name][:] *= 16.0
+    net.set_params(flat.astype(np.float32))
     edges = net.forward(st)
     ref = net.output().astype(np.float64)[:, :3]
     net.infer(st)
     got = net.output().astype(np.float64)[:, :3]
     net.close()
     st.close()
-    print(f"n {n}, {edges} edges", flush=True)
+    rel = np.sqrt(((ref - got) ** 2).mean()) / np.sqrt((got ** 2).mean())
+    print(f"n {n}, {edges} edges, rel.rms {rel:.2e}", flush=True)
     scale = np.abs(got).max()
     assert np.isfinite(got).all()
     for part in (slice(0, n), slice(n - 50000, n)):
@@ -55,3 +61,10 @@ def test_more_than_a_million_particles(ctx):
     particle 1,048,576."""
     edges = compare(ctx, 1100000, 1.9, 16 * 1100000)
     assert edges < 16 * 1100000
+
+
+def test_more_than_sixteen_million_edges(ctx):
+    """One item of the edge inputs per edge: 65,536 work-groups end at edge
+    16,777,216."""
+    edges = compare(ctx, 700000, 1.0, 34 * 700000)
+    assert edges > 65536 * 256
