@@ -1330,11 +1330,12 @@ static inline float* G(clsph_nn* m, int id) { return m->grad + param_offset(id);
 void forward(clsph_nn* m, const float4* acc0, float gx, float gy, float gz) {
   hipStream_t s = m->ctx->stream;
   const int n = (int)m->n;
-  if (n)
+  if (n) {
     hipLaunchKernelGGL(k_edge_layer, dim3((m->n + kEdgeParts - 1) / kEdgeParts), dim3(256), 0, s,
                        m->E1, W(m, E_W1), P(m, E_B1), m->off, m->n, m->S, m->mask);
-  hipLaunchKernelGGL(k_pack_u, dim3((uint32_t)(((size_t)n * (kIn / 8) + 255) / 256)), dim3(256), 0, s, m->S, m->nu, acc0,
-                     m->degc, m->n, gx, gy, gz, m->u);
+    hipLaunchKernelGGL(k_pack_u, grid_of_all((size_t)n * (kIn / 8)), dim3(256), 0, s, m->S, m->nu,
+                       acc0, m->degc, m->n, gx, gy, gz, m->u);
+  }
   gemm_silu(s, m->u, kIn, W(m, N_W1), kNodeW, P(m, N_B1), m->p1, m->y1, n, kNodeW, kIn);
   gemm_silu(s, m->y1, kNodeW, W(m, N_W2), kNodeW, P(m, N_B2), m->p2, m->y2, n, kNodeW, kNodeW);
   gemm(s, false, false, false, m->y2, kNodeW, W(m, N_W3), kOut, m->out, kOut, n, kOut, kNodeW,
