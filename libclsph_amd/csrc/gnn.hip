@@ -389,12 +389,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         const uint32_t k = quad - (uint32_t)__shfl(start, p, 64);
         const uint32_t d = (uint32_t)__shfl(deg, p, 64);
         const bool on = t < tiles && quad < total;
-        const bool valid = on && 4 * k + r < d;
         const uint32_t i = i0 + p * stride;
         uint32_t j = i0;
         u32x4 lo = {0u, 0u, 0u, 0u}, hi = {0u, 0u, 0u, 0u};
-        if (valid) {
-          j = nbr[((size_t)k * n + i) * 4 + r];
+        if (on) {
+          // past the list's end the quad's first edge again, with a factor of
+          // zero: finite wherever that edge's own term is
+          j = nbr[((size_t)k * n + i) * 4 + (4 * k + r < d ? r : 0u)];
           float f[kFeat];
           edge_features(pos[i], pos[j], vel[i], vel[j], nu[i], nu[j], inv_h, f);
           f[12] = f[13] = f[14] = 1.f;
@@ -403,7 +404,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         rec[rec_at(lane, 0)] = lo;
         rec[rec_at(lane, 1)] = hi;
         if (ROUND2) {
-          const uint32_t one = valid ? 0x3F80u << (16 * (p & 1)) : 0u, h = p >> 1;
+          const uint32_t one = on ? 0x3F80u << (16 * (p & 1)) : 0u, h = p >> 1;
           rec[rec_at(lane, 2)] =
               u32x4{h == 0 ? one : 0u, h == 1 ? one : 0u, h == 2 ? one : 0u, h == 3 ? one : 0u};
           rec[rec_at(lane, 3)] =
