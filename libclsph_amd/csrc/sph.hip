@@ -243,16 +243,19 @@ __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// LDS of one particle in a walk by L lanes.
+// LDS of one particle in a walk by L lanes; in arrays, every element's lists
+// are read 16 bytes at a time.
 constexpr uint32_t kRuns = 18;  // runs of a particle's half-cells: 9 rows of at most two
 template <int L>
-struct LaneWalk {
+struct alignas(16) LaneWalk {
   static constexpr uint32_t kHits = L == 16 ? 64u : 32u;
   float t[kHits];                // neighbours not yet summed: h^2 - r^2
   uint32_t j[kHits];             // and their sorted indices
   uint32_t run_end[kRuns + 1];   // the runs laid end to end
   uint32_t run_shift[kRuns + 1]; // sorted index less laid-out index
 };
+static_assert(sizeof(LaneWalk<4>) % 16 == 0 && sizeof(LaneWalk<16>) % 16 == 0,
+              "16-byte reads of every element are aligned");
 
 // Density sum and neighbour list of one particle i by L consecutive lanes,
 // straight from the sorted positions: its runs of half-cells are looked up by
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(kLanesBlock) void k_density_lanes(
     uint4* __restrict__ nbr, uint32_t* __restrict__ nbr_count, float2* __restrict__ nu,
     uint32_t n) {
   constexpr uint32_t kParts = kLanesBlock / L;  // particles per work-group
-  __shared__ __attribute__((aligned(16))) LaneWalk<L> walks[kParts];
+  __shared__ LaneWalk<L> walks[kParts];
   // a 64-particle entry of the work list is shared by 64 / kParts work-groups
   constexpr uint32_t kShare = 64u / kParts;
   const BlockDesc b = blocks[blockIdx.x / kShare];
