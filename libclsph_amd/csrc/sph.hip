@@ -62,7 +62,10 @@ __device__ inline void for_each_run(const uint32_t hc[3], uint32_t base,
                                     F&& fn) {
   const uint32_t x0 = hc[0] - 1u;
   const bool even = (x0 & 1u) == 0u;
+  // not unrolled: nine rows' addresses ahead cost its callers 22 registers
+#pragma unroll 1
   for (uint32_t dz = 0; dz < 3; ++dz)
+#pragma unroll 1
     for (uint32_t dy = 0; dy < 3; ++dy) {
       uint32_t y = hc[1] + dy - 1u, z = hc[2] + dz - 1u;
       uint32_t a = base + half_key(x0, y, z);
@@ -793,39 +796,29 @@ __device__ inline float4 force_close(const ForceSums& fs, float rho_i,
   return make_float4(f.x / rho_i + g.s[0], f.y / rho_i + g.s[1], f.z / rho_i + g.s[2], 0.f);
 }
 
-// The forces stage by sixteen lanes per particle, for states too small to
-// fill the chip with one particle per lane (rule in launch_forces): a round
-// takes the next sixteen neighbours of the list, one per lane, and leaves
-// their terms in LDS; ten lanes then each add one sum's terms in list order,
-// so that every sum is the one lane's of k_forces to the bit. Bound by the
-// latency of the list, the two gathers and the serial sums; the next round's
-// gathers are in flight meanwhile (4,096 particles: 4.3 us, a lane each 10.5).
+// The acceleration of particle i by sixteen consecutive lanes: a round takes
+// the next sixteen neighbours of the list, one per lane, and leaves their terms
+// in LDS (w, kForceTerms rows); ten lanes then each add one sum's terms in list
+// order, so that every sum is the one lane's of k_forces to the bit. The next
+// round's gathers are in flight meanwhile. Every lane of the wave calls it
+// (`live` false: nothing is written).
 constexpr int kForceLanes = 16, kForceLanesBlock = 256;
-constexpr uint32_t kForceLanesMax = 57344;  // particles up to which they do
 constexpr uint32_t kForceTerms = 14;  // PairTerms' floats, in order
 constexpr uint32_t kForcePitch = 20;  // floats between terms: 16-byte reads, spread over banks
-__global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
-    const float4* __restrict__ fab, const float* __restrict__ rho,
-    const uint32_t* __restrict__ table, const uint4* __restrict__ nbr,
-    const uint32_t* __restrict__ nbr_count, const BlockDesc* __restrict__ blocks,
-    const DevParams* __restrict__ dps, const BatchParams* __restrict__ bp,
-    float4* __restrict__ acc_out, uint32_t n) {
-  constexpr uint32_t L = kForceLanes, kParts = kForceLanesBlock / L, kShare = 64u / kParts;
-  __shared__ __attribute__((aligned(16))) float terms[kParts][kForceTerms * kForcePitch];
-  // a 64-particle entry of the work list is shared by kShare work-groups
-  const BlockDesc b = blocks[blockIdx.x / kShare];
-  const DevParams* dp = dps + b.scene;
-  const uint32_t part = threadIdx.x / L, sub = threadIdx.x % L;
-  const uint32_t p = b.first + (blockIdx.x % kShare) * kParts + part;
-  const uint32_t se = dp->begin + dp->n;
-  const bool live = p < se;
-  if (!__any(live)) return;
-  const uint32_t i = live ? p : se - 1u;
+__device__ inline void force_lanes(float* w, bool live, uint32_t i,
+                                   const float4* __restrict__ fab, const float* __restrict__ rho,
+                                   const uint32_t* __restrict__ table,
+                                   const uint4* __restrict__ nbr,
+                                   const uint32_t* __restrict__ nbr_count,
+                                   const DevParams* __restrict__ dp,
+                                   const BatchParams* __restrict__ bp,
+                                   float4* __restrict__ acc_out, uint32_t n) {
+  constexpr uint32_t L = kForceLanes;
+  const uint32_t sub = threadIdx.x % L;
   const ForceConsts k = force_consts(dp);
   const float4 ai = fab[2u * i], bi = fab[2u * i + 1u];
   const uint32_t all = nbr_count[i];
   const uint32_t cnt = live ? (all < kMaxNeighbours ? all : kMaxNeighbours) : 0u;
-  float* w = terms[part];
   auto index = [&](uint32_t q) {  // past the end: the particle itself
     return q < cnt ? reinterpret_cast<const uint32_t*>(nbr)[4u * ((size_t)(q >> 2) * n + i) + (q & 3u)]
                    : i;
@@ -873,10 +866,68 @@ __global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
   acc_out[i] = force_close(fs, rho[i], dp);
 }
 
-// OVERFLOW_ONLY: only the particles whose neighbours overflow the list
-// (more than kMaxNeighbours), for callers that sum the listed ones
-// themselves.
-template <bool OVERFLOW_ONLY>
+// The forces stage by sixteen lanes per particle, for states too small to
+// fill the chip with one particle per lane (rule in launch_forces). Bound by
+// the latency of the list, the two gathers and the serial sums (4,096
+// particles: 4.3 us, a lane each 10.5).
+constexpr uint32_t kForceLanesMax = 57344;  // particles up to which they do
+__global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
+    const float4* __restrict__ fab, const float* __restrict__ rho,
+    const uint32_t* __restrict__ table, const uint4* __restrict__ nbr,
+    const uint32_t* __restrict__ nbr_count, const BlockDesc* __restrict__ blocks,
+    const DevParams* __restrict__ dps, const BatchParams* __restrict__ bp,
+    float4* __restrict__ acc_out, uint32_t n) {
+  constexpr uint32_t kParts = kForceLanesBlock / kForceLanes, kShare = 64u / kParts;
+  __shared__ __attribute__((aligned(16))) float terms[kParts][kForceTerms * kForcePitch];
+  // a 64-particle entry of the work list is shared by kShare work-groups
+  const BlockDesc b = blocks[blockIdx.x / kShare];
+  const DevParams* dp = dps + b.scene;
+  const uint32_t part = threadIdx.x / kForceLanes;
+  const uint32_t p = b.first + (blockIdx.x % kShare) * kParts + part;
+  const uint32_t se = dp->begin + dp->n;
+  const bool live = p < se;
+  if (!__any(live)) return;
+  force_lanes(terms[part], live, live ? p : se - 1u, fab, rho, table, nbr, nbr_count, dp, bp,
+              acc_out, n);
+}
+
+// The forces stage for the particles whose neighbours overflow the list only
+// (more than kMaxNeighbours), for callers that sum the others themselves. A
+// wave reads the counts of a 64-particle entry of the work list, and nearly
+// always leaves; its overflowing particles are taken four at a time, by
+// sixteen lanes each. Bound by that one load while no list overflows: 4.5 us
+// at 1,048,576 particles (by a lane each, whose pipelined list sum took 131
+// registers and left three waves per SIMD, 7.1; a macro step of 262,144 whose
+// lists overflow 526 and 534 us).
+__global__ __launch_bounds__(kForceLanesBlock) void k_forces_overflow(
+    const float4* __restrict__ fab, const float* __restrict__ rho,
+    const uint32_t* __restrict__ table, const uint4* __restrict__ nbr,
+    const uint32_t* __restrict__ nbr_count, const BlockDesc* __restrict__ blocks, uint32_t entries,
+    const DevParams* __restrict__ dps, const BatchParams* __restrict__ bp,
+    float4* __restrict__ acc_out, uint32_t n) {
+  constexpr uint32_t kParts = kForceLanesBlock / kForceLanes;
+  __shared__ __attribute__((aligned(16))) float terms[kParts][kForceTerms * kForcePitch];
+  // the same in all lanes, so that the scene's parameters stay in scalar registers
+  const uint32_t entry = blockIdx.x * (kForceLanesBlock / 64u) +
+                         (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (entry >= entries) return;
+  const BlockDesc b = blocks[entry];
+  const DevParams* dp = dps + b.scene;
+  const uint32_t lane = threadIdx.x & 63u, p = b.first + lane;
+  uint64_t over = __ballot(p < dp->begin + dp->n && nbr_count[p] > kMaxNeighbours);
+  while (over) {
+    // the wave's four groups of lanes take the four lowest particles left
+    uint64_t mine = over;
+    for (uint32_t q = 0; q < lane / kForceLanes; ++q) mine &= mine - 1u;
+    force_lanes(terms[threadIdx.x / kForceLanes], mine != 0u,
+                b.first + (uint32_t)__builtin_ctzll(mine ? mine : over), fab, rho, table, nbr,
+                nbr_count, dp, bp, acc_out, n);
+    wave_lds_fence();  // the sums are read before the next round's terms
+    for (int q = 0; q < 4; ++q) over &= over - 1u;
+  }
+}
+
+// The forces stage by a lane per particle.
 __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__ fab,
                                                       const float* __restrict__ rho,
                                                       const uint32_t* __restrict__ table,
@@ -890,7 +941,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_forces(const float4* __restrict__
   // runs of 4 work-groups per XCD: neighbour records shared in an L2
   uint32_t i = particle_of<4>(blocks, dps, scene);
   if (i == 0xFFFFFFFFu) return;
-  if (OVERFLOW_ONLY && nbr_count[i] <= kMaxNeighbours) return;
   const DevParams* dp = dps + scene;
   const ForceConsts k = force_consts(dp);
   const uint32_t F = usable_key_end(dp, bp);
@@ -991,7 +1041,7 @@ void launch_forces(clsph_state* s) {
                        s->blocks[0], s->dps, s->bp, s->acc_s, s->n);
     return;
   }
-  hipLaunchKernelGGL((k_forces<false>), dim3(s->nblocks_of(kStageForces)),
+  hipLaunchKernelGGL(k_forces, dim3(s->nblocks_of(kStageForces)),
                      dim3(s->bs_of(kStageForces)), 0, s->ctx->stream, s->fab, s->rho_s,
                      s->table, s->nbr, s->nbr_count, s->table_of(kStageForces), s->dps, s->bp,
                      s->acc_s, s->n);
@@ -999,10 +1049,10 @@ void launch_forces(clsph_state* s) {
 
 void launch_forces_overflow(clsph_state* s) {
   if (s->n == 0) return;
-  hipLaunchKernelGGL((k_forces<true>), dim3(s->nblocks_of(kStageForces)),
-                     dim3(s->bs_of(kStageForces)), 0, s->ctx->stream, s->fab, s->rho_s,
-                     s->table, s->nbr, s->nbr_count, s->table_of(kStageForces), s->dps, s->bp,
-                     s->acc_s, s->n);
+  constexpr uint32_t kWaves = kForceLanesBlock / 64;
+  hipLaunchKernelGGL(k_forces_overflow, dim3((s->nblocks[0] + kWaves - 1) / kWaves),
+                     dim3(kForceLanesBlock), 0, s->ctx->stream, s->fab, s->rho_s, s->table, s->nbr,
+                     s->nbr_count, s->blocks[0], s->nblocks[0], s->dps, s->bp, s->acc_s, s->n);
 }
 
 }  // namespace clsph
