@@ -440,15 +440,17 @@ __device__ inline uint32_t compact10(uint32_t v) {
 // 256 particles) where all the work-group's quads fit, otherwise a cell
 // (4x4x4, 512 for 64): quads stage a quarter fewer candidates for the same
 // particles, but when dense the first ones that fit hold fewer of them. At 8
-// waves 4,820 candidates keep a work-group within 80 KB, so that two fit per
-// CU; below, 768 per wave.
+// waves 4,888 candidates fill a work-group's half of a CU's LDS: in settled
+// fluid a cell that just doesn't fit leaves a few particles to a walk of HBM
+// after all others (with 4,820 candidates, 207,000 and 262,144 particles took
+// 146 and 135 us after 1,800 substeps, now 82 and 88); below, 768 per wave.
 constexpr uint32_t kQuadBox = 144, kCellBox = 64;  // half-cells of a halo
 template <int WAVES>
 struct DensityHalos {
   static constexpr uint32_t kQuads = WAVES < 8 ? (WAVES < 4 ? 1u : 3u) : 6u;  // staged at most
   static constexpr uint32_t kEntries = kQuads * kQuadBox;
   static constexpr uint32_t kCells = kEntries / kCellBox;
-  static constexpr uint32_t kCap = WAVES < 8 ? 768u * WAVES - 4u : 4820u;
+  static constexpr uint32_t kCap = WAVES < 8 ? 768u * WAVES - 4u : 4888u;
   float4 cand[kCap + 4];               // + the padding of a group of four
   uint32_t off[kEntries + 1u];         // halo by halo, half-cell by half-cell
   uint32_t unit[kCells];               // the units' Morton codes
@@ -997,10 +999,11 @@ void launch_density(clsph_state* s, float2* nu) {
   // lanes to spare. Stage time on evolved dam breaks, 1 / 4 / 16 lanes:
   // 16,384 particles 86 / 25 / 15 us, 50,021 49 / 31 / 30, 65,536
   // 48 / 34 / 36, 131,071 62 / 49 / 58. 1 / 4 lanes after 20, 200, 1,000 and
-  // 1,800 substeps: 160,000 39, 64, 59, 85 / 48, 47, 51, 62 us, 180,225 73, 41,
-  // 62, 98 / 53, 50, 57, 72, 207,000 41, 42, 63, 145 / 62, 58, 59, 77, 262,144
-  // 42, 58, 64, 135 / 73, 67, 71, 94, 524,288 77, 85, 124, 165 / 133, 122, 129,
-  // 180 (settled fluid is two to three times as dense).
+  // 1,800 substeps: 131,071 31, 46, 58, 81 / 46, 43, 39, 56 us, 160,000 40, 64,
+  // 59, 84 / 50, 46, 51, 61, 180,225 74, 41, 62, 82 / 55, 50, 56, 70, 207,000
+  // 41, 42, 63, 82 / 63, 58, 58, 77, 262,144 42, 58, 65, 88 / 74, 67, 71, 93,
+  // 524,288 78, 85, 125, 165 / 133, 122, 129, 178 (settled fluid is two to
+  // three times as dense).
   if (s->n <= kLanes4Max) {
     // 64-particle entries of the work list, whatever the stage's block size
     auto lanes = [&](auto kernel, uint32_t share) {
