@@ -443,13 +443,15 @@ __device__ inline uint32_t compact10(uint32_t v) {
 // waves 4,888 candidates fill a work-group's half of a CU's LDS: in settled
 // fluid a cell that just doesn't fit leaves a few particles to a walk of HBM
 // after all others (with 4,820 candidates, 207,000 and 262,144 particles took
-// 146 and 135 us after 1,800 substeps, now 82 and 88); below, 768 per wave.
+// 146 and 135 us after 1,800 substeps, now 82 and 88); below, 768 per wave and
+// two cells per wave.
 constexpr uint32_t kQuadBox = 144, kCellBox = 64;  // half-cells of a halo
 template <int WAVES>
 struct DensityHalos {
   static constexpr uint32_t kQuads = WAVES < 8 ? (WAVES < 4 ? 1u : 3u) : 6u;  // staged at most
-  static constexpr uint32_t kEntries = kQuads * kQuadBox;
-  static constexpr uint32_t kCells = kEntries / kCellBox;
+  static constexpr uint32_t kCells = WAVES < 8 ? 2u * WAVES : 13u;
+  static constexpr uint32_t kEntries =  // half-cells of the halos at most
+      kQuads * kQuadBox > kCells * kCellBox ? kQuads * kQuadBox : kCells * kCellBox;
   static constexpr uint32_t kCap = WAVES < 8 ? 768u * WAVES - 4u : 4888u;
   float4 cand[kCap + 4];               // + the padding of a group of four
   uint32_t off[kEntries + 1u];         // halo by halo, half-cell by half-cell
@@ -494,7 +496,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
                                                         uint32_t* __restrict__ nbr_count,
                                                         float2* __restrict__ nu, uint32_t n) {
   using Halos = DensityHalos<WAVES>;
-  static_assert(Halos::kEntries < (WAVES == 1 ? 192u : 128u * WAVES), "kPer entries per thread");
+  constexpr int kPer = WAVES == 1 ? 3 : 2;  // half-cells per thread
+  static_assert(Halos::kEntries <= (uint32_t)kPer * 64u * WAVES, "every half-cell has a thread");
   __shared__ Halos sh;
   // runs of 16 work-groups per XCD: neighbouring halos share an L2
   const BlockDesc b = blocks[xcd_block<16>(blockIdx.x, gridDim.x)];
@@ -528,7 +531,6 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
     if (starts && ui < Halos::kCells) sh.unit[ui] = key >> bits;
   };
   find_units(5u);
-  constexpr int kPer = WAVES == 1 ? 3 : 2;  // half-cells per thread
   uint32_t rs[kPer], rc[kPer], ex[kPer], staged, box;
   for (;;) {
     const uint32_t most = F == 0u ? 0u : (side == 6u ? Halos::kQuads : Halos::kCells);
@@ -581,10 +583,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const uint32_t q = (uint32_t)kPer * t + (uint32_t)u;
-      if (q <= Halos::kEntries) sh.off[q] = at;
+      if (q < Halos::kEntries) sh.off[q] = at;
       ex[u] = at;
       at += rc[u];
     }
+    if (t == WAVES * 64u - 1u) sh.off[Halos::kEntries] = at;
     __syncthreads();
     // halos staged: the leading ones whose candidates fit
     staged = 0;

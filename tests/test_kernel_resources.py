@@ -42,3 +42,12 @@ def test_density_staging_fills_half_a_compute_unit(kernels):
     (name,) = [k for k in kernels if "k_densityILi8E" in k]
     lds = int(re.search(r"LDS Size \[bytes/block\]: (\d+)", kernels[name]).group(1))
     assert 81920 - 128 < lds <= 81920
+
+
+@pytest.mark.parametrize("waves", [2, 4])
+def test_smaller_work_groups_stage_two_cells_per_wave(kernels, waves):
+    """768 candidates per wave (16 bytes) and the offsets of the 64 half-cells
+    around each of two cells per wave."""
+    (name,) = [k for k in kernels if f"k_densityILi{waves}E" in k]
+    lds = int(re.search(r"LDS Size \[bytes/block\]: (\d+)", kernels[name]).group(1))
+    assert lds >= 16 * 768 * waves + 4 * (64 * 2 * waves + 1)
