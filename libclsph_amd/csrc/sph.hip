@@ -214,6 +214,49 @@ __device__ inline void density_walk_halo(DensityWalk& w, uint32_t i, float4 xi,
   }
 }
 
+// One lane's walk of the sorted positions in HBM, for small work-groups: the
+// same half-cells in the same order as density_walk_halo, as runs of adjacent
+// half-cells, candidates loaded four at a time so that their latencies overlap
+// (pos is padded by 4 entries past the particles, so a group needs no clamp).
+__device__ inline void density_walk_global(DensityWalk& w, uint32_t i, float4 xi,
+                                           const uint32_t hc[3], const float fr[3],
+                                           const DevParams* __restrict__ dp, uint32_t F,
+                                           const float4* __restrict__ pos,
+                                           const uint32_t* __restrict__ table, float h2,
+                                           uint32_t n) {
+  const float lo_x = fr[0] * fr[0], hi_x = (1.f - fr[0]) * (1.f - fr[0]);
+  for (int dz = -1; dz <= 1; ++dz) {
+    const float az = dz < 0 ? fr[2] : (dz > 0 ? 1.f - fr[2] : 0.f);
+    for (int dy = -1; dy <= 1; ++dy) {
+      const float ay = dy < 0 ? fr[1] : (dy > 0 ? 1.f - fr[1] : 0.f);
+      const float ryz = az * az + ay * ay;
+      if (ryz >= kReach2) continue;
+      const uint32_t y = hc[1] + (uint32_t)dy, z = hc[2] + (uint32_t)dz;
+      const uint32_t xa = lo_x + ryz < kReach2 ? hc[0] - 1u : hc[0];
+      const uint32_t xb = hi_x + ryz < kReach2 ? hc[0] + 1u : hc[0];
+      uint32_t x = xa;
+      // half-cells 2k and 2k + 1 share a cell: at most two runs per row
+      for (int piece = 0; piece < 2 && x <= xb; ++piece) {
+        const uint32_t xe = (x | 1u) < xb ? (x | 1u) : xb;
+        uint32_t s, e;
+        half_range(dp->key_base + half_key(x, y, z), xe - x + 1u, table, F, n, s, e);
+        for (uint32_t j0 = s; j0 < e; j0 += 4) {
+          const float4* pj = pos + j0;
+          float4 c[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) c[u] = pj[u];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint32_t j = j0 + (uint32_t)u;
+            w.visit(j < e, dist2(xi, c[u]), h2, (u32x2){j, j}, i);
+          }
+        }
+        x = xe + 1u;
+      }
+    }
+  }
+}
+
 // Density and pressure of particle i from its kernel sum (sph.cl:36-39), and
 // what the later stages read: its neighbour count, its force inputs
 // fab[2i] = (x, p / rho^2), fab[2i + 1] = (v, m / rho) and, with `nu`, the
@@ -444,11 +487,12 @@ __device__ inline uint32_t compact10(uint32_t v) {
 // fluid a cell that just doesn't fit leaves a few particles to a walk of HBM
 // after all others (with 4,820 candidates, 207,000 and 262,144 particles took
 // 146 and 135 us after 1,800 substeps, now 82 and 88); below, 768 per wave and
-// two cells per wave.
+// two cells per wave. One wave's particles nearly always span two quads of
+// which one fits, so it stages cells only.
 constexpr uint32_t kQuadBox = 144, kCellBox = 64;  // half-cells of a halo
 template <int WAVES>
 struct DensityHalos {
-  static constexpr uint32_t kQuads = WAVES < 8 ? (WAVES < 4 ? 1u : 3u) : 6u;  // staged at most
+  static constexpr uint32_t kQuads = WAVES == 8 ? 6u : WAVES == 4 ? 3u : WAVES == 2 ? 1u : 0u;
   static constexpr uint32_t kCells = WAVES < 8 ? 2u * WAVES : 13u;
   static constexpr uint32_t kEntries =  // half-cells of the halos at most
       kQuads * kQuadBox > kCells * kCellBox ? kQuads * kQuadBox : kCells * kCellBox;
@@ -460,7 +504,11 @@ struct DensityHalos {
   uint32_t wave_units[WAVES];
 };
 // Lanes per particle outside the staged halos, and what their walks keep in
-// the candidates' bytes (two 80 KB work-groups per CU leave no others).
+// the candidates' bytes (two 80 KB work-groups per CU leave no others). One or
+// two waves stage too little of dense fluid to leave many of their particles to
+// four lanes each: those walk one to a lane, beside the staged ones (207,000
+// particles after 20 and 1,800 substeps, work-groups of 64: 131 and 182 us by
+// four lanes, 120 and 148 by one; of 128: 87 and 214, 91 and 169).
 constexpr int kRestLanes = 4;
 template <int WAVES>
 struct DensityRest {
@@ -474,12 +522,13 @@ struct DensityRest {
 // first stages the halos of the units its particles fall in (DensityHalos) in
 // LDS (coalesced runs of the sorted positions); particles then walk their
 // 3x3x3 half-cells there, one to a lane. Those of units beyond the staging
-// capacity, and every particle when
-// the table is unusable, are then walked from HBM by four lanes each, with
-// the same visiting order: a lane's walk of HBM by itself took 30-50 us, in
-// some work-group of every launch. With cells only, whose halos overlap more,
-// 207,000 particles took 65 us instead of 41 after 20 substeps, 1,048,576 209,
-// 149 and 219 instead of 198, 147 and 203 after 20, 200 and 1,000, 2,097,152
+// capacity, and every particle when the table is unusable, are walked from HBM
+// with the same visiting order: by four lanes each after the others (a lane's
+// walk of HBM by itself took 30-50 us, in some work-group of every launch), in
+// small work-groups by their own lanes (kRestLanes). With cells only, whose
+// halos overlap more, 207,000 particles took 65 us instead of 41 after 20
+// substeps, 1,048,576 209, 149 and 219 instead of 198, 147 and 203 after 20,
+// 200 and 1,000, 2,097,152
 // 389, 339 and 446 instead of 376, 325 and 398.
 template <int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict__ pos,
@@ -496,7 +545,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
                                                         uint32_t* __restrict__ nbr_count,
                                                         float2* __restrict__ nu, uint32_t n) {
   using Halos = DensityHalos<WAVES>;
-  constexpr int kPer = WAVES == 1 ? 3 : 2;  // half-cells per thread
+  constexpr int kPer = 2;  // half-cells per thread
   static_assert(Halos::kEntries <= (uint32_t)kPer * 64u * WAVES, "every half-cell has a thread");
   __shared__ Halos sh;
   // runs of 16 work-groups per XCD: neighbouring halos share an L2
@@ -513,7 +562,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
   // when it is the first particle or its unit differs from its predecessor's.
   const uint32_t key = live ? keys[i] - dp->key_base : 0u;
   const uint32_t prev = (live && t > 0) ? keys[i - 1] - dp->key_base : 0u;
-  uint32_t units, ui, side = 6u;
+  uint32_t units, ui, side = Halos::kQuads ? 6u : 4u;
   auto find_units = [&](uint32_t bits) {
     const bool starts = live && (t == 0 || (key >> bits) != (prev >> bits));
     const uint64_t mask = __ballot(starts);
@@ -530,7 +579,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
     ui = before + (uint32_t)__popcll(mask & (~0ull >> (63u - lane))) - 1u;
     if (starts && ui < Halos::kCells) sh.unit[ui] = key >> bits;
   };
-  find_units(5u);
+  find_units(side == 6u ? 5u : 3u);
   uint32_t rs[kPer], rc[kPer], ex[kPer], staged, box;
   for (;;) {
     const uint32_t most = F == 0u ? 0u : (side == 6u ? Halos::kQuads : Halos::kCells);
@@ -610,17 +659,21 @@ __global__ __launch_bounds__(WAVES * 64) void k_density(const float4* __restrict
   }
   __syncthreads();
 
-  if (live && ui < staged) {
+  constexpr bool kRest = WAVES >= 4;  // the particles not staged follow, by several lanes
+  if (live && (!kRest || ui < staged)) {
     const float4 xi = pos[i];
     uint32_t hc[3];
     float fr[3];
     half_cell_frac(xi, dp, hc, fr);
     DensityWalk w(nbr, i, n, h2);
-    density_walk_halo(w, i, xi, hc, fr, side, sh.cand, sh.off + box * ui, h2);
+    if (kRest || ui < staged)
+      density_walk_halo(w, i, xi, hc, fr, side, sh.cand, sh.off + box * ui, h2);
+    else
+      density_walk_global(w, i, xi, hc, fr, dp, F, pos, table, h2, n);
     w.finish();
     density_store(dp, i, xi, w.acc, w.cnt, vel, rho, prs, fab, nbr_count, nu);
   }
-  if (staged == units) return;  // uniform: every unit was staged
+  if (!kRest || staged == units) return;  // uniform: every particle has been walked
   // the rest, in the order of their threads
   const bool left = live && ui >= staged;
   const uint64_t lm = __ballot(left);

@@ -1,0 +1,33 @@
+"""Times of stages against each other, where a work-group size or the state of
+the fluid has once cost a multiple."""
+import pytest
+
+from libclsph_amd import learned as lrn
+from libclsph_amd import native, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def test_small_density_work_groups_in_settled_fluid():
+    """Work-groups of 64 and 128 threads against the default of 512 after 1,800
+    substeps: 1.80 and 2.06 times as long, 2.2 and 2.6 when four lanes took
+    each particle outside the staged halos; bounds in between."""
+    ctx = native.Context(0)
+    sc = scenes.dam_break(207000, seed=1)
+    st = lrn.make_state(ctx, sc)
+    st.upload(sc.particles)
+    for _ in range(36):
+        st.step(50)
+        ctx.sync()
+    for name in ("grid", "hash", "sort", "density"):
+        st.stage(name)
+    us = {}
+    for size in (64, 128, 512):
+        st.set_block_sizes([0, 0, 0, 0, size, 0, 0])
+        st.stage("density")
+        us[size] = 1e3 * min(st.time_stage("density", 30) for _ in range(3))
+    print({k: round(v, 1) for k, v in us.items()}, flush=True)
+    st.close()
+    ctx.close()
+    assert us[64] <= 2.0 * us[512]
+    assert us[128] <= 2.3 * us[512]
