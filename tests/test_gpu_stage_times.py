@@ -4,6 +4,7 @@ import pytest
 
 from libclsph_amd import learned as lrn
 from libclsph_amd import native, scenes
+from test_gpu_sort_paths import cloud, state_of
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +32,20 @@ def test_small_density_work_groups_in_settled_fluid():
     ctx.close()
     assert us[64] <= 2.0 * us[512]
     assert us[128] <= 2.3 * us[512]
+
+
+def test_a_wide_table_is_filled_by_the_whole_chip():
+    """5,000 particles in two far corners: the cell table of 77 million keys
+    takes 2.1 times as long as that of 8.4 million, 4.1 times when 128
+    work-groups wrote its long runs of empty keys; a bound in between."""
+    ctx = native.Context(0)
+    us = []
+    for side in (5.0, 20.0):
+        st = state_of(ctx, cloud(5000, side, corners=True), 1 << 24)
+        for name in ("grid", "hash", "sort", "cell_table"):
+            st.stage(name)
+        us.append(1e3 * min(st.time_stage("cell_table", 20) for _ in range(3)))
+        st.close()
+    ctx.close()
+    print(["%.1f" % u for u in us], flush=True)
+    assert us[1] <= 3.0 * us[0]
