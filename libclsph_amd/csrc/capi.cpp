@@ -980,10 +980,12 @@ int clsph_bounce_capped(clsph_state* st, uint32_t* count) {
 
 int clsph_time_steps(clsph_state* st, uint32_t nsteps, float* ms) {
   if (!st || !ms) return CLSPH_EINVAL;
-  // the captures stay out of the timed region
+  // the captures stay out of the timed region, also those of a call that
+  // itself reaches kGraphAfter
   int rc = ensure_graph(st, 0);
   if (nsteps >= kGraphAfter) st->graph_steps = kGraphAfter;
-  for (int k = 1; !rc && k < kNumGraphs && st->graph_steps == kGraphAfter; ++k)
+  const bool more = nsteps >= kGraphAfter - st->graph_steps;
+  for (int k = 1; !rc && more && k < kNumGraphs; ++k)
     if (kGraphSteps[k] <= nsteps) rc = ensure_graph(st, k);
   if (rc) return rc;
   hipEvent_t a, b;
