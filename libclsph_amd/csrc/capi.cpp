@@ -988,17 +988,21 @@ int clsph_time_steps(clsph_state* st, uint32_t nsteps, float* ms) {
   for (int k = 1; !rc && more && k < kNumGraphs; ++k)
     if (kGraphSteps[k] <= nsteps) rc = ensure_graph(st, k);
   if (rc) return rc;
-  hipEvent_t a, b;
-  HIPCK(st->ctx, hipEventCreate(&a));
-  HIPCK(st->ctx, hipEventCreate(&b));
-  HIPCK(st->ctx, hipEventRecord(a, st->ctx->stream));
-  rc = launch_steps(st, nsteps);
+  hipEvent_t ev[2] = {};
+  auto timed = [&]() -> int {
+    for (hipEvent_t& e : ev) HIPCK(st->ctx, hipEventCreate(&e));
+    HIPCK(st->ctx, hipEventRecord(ev[0], st->ctx->stream));
+    int r = launch_steps(st, nsteps);
+    if (r) return r;
+    HIPCK(st->ctx, hipEventRecord(ev[1], st->ctx->stream));
+    HIPCK(st->ctx, hipEventSynchronize(ev[1]));
+    HIPCK(st->ctx, hipEventElapsedTime(ms, ev[0], ev[1]));
+    return CLSPH_OK;
+  };
+  rc = timed();
+  for (hipEvent_t e : ev)
+    if (e) (void)hipEventDestroy(e);
   if (rc) return rc;
-  HIPCK(st->ctx, hipEventRecord(b, st->ctx->stream));
-  HIPCK(st->ctx, hipEventSynchronize(b));
-  HIPCK(st->ctx, hipEventElapsedTime(ms, a, b));
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
   st->acc_zero = true;
   st->fields_canonical = false;
   st->stage = kStageAdvect;
