@@ -1047,7 +1047,7 @@ static void gemm_cast(hipStream_t s, const uint16_t* A, const uint16_t* B, uint1
   nn::GemmArgs g{};
   g.A = A, g.lda = kWidth, g.B = B, g.ldb = kWidth, g.out16 = out16, g.ldc = ldo;
   g.M = M, g.N = kWidth, g.K = kWidth, g.alpha = 1.f, g.bias = bias, g.rowscale = rowscale;
-  gemm(s, false, false, nn::kEpiCast, g);
+  gemm<false, false, nn::kEpiCast>(s, g);
 }
 
 // Second and third layer of an edge round: s1 -> z2 -> S = bf16(sum silu(z2) / C).
@@ -1106,7 +1106,7 @@ void forward(clsph_gnn* m, const DevParams* dp, float4* acc, float gx, float gy,
   g.A = m->E1, g.lda = kFeat, g.B = W(m, E2_W1), g.ldb = kWidth, g.C = m->z1[1], g.ldc = kWidth;
   g.M = e, g.N = kWidth, g.K = kFeat, g.alpha = 1.f, g.bias = P(m, E2_B1);
   g.out16 = m->s1[1], g.row_add = m->PA, g.row_of = m->dst, g.row_add2 = m->PB, g.row_of2 = m->src;
-  gemm(s, false, false, nn::kEpiEdgeSilu, g);
+  gemm<false, false, nn::kEpiEdgeSilu>(s, g);
   edge_tail(m, 1, E2_W2, E2_B2, s);
   node_round2(m, acc, gx, gy, gz, s);
 }

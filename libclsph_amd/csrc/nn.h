@@ -169,7 +169,18 @@ struct GemmArgs {
   const uint32_t* row_of;
   const uint32_t* row_of2;
 };
-void gemm(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g);
+// The (transposes, epilogue) combinations it is built for.
+constexpr bool gemm_built(bool ta, bool tb, int epi) {
+  return epi == kEpiStore || epi == kEpiAdd ||
+         (!ta && (tb ? epi == kEpiDsilu
+                     : epi == kEpiSilu || epi == kEpiEdgeSilu || epi == kEpiCast));
+}
+void gemm_launch(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g);
+template <bool TA, bool TB, int EPI>
+void gemm(hipStream_t s, const GemmArgs& g) {
+  static_assert(gemm_built(TA, TB, EPI), "no such matrix product");
+  gemm_launch(s, TA, TB, EPI, g);
+}
 void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
           const uint16_t* B, int ldb, float* C, int ldc, int M, int N, int K, float alpha,
           const float* bias = nullptr, const float* rowscale = nullptr);

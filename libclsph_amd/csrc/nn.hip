@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
 // until about two work-groups per compute unit share it, 256 of K each at
 // least: a weight gradient over 16,384 particles runs on 64 work-groups, not
 // on 4 (311 -> 15 us), over 557,000 edges on 512, not on 136 (357 -> 55).
-void gemm(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g) {
+void gemm_launch(hipStream_t s, bool ta, bool tb, int epi, GemmArgs g) {
   if (g.M <= 0 || g.N <= 0 || g.K <= 0) return;
   const int mt = (g.M + kTile - 1) / kTile, nt = (g.N + kTile - 1) / kTile;
   int splits = 1;
@@ -281,7 +281,7 @@ void gemm(hipStream_t s, bool ta, bool tb, bool add, const uint16_t* A, int lda,
   GemmArgs g{};
   g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = C, g.ldc = ldc;
   g.M = M, g.N = N, g.K = K, g.alpha = alpha, g.bias = bias, g.rowscale = rowscale;
-  gemm(s, ta, tb, add ? kEpiAdd : kEpiStore, g);
+  gemm_launch(s, ta, tb, add ? kEpiAdd : kEpiStore, g);
 }
 
 // A weight gradient and its bias gradient: W (M x N) += A^T B, b (N) += the
@@ -291,7 +291,7 @@ void gemm_weight_grad(hipStream_t s, const uint16_t* A, int lda, const uint16_t*
   GemmArgs g{};
   g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = W, g.ldc = N;
   g.M = M, g.N = N, g.K = K, g.alpha = 1.f, g.colsum = b;
-  gemm(s, true, false, kEpiAdd, g);
+  gemm<true, false, kEpiAdd>(s, g);
 }
 
 // Column sums (optionally row-weighted) of f32 rows, `cols` of them (a
@@ -340,7 +340,7 @@ void gemm_silu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, int
   GemmArgs g{};
   g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = C, g.ldc = N, g.out16 = out16;
   g.M = M, g.N = N, g.K = K, g.alpha = 1.f, g.bias = bias;
-  gemm(s, false, false, kEpiSilu, g);
+  gemm<false, false, kEpiSilu>(s, g);
 }
 
 // out16 = bf16(A B^T silu'(pre)); out16 may be A itself when N fits one tile
@@ -351,7 +351,7 @@ void gemm_dsilu(hipStream_t s, const uint16_t* A, int lda, const uint16_t* B, in
   g.A = A, g.lda = lda, g.B = B, g.ldb = ldb, g.C = const_cast<float*>(pre), g.ldc = N;
   g.out16 = out16;
   g.M = M, g.N = N, g.K = K, g.alpha = 1.f;
-  gemm(s, false, true, kEpiDsilu, g);
+  gemm<false, true, kEpiDsilu>(s, g);
 }
 
 // ---------------------------------------------------------------------------
