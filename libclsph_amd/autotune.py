@@ -7,7 +7,9 @@ the neighbour loops). For each scene-size bucket (log2 of the scene particle
 count) the tuner builds a batch of equal dam breaks of that size, measures
 graph-replayed substeps for every candidate size of one stage at a time
 (coordinate descent, two sweeps) and records the fastest setting. A batch is
-then run with the entry of its particle-weighted median scene size.
+then run with the entry of its particle-weighted median scene size. Stages
+whose kernels choose their own work-groups in a state of that many particles
+are left out.
 
     python -m libclsph_amd.autotune --out table.json [--buckets 12 14 16 18]
 """
@@ -23,6 +25,11 @@ CANDIDATES = (64, 128, 256, 512)
 # Stages that run over the work-group table (stage order of clsph_time_stage).
 TUNED = {"hash": 1, "density": 4, "forces": 5, "advect": 6}
 DEFAULT = [256, 256, 256, 256, 512, 512, 256]  # the state's own defaults
+# Particles of a state (all scenes) up to which a stage's kernel chooses its
+# own work-groups: kLanes4Max and kForceLanesMax in csrc/sph.hip, and for
+# single scenes kFusedMax in csrc/sort.hip.
+OWN_UP_TO = {"density": 180224, "forces": 57344}
+OWN_SINGLE_UP_TO = {"hash": 655360}
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning", "mi355x.json")
 
 
@@ -52,6 +59,12 @@ def sizes_for(counts, table=None):
     return list(table[key]["sizes"])
 
 
+def tunable(name, particles, scenes):
+    """Whether the stage's work-group size has an effect in such a state."""
+    return particles > max(OWN_UP_TO.get(name, 0),
+                           OWN_SINGLE_UP_TO.get(name, 0) if scenes == 1 else 0)
+
+
 def time_config(state, sizes, steps):
     state.set_block_sizes(sizes)
     state.step(3)  # capture + settle
@@ -75,6 +88,8 @@ def tune_state(state, steps=20, sweeps=2, log=print, margin=0.01):
     sizes = list(state.block_sizes())
     for _ in range(sweeps):
         for name, stage in TUNED.items():
+            if not tunable(name, state.n, len(getattr(state, "counts", [state.n]))):
+                continue
             for c in CANDIDATES:
                 if c == sizes[stage]:
                     continue
