@@ -290,26 +290,34 @@ __global__ __launch_bounds__(kScatBlock) void k_lsd_scatter(
   for (uint32_t q = threadIdx.x; q < kStageQ; q += kScatBlock)
     stage[q] = make_uint4(0u, 0u, 0u, 0u);
   if constexpr (FOLD) {
-    // totals and counts of the tiles before this one: for few digits, several
-    // threads share one and take every S-th tile
+    // totals and counts of the tiles before this one: a thread takes four
+    // digits (one 16-byte load a tile), several threads every S-th tile each
     for (uint32_t d = threadIdx.x; d < nb; d += kScatBlock) tot[d] = dshift[d] = 0u;
     __syncthreads();
-    const uint32_t S = nb < (uint32_t)kScatBlock ? (uint32_t)kScatBlock >> db : 1u;
-    const uint32_t first = nb < (uint32_t)kScatBlock ? threadIdx.x >> db : 0u;
-    for (uint32_t d = S > 1u ? threadIdx.x & (nb - 1u) : threadIdx.x; d < nb; d += kScatBlock) {
-      uint32_t all = 0, before = 0;
+    if (db >= 2u) {
+      const uint32_t d = 4u * (threadIdx.x & ((nb >> 2) - 1u));
+      const uint32_t S = (uint32_t)kScatBlock >> (db - 2u);
+      uint32_t all[4] = {0u, 0u, 0u, 0u}, before[4] = {0u, 0u, 0u, 0u};
 #pragma unroll 8
-      for (uint32_t q = first; q < gridDim.x; q += S) {
-        const uint32_t c = offsets[((size_t)q << db) + d];
-        all += c;
-        before += q < blockIdx.x ? c : 0u;
+      for (uint32_t q = threadIdx.x >> (db - 2u); q < gridDim.x; q += S) {
+        const uint4 c4 = *(const uint4*)(offsets + ((size_t)q << db) + d);
+        const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          all[k] += c[k];
+          before[k] += q < blockIdx.x ? c[k] : 0u;
+        }
       }
-      if (S > 1u) {
-        atomicAdd(&tot[d], all);
-        atomicAdd(&dshift[d], before);
-      } else {
-        tot[d] = all;
-        dshift[d] = before;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        atomicAdd(&tot[d + k], all[k]);
+        atomicAdd(&dshift[d + k], before[k]);
+      }
+    } else if (threadIdx.x < nb) {
+      for (uint32_t q = 0; q < gridDim.x; ++q) {
+        const uint32_t c = offsets[((size_t)q << db) + threadIdx.x];
+        tot[threadIdx.x] += c;
+        dshift[threadIdx.x] += q < blockIdx.x ? c : 0u;
       }
     }
     __syncthreads();
@@ -793,7 +801,13 @@ void launch_cell_table(clsph_state* s) {
 // 16,384 70.9 / 65.3 / 62.1, 50,021 (25 tiles) 98.0 / 95.1 / 91.8, 98,304 (48)
 // 105.2 / 104.9 / 101.3, 131,071 (64) 118.6 / 119.5 / 116.2 (115.2 with the
 // scan); 524,288 213.8 and with the one kernel 210.5, 1,048,576 364.3 and 364.8.
-constexpr uint32_t kFoldTiles = 48;
+// A work-group reads all tiles' counts of all digits, of which a table of more
+// than 2^20 cells can ask for 2,048: the passes of 16,384 / 30,001 / 98,304
+// particles in such a one take 31 / 32 / 36 us with scans and 30 / 35 / 58
+// without. (With a digit at a time per thread 43 / 58 / 125, and 300 scenes of
+// 200 particles 37 instead of 27.)
+constexpr uint32_t kFoldTiles = 48, kFoldTilesWide = 12;
+constexpr uint32_t kFoldKeys = 8u << 20;  // capacity of a table that isn't wide
 constexpr uint32_t kFusedMax = 655360;
 
 // The LSD passes and the cell pass; `counted`: the keys and the first pass's
@@ -817,7 +831,7 @@ static void sort_keys(clsph_state* s, bool counted) {
     else if (per <= 32) go(k_lsd_scan<32>);
     else go(k_lsd_scan<0>);
   };
-  const bool fold = tiles <= kFoldTiles;
+  const bool fold = tiles <= (s->table_cap <= kFoldKeys ? kFoldTiles : kFoldTilesWide);
   for (uint32_t p = 0; p < s->sort_passes; ++p) {
     uint32_t* kout = (p & 1) ? s->key_u : s->key_t;
     uint32_t* vout = (p & 1) ? s->val_u : s->val_t;

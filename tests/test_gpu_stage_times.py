@@ -49,3 +49,22 @@ def test_a_wide_table_is_filled_by_the_whole_chip():
     ctx.close()
     print(["%.1f" % u for u in us], flush=True)
     assert us[1] <= 3.0 * us[0]
+
+
+def test_digit_counts_of_a_wide_table_are_added_up_at_no_loss():
+    """The LSD passes (the sort stage less its cell pass) in a table of 2.1
+    million cells, whose digits have 2,048 values, on either side of the 48
+    tiles up to which the scatter may add up the tiles' counts: as long, 3.3
+    times when it did so whatever the digits; a bound in between."""
+    ctx = native.Context(0)
+    us = []
+    for n in (98304, 98305):
+        st = state_of(ctx, cloud(n, 9.5), 1 << 22)
+        for name in ("grid", "hash", "sort", "cell_table"):
+            st.stage(name)
+        us.append(1e3 * min(st.time_stage("sort", 20) - st.time_stage("cell_table", 20)
+                            for _ in range(5)))
+        st.close()
+    ctx.close()
+    print(["%.1f" % u for u in us], flush=True)
+    assert us[0] <= 1.6 * us[1]
