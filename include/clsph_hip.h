@@ -136,8 +136,9 @@ int clsph_batch_bounce_capped(clsph_state* st, uint32_t scene, uint32_t* count);
  * clsph_time_stage; 64, 128, 256 or 512; 0 keeps the current one). The
  * autotuner sets these; results do not depend on them. Kernels of several
  * lanes per particle choose their own: density in states of up to 180,224
- * particles (of all scenes), forces up to 57,344; so does the kernel that
- * hashes a single scene of up to 655,360 particles in clsph_step. */
+ * particles (of all scenes), forces up to 57,344 (28,672 where no scene has
+ * more than 8,192); so does the kernel that hashes a single scene of up to
+ * 655,360 particles in clsph_step. */
 int clsph_set_block_sizes(clsph_state* st, const uint32_t sizes[7]);
 int clsph_get_block_sizes(const clsph_state* st, uint32_t sizes[7]);
 

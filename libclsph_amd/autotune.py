@@ -26,9 +26,11 @@ CANDIDATES = (64, 128, 256, 512)
 TUNED = {"hash": 1, "density": 4, "forces": 5, "advect": 6}
 DEFAULT = [256, 256, 256, 256, 512, 512, 256]  # the state's own defaults
 # Particles of a state (all scenes) up to which a stage's kernel chooses its
-# own work-groups: kLanes4Max and kForceLanesMax in csrc/sph.hip, and for
-# single scenes kFusedMax in csrc/sort.hip.
+# own work-groups: kLanes4Max and kForceLanesMax in csrc/sph.hip (where no scene
+# is larger than kSmallScene, kForceLanesSmallMax), and for single scenes
+# kFusedMax in csrc/sort.hip.
 OWN_UP_TO = {"density": 180224, "forces": 57344}
+SMALL_SCENE, OWN_SMALL_UP_TO = 8192, {"forces": 28672}
 OWN_SINGLE_UP_TO = {"hash": 655360}
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning", "mi355x.json")
 
@@ -59,10 +61,15 @@ def sizes_for(counts, table=None):
     return list(table[key]["sizes"])
 
 
-def tunable(name, particles, scenes):
-    """Whether the stage's work-group size has an effect in such a state."""
-    return particles > max(OWN_UP_TO.get(name, 0),
-                           OWN_SINGLE_UP_TO.get(name, 0) if scenes == 1 else 0)
+def tunable(name, counts):
+    """Whether the stage's work-group size has an effect in a state of scenes
+    of that many particles."""
+    own = OWN_UP_TO.get(name, 0)
+    if max(counts) <= SMALL_SCENE:
+        own = OWN_SMALL_UP_TO.get(name, own)
+    if len(counts) == 1:
+        own = max(own, OWN_SINGLE_UP_TO.get(name, 0))
+    return sum(counts) > own
 
 
 def time_config(state, sizes, steps):
@@ -88,7 +95,7 @@ def tune_state(state, steps=20, sweeps=2, log=print, margin=0.01):
     sizes = list(state.block_sizes())
     for _ in range(sweeps):
         for name, stage in TUNED.items():
-            if not tunable(name, state.n, len(getattr(state, "counts", [state.n]))):
+            if not tunable(name, getattr(state, "counts", [state.n])):
                 continue
             for c in CANDIDATES:
                 if c == sizes[stage]:

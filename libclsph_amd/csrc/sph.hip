@@ -8,6 +8,8 @@
 // h of particle i lies in the 3x3x3 block of half-cells around i's own:
 // visiting that block drops exactly the terms chi zeroes, and the sums are
 // the reference's up to FP32 rounding (summation order differs).
+#include <algorithm>
+
 #include "state.h"
 
 namespace clsph {
@@ -929,6 +931,8 @@ __device__ inline void force_lanes(float* w, bool live, uint32_t i,
 // the latency of the list, the two gathers and the serial sums (4,096
 // particles: 4.3 us, a lane each 10.5).
 constexpr uint32_t kForceLanesMax = 57344;  // particles up to which they do
+constexpr uint32_t kSmallScene = 8192;      // particles of a scene up to which, with none
+constexpr uint32_t kForceLanesSmallMax = 28672;  // larger, they do up to this many
 __global__ __launch_bounds__(kForceLanesBlock) void k_forces_lanes(
     const float4* __restrict__ fab, const float* __restrict__ rho,
     const uint32_t* __restrict__ table, const uint4* __restrict__ nbr,
@@ -1092,8 +1096,12 @@ void launch_forces(clsph_state* s) {
   // settled dam break. Stage times with 1 / 16 lanes, early and settled: 4,096
   // particles 10.5 / 4.3 and 15.5 / 5.6 us, 16,384 11.6 / 6.3 and 22.7 / 8.9,
   // 50,021 12.1 / 13.4 and 28.1 / 20.4, 65,536 12.1 / 15.6 and 28.9 / 24.3,
-  // 98,304 12.2 / 22.1 and 28.2 / 32.4.
-  if (s->n <= kForceLanesMax) {
+  // 98,304 12.2 / 22.1 and 28.2 / 32.4. Small scenes' lists stay short however
+  // many scenes there are: 100 of 200 particles 7.9 / 8.7 and 9.3 / 9.3, 20 of
+  // 1,500 10.8 / 9.8 and 14.1 / 11.6, 400 of 100 8.7 / 13.1 and 9.3 / 14.0, 100
+  // of 500 10.3 / 13.8 and 11.5 / 16.3, 14 of 4,000 11.3 / 14.7 and 16.2 / 18.8.
+  const uint32_t largest = *std::max_element(s->scene_n.begin(), s->scene_n.end());
+  if (s->n <= (largest > kSmallScene ? kForceLanesMax : kForceLanesSmallMax)) {
     constexpr uint32_t kShare = 64u * kForceLanes / kForceLanesBlock;
     hipLaunchKernelGGL(k_forces_lanes, dim3(s->nblocks[0] * kShare), dim3(kForceLanesBlock), 0,
                        s->ctx->stream, s->fab, s->rho_s, s->table, s->nbr, s->nbr_count,

@@ -15,6 +15,8 @@ def constant(source, name):
 def test_limits_are_the_kernels():
     assert autotune.OWN_UP_TO == {"density": constant("sph.hip", "kLanes4Max"),
                                   "forces": constant("sph.hip", "kForceLanesMax")}
+    assert autotune.SMALL_SCENE == constant("sph.hip", "kSmallScene")
+    assert autotune.OWN_SMALL_UP_TO == {"forces": constant("sph.hip", "kForceLanesSmallMax")}
     assert autotune.OWN_SINGLE_UP_TO == {"hash": constant("sort.hip", "kFusedMax")}
 
 
@@ -43,7 +45,8 @@ class Recorder:
     ([4096], {"advect"}), ([65536], {"forces", "advect"}),
     ([262144], {"density", "forces", "advect"}),
     ([1048576], {"hash", "density", "forces", "advect"}),
-    ([2048] * 16, {"hash", "advect"}), ([4096] * 16, {"hash", "forces", "advect"}),
+    ([2048] * 14, {"hash", "advect"}), ([2048] * 15, {"hash", "forces", "advect"}),
+    ([8193] * 6, {"hash", "advect"}), ([4096] * 16, {"hash", "forces", "advect"}),
     ([16384] * 16, {"hash", "density", "forces", "advect"})])
 def test_stages_that_choose_their_own_are_left_out(counts, stages):
     state = Recorder(counts)
