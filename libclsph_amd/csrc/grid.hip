@@ -73,9 +73,10 @@ __device__ void batch_keys(DevParams* __restrict__ dps, BatchParams* __restrict_
 // the batch's keys (batch_keys); a single scene does so from the values in
 // its registers. The parameters thread 0 needs are loaded before the
 // reduction, so that their latency overlaps it.
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void k_grid_params(
-    DevParams* __restrict__ dps, const float* __restrict__ partial, uint32_t stride,
-    BatchParams* __restrict__ bp) {
+__global__ __launch_bounds__(1024) void k_grid_params(DevParams* __restrict__ dps,
+                                                      const float* __restrict__ partial,
+                                                      uint32_t stride,
+                                                      BatchParams* __restrict__ bp) {
   __shared__ float red[6][16];
   DevParams* dp = dps + blockIdx.x;
   const float h = dp->p.h;
@@ -84,11 +85,13 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
   float v[6];
   if (!scene_box<16>(dp, partial, stride, red, v)) return;
   if (threadIdx.x != 0 && gridDim.x == 1u) return;
-  GridOf g = {};
-  if (threadIdx.x == 0) g = grid_of(v, h, np, dp);
-  if (gridDim.x == 1u) {
-    single_layout(dp, bp, g.cells, err0 | g.err, table_cap, sort_passes);
-    return;
+  if (threadIdx.x == 0) {
+    const GridOf g = grid_of(v, h, np);
+    store_grid(dp, g, np);
+    if (gridDim.x == 1u) {
+      single_layout(dp, bp, g.cells, err0 | g.err, table_cap, sort_passes);
+      return;
+    }
   }
   // the scenes' grids are in place once every work-group has passed here
   uint32_t last = 0;

@@ -48,16 +48,15 @@ __device__ inline bool scene_box(const DevParams* __restrict__ dp,
                                  float (&red)[6][WAVES], float v[6]) {
   const float inf = __builtin_huge_valf();
   for (int k = 0; k < 6; ++k) v[k] = k < 3 ? inf : -inf;
-  // eight partial boxes per thread in flight at a time; past the end the first
-  // of them again, so that no load is conditional
+  // eight partial boxes per thread in flight at a time
   const uint32_t b0 = dp->block_begin, b1 = dp->block_end;
   for (uint32_t b = b0 + threadIdx.x; b < b1; b += 8u * blockDim.x) {
     float q[8][6];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const uint32_t bu = b + (uint32_t)u * blockDim.x, at = bu < b1 ? bu : b;
+      const uint32_t bu = b + (uint32_t)u * blockDim.x;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) q[u][k] = partial[k * stride + at];
+      for (int k = 0; k < 6; ++k) q[u][k] = bu < b1 ? partial[k * stride + bu] : (k < 3 ? inf : -inf);
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -88,22 +87,15 @@ __device__ inline bool scene_box(const DevParams* __restrict__ dp,
 }
 
 // The grid of one scene from its bounding box v = (min xyz, max xyz), its
-// smoothing length h and particle count n, with the error bits it raises. With
-// `out` (one thread) each field is stored there as soon as it is known: in a
-// batch the next step waits for the stores.
+// smoothing length h and particle count n, with the error bits it raises.
 struct GridOf {
   float mn[3], mx[3];
   uint32_t gs[3], cells, err;
 };
-__device__ inline GridOf grid_of(const float v[6], float h, uint32_t n,
-                                 DevParams* __restrict__ out) {
+__device__ inline GridOf grid_of(const float v[6], float h, uint32_t n) {
 #pragma clang fp contract(off)
   GridOf g = {};
-  if (out) out->capped = 0;
-  if (n == 0) {
-    if (out) out->p.grid_cell_count = 0;
-    return g;
-  }
+  if (n == 0) return g;
   // Initial values are numeric_limits<cl_int>::max()/min() as float; a
   // position replaces them only when strictly smaller / larger.
   const float init_min = 2147483648.0f, init_max = -2147483648.0f;
@@ -115,23 +107,26 @@ __device__ inline GridOf grid_of(const float v[6], float h, uint32_t n,
     g.mx[a] += L * 2;
     g.gs[a] = (uint32_t)((g.mx[a] - g.mn[a]) / L);
     if (g.gs[a] >= 1024u) g.err |= kErrGridDim;
-    if (out) {
-      out->p.min_point.s[a] = g.mn[a];
-      out->p.max_point.s[a] = g.mx[a];
-    }
   }
   g.cells = morton3(g.gs[0], g.gs[1], g.gs[2]);
   if (g.cells >= (1u << 29)) g.err |= kErrFineKey;
-  if (out) {
-    out->p.min_point.s[3] = 0.f;
-    out->p.max_point.s[3] = 0.f;
-    out->p.grid_size_x = (int32_t)g.gs[0];
-    out->p.grid_size_y = (int32_t)g.gs[1];
-    out->p.grid_size_z = (int32_t)g.gs[2];
-    out->p.grid_cell_count = g.cells;
-    if (g.err) atomicOr(&out->err, g.err);
-  }
   return g;
+}
+
+__device__ inline void store_grid(DevParams* __restrict__ dp, const GridOf& g, uint32_t n) {
+  dp->capped = 0;
+  dp->p.grid_cell_count = g.cells;
+  if (n == 0) return;
+  for (int a = 0; a < 3; ++a) {
+    dp->p.min_point.s[a] = g.mn[a];
+    dp->p.max_point.s[a] = g.mx[a];
+  }
+  dp->p.min_point.s[3] = 0.f;
+  dp->p.max_point.s[3] = 0.f;
+  dp->p.grid_size_x = (int32_t)g.gs[0];
+  dp->p.grid_size_y = (int32_t)g.gs[1];
+  dp->p.grid_size_z = (int32_t)g.gs[2];
+  if (g.err) atomicOr(&dp->err, g.err);
 }
 
 // Half-cell keys of a state of one scene with `cells` cells and error bits

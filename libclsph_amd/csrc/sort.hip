@@ -154,11 +154,14 @@ __global__ __launch_bounds__(kLsdBlock) void k_grid_count(
   const uint32_t np = dp->n, err0 = dp->err, table_cap = bp->table_cap, passes = bp->sort_passes;
   float v[6];
   if (scene_box<kLsdBlock / 64>(dp, partial, stride, red, v) && threadIdx.x == 0) {
-    const GridOf g = grid_of(v, h, np, blockIdx.x == 0 ? dp : nullptr);
+    const GridOf g = grid_of(v, h, np);
     const uint32_t err = err0 | g.err;  // the same in every work-group, stored by now or not
     for (int a = 0; a < 3; ++a) g_min[a] = g.mn[a];
     g_db = key_layout(single_total(single_keys(g.cells, err)), passes).digit_bits;
-    if (blockIdx.x == 0) single_layout(dp, bp, g.cells, err, table_cap, passes);
+    if (blockIdx.x == 0) {
+      store_grid(dp, g, np);
+      single_layout(dp, bp, g.cells, err, table_cap, passes);
+    }
   }
   __syncthreads();
   const float mn[3] = {g_min[0], g_min[1], g_min[2]};
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(kScanBlock) void k_lsd_scan(uint32_t* __restrict__ 
 //
 // FOLD: `offsets` holds the tiles' counts as k_lsd_count left them, and the
 // work-group adds up each digit's counts over the tiles for itself, for few
-// tiles (rule in sort_keys).
+// tiles (rule in launch_sort).
 constexpr int kScatBlock = 512;                         // scatter threads per tile
 constexpr int kScatItems = kLsdTile / kScatBlock;       // keys per thread
 constexpr int kScatWaves = kScatBlock / 64;
