@@ -1029,8 +1029,8 @@ void launch_edge_inputs(clsph_gnn* m, clsph_state* st) {
   hipStream_t s = st->ctx->stream;
   uint32_t n = m->n, e = m->e;
   const DevParams& d = st->host_dps[0];
-  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
-                     m->src, m->dst, m->degc);
+  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr,
+                     st->nbr_count, m->off, n, m->src, m->dst, m->degc);
   uint32_t cnt = e > n ? e : n;
   hipLaunchKernelGGL(k_edge_inputs, grid_of_all(cnt), dim3(256), 0, s, st->pos_s, st->vel_s,
                      st->rho_s, st->prs_s, m->src, m->dst, e, n, d.p.h, d.p.fluid_density,

@@ -1315,8 +1315,8 @@ void launch_edge_inputs(clsph_nn* m, clsph_state* st) {
   hipStream_t s = st->ctx->stream;
   uint32_t n = m->n, e = m->e;
   const DevParams& d = st->host_dps[0];
-  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr, st->nbr_count, m->off, n,
-                     m->src, m->dst, m->degc);
+  hipLaunchKernelGGL(k_graph, dim3(n ? (n + 255) / 256 : 1, 8), dim3(256), 0, s, st->nbr,
+                     st->nbr_count, m->off, n, m->src, m->dst, m->degc);
   hipLaunchKernelGGL(k_node_inputs, grid_of_all(n), dim3(256), 0, s, st->rho_s, st->prs_s, n,
                      d.p.fluid_density, d.p.K, (float2*)m->nu);
   hipLaunchKernelGGL(k_edge_inputs, grid_for(e), dim3(256), 0, s, st->fab,

@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kScanBlock) void k_lsd_scan(uint32_t* __restrict__ 
 //
 // FOLD: `offsets` holds the tiles' counts as k_lsd_count left them, and the
 // work-group adds up each digit's counts over the tiles for itself, for few
-// tiles (rule in launch_sort).
+// tiles (rule in sort_keys).
 constexpr int kScatBlock = 512;                         // scatter threads per tile
 constexpr int kScatItems = kLsdTile / kScatBlock;       // keys per thread
 constexpr int kScatWaves = kScatBlock / 64;
