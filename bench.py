@@ -2,7 +2,7 @@
 
 Default workload: the 1,048,576-particle dam break (0.4 x 0.8 x 0.4 m block
 at spacing 0.5 h in a 1 m box, dt 1e-4 s). W untimed warm-up substeps, then
-K timed substeps replayed from one captured HIP graph, with state resident
+K timed substeps replayed from captured HIP graphs, with state resident
 in HBM. Prints one JSON line with particle-steps/s, the roofline of the
 dominant kernel (timed live with HIP events on the library stream) and a CPU
 baseline (the oracle on the host cores over a bounded sample).
